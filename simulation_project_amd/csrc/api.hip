@@ -540,6 +540,10 @@ template <typename R> struct Engine : EngineBase {
         HIPC(hipMemcpy(d.tris, th.data(), sizeof(TriD<R>) * std::max(1, d.ntri), hipMemcpyHostToDevice));
         ALLOC(tris0, std::max(1, d.ntri));
         HIPC(hipMemcpy(tris0, th.data(), sizeof(TriD<R>) * std::max(1, d.ntri), hipMemcpyHostToDevice));
+        std::vector<R> tab(kMarchTab, R(0));
+        for (int k = 1; k < kMarchTab; ++k) tab[k] = tab[k - 1] + d.c.cell;
+        ALLOC(d.march_tab, kMarchTab);
+        HIPC(hipMemcpy(d.march_tab, tab.data(), sizeof(R) * kMarchTab, hipMemcpyHostToDevice));
         ALLOC(d.tri_emit, d.ntri + 1); ALLOC(d.tri_off, d.ntri + 1);
         ALLOC(d.pair_n, 1); ALLOC(d.uniq_n, 1); ALLOC(d.overflow, 1);
         HIPC(hipMemset(d.overflow, 0, sizeof(int)));
@@ -1221,7 +1225,7 @@ template <typename R> struct BatchGroup {
         const SortJob* jobs = nullptr;
         WorkList tiles, singles;
     };
-    WorkList wp, wt64, wt256, wpairs, wone, wdrag, wtherm, wturb, wc256;
+    WorkList wp, wmarch, wt256, wpairs, wone, wdrag, wtherm, wturb, wc256;
     int2* walk_items = nullptr;        // (bucket, cell) of the cell walks, one per cell of the buckets
     int* walk_n = nullptr;
     size_t walk_cap = 0;
@@ -1307,7 +1311,7 @@ template <typename R> struct BatchGroup {
             int n;
         };
         auto items_of = [&](const std::vector<int2>& v) { return Ref{put(v.data(), v.size() * sizeof(int2)), (int)v.size()}; };
-        std::vector<int2> p, t64, t256, pairs, one, drag, therm, turb, peos, c256;
+        std::vector<int2> p, tmarch, t256, pairs, one, drag, therm, turb, peos, c256;
         const int n = (int)eng.size();
         size_t ncells = 0;
         for (int k = 0; k < n; ++k) {
@@ -1321,7 +1325,7 @@ template <typename R> struct BatchGroup {
                 if (d.c.turb && d.turb_nu) turb.push_back(make_int2(k, j));
             }
             if (d.ntri > 0) {
-                for (int j = 0; j < (int)grid_for(d.ntri, 64); ++j) t64.push_back(make_int2(k, j));
+                for (int j = 0; j < tri_march_blocks(d.ntri); ++j) tmarch.push_back(make_int2(k, j));
                 for (int j = 0; j < (int)grid_for(d.ntri, 256); ++j) t256.push_back(make_int2(k, j));
                 for (int j = 0; j < (int)grid_for(d.pair_cap, 256); ++j) pairs.push_back(make_int2(k, j));
             }
@@ -1331,7 +1335,7 @@ template <typename R> struct BatchGroup {
             }
             one.push_back(make_int2(k, 0));
         }
-        const Ref rp = items_of(p), r64 = items_of(t64), r256 = items_of(t256), rpairs = items_of(pairs),
+        const Ref rp = items_of(p), rmarch = items_of(tmarch), r256 = items_of(t256), rpairs = items_of(pairs),
                   rone = items_of(one), rdrag = items_of(drag), rtherm = items_of(therm), rturb = items_of(turb),
                   rpeos = items_of(peos), rc256 = items_of(c256);
         // fills: cell ranges of the particle binning; triangle counts per cell (and the pair count of
@@ -1427,7 +1431,7 @@ template <typename R> struct BatchGroup {
         }
         HIPC(hipMemcpy(tab, img.data(), img.size(), hipMemcpyHostToDevice));
         auto wl = [&](Ref r) { return WorkList{reinterpret_cast<const int2*>(tab + r.off), r.n}; };
-        wp = wl(rp); wt64 = wl(r64); wt256 = wl(r256); wpairs = wl(rpairs); wone = wl(rone);
+        wp = wl(rp); wmarch = wl(rmarch); wt256 = wl(r256); wpairs = wl(rpairs); wone = wl(rone);
         wdrag = wl(rdrag); wtherm = wl(rtherm); wturb = wl(rturb); wp_eos = wl(rpeos); wc256 = wl(rc256);
         if (ncells > walk_cap) {
             if (walk_items) (void)hipFree(walk_items);
@@ -1478,9 +1482,9 @@ template <typename R> struct BatchGroup {
     void tri(hipStream_t st) {
         const BatchLaunch<R> b = launch();
         fill_int_batched(fill_tri, fill_tri_w, st);
-        launch_tri_count_b(b, wt64, st);
+        launch_tri_count_b(b, wmarch, st);
         exclusive_scan_batched(scan_emit, scan_emit_t, scan_emit_1, st);
-        launch_tri_fill_b(b, wt64, st);
+        launch_tri_fill_b(b, wmarch, st);
         for (const Pass& q : tsort) radix_pass_batched(8, q.jobs, q.tiles, q.singles, st);
         launch_pairs_b(b, 0, wpairs, st);
         exclusive_scan_batched(scan_flag, scan_flag_t, scan_flag_1, st);

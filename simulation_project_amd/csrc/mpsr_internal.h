@@ -376,6 +376,9 @@ struct NbList {
 // initial lattice at 2.1 l0; rows with more walk the stencil)
 static constexpr int kGradWidth = 64;
 
+// entries of Dev::march_tab (a multiple of 64)
+static constexpr int kMarchTab = 1024;
+
 template <typename R> struct Dev {
     int N = 0, cap = 0;
     int block = 256;                  // threads per block of the per-particle kernels (64..512)
@@ -400,6 +403,7 @@ template <typename R> struct Dev {
     mpsr_drag_params* drag = nullptr;
     RotCoef<R>* rot = nullptr;        // [nmodel] for the current step, or the table base when
     const int* step_ctr = nullptr;    // ... this device step counter picks the row (graph replays)
+    R* march_tab = nullptr;           // [kMarchTab] distances of a wall march: 0, then + cell each
     int* tri_emit = nullptr;          // [ntri + 1] emitted cell count per triangle
     int* tri_off = nullptr;           // [ntri + 1]
     int* pair_n = nullptr;            // device count of emitted (cell, triangle) pairs
@@ -508,7 +512,7 @@ template <typename R> void launch_reset_walls(const Dev<R>& d, const TriD<R>* tr
 
 // ---- batched forms of the step kernels ------------------------------------------------------
 // devs: device table of the domains; a work list of (domain, block).  P: blocks of `block`
-// particles; T64 / T256: blocks of 64 / 256 triangles; pairs: blocks of 256 of the pair capacity;
+// particles; tri: the march's workgroups (tri_march_blocks), T256: blocks of 256 triangles; pairs: blocks of 256 of the pair capacity;
 // one: one item per domain.  Each domain's Dev holds the buffers its last sort left the keys and
 // permutation in (skeys, perm), and for replays its rotation table and step counter.
 template <typename R> struct BatchLaunch {
@@ -536,8 +540,9 @@ template <typename R> struct PndRows {
     int nb_width;
 };
 template <typename R> void launch_pnd_ppe_b(const BatchLaunch<R>& b, const PndRows<R>* rows, WorkList p, hipStream_t st);
-template <typename R> void launch_tri_count_b(const BatchLaunch<R>& b, WorkList t64, hipStream_t st);
-template <typename R> void launch_tri_fill_b(const BatchLaunch<R>& b, WorkList t64, hipStream_t st);
+int tri_march_blocks(int ntri);   // workgroups of the triangle march: the items per domain of `tri`
+template <typename R> void launch_tri_count_b(const BatchLaunch<R>& b, WorkList tri, hipStream_t st);
+template <typename R> void launch_tri_fill_b(const BatchLaunch<R>& b, WorkList tri, hipStream_t st);
 // the pair kernels of launch_tri_bin after the pair sort; `pass` = 0 flags, 1 compacts, 2 ranges
 template <typename R> void launch_pairs_b(const BatchLaunch<R>& b, int pass, WorkList pairs, hipStream_t st);
 // each bucket's cell walks (c256: (bucket, block of 256 cells) of the buckets with particles);

@@ -12,6 +12,7 @@
 //   k_translate        UpdateTrianglePosition_Kernel (Kern :463-482)
 //   k_rotate           RotateTrianglePosition_Kernel (Kern :930-998); cos/sin of the step's
 //                      angle come from the host so the rotation is bit-reproducible
+#include <algorithm>
 #include "mpsr_internal.h"
 #include "walls_geom.h"
 
@@ -66,44 +67,221 @@ template <typename R, typename F> __device__ inline void march_triangle(const Co
     } while (mBC >= cs && mAB >= cs && mCA >= cs && ++iter < kMaxShrink);
 }
 
-template <typename R>
-__device__ inline void tri_count_body(int blk, int T, Consts<R> c, const TriD<R>* __restrict__ tris, int* emit) {
-    const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= T) return;
-    const TriD<R> tr = tris[t];
-    int n = 0;
-    march_triangle(c, tr, [&](int) { ++n; });
-    emit[t] = n;
+// A triangle whose longest edge exceeds kLongEdge cells is marched by its whole workgroup: a wall of
+// a few large triangles is one long serial chain per triangle otherwise, with as many lanes of the
+// GPU at work as there are triangles (the reference's 14-triangle deck: 595 us a pass with one lane
+// per triangle, 28.7 us so; a 12-triangle FP64 tank 409 and 28.0 us).  The shrinking alone is a chain, and only of the vertices: one wave walks it, lane l
+// holding vertex l % 3 of up to kMarchIters copies at a time.  The lines of those copies are then
+// marched by the workgroup's waves, 64 samples of a line at once, with the distances along the line
+// read from a table of the repeated sums 0, cell, cell + cell, ... the serial march forms.  The same
+// samples, the same arithmetic and the same test against the previous sample inside the grid, so a
+// triangle has the same emissions, in another order (a cell's pairs are sorted by triangle).
+// What remains is the chain of the copies.  Shorter edges (a finely meshed drum: 2-3 samples a line)
+// leave most of a wave idle in that form and stay with one lane per triangle (10k such triangles:
+// 7.2 us a pass).
+static constexpr int kLongEdge = 4;
+static constexpr int kMarchIters = 32;
+static constexpr int kMarchBlock = 256;
+template <typename R> struct MarchLds {
+    R v[kMarchIters][9];
+    int first[3 * kMarchIters], last[3 * kMarchIters];   // first and last cell of each line, -1: none
+    int copies, more, count, nlong;
+    int longs[kMarchBlock];
+};
+// the next slots of the triangle for the lanes that emit; every lane of the wave calls it
+template <typename R, typename F> __device__ inline void emit_wave(bool em, int cid, MarchLds<R>& L, F&& put) {
+    const unsigned long long mask = __ballot(em);
+    if (!mask) return;
+    int base = 0;
+    if (lane_id() == 0) base = atomicAdd(&L.count, (int)__popcll(mask));
+    base = __shfl(base, 0, 64);
+    if (em) put(base + __popcll(mask & ((1ull << lane_id()) - 1ull)), cid);
 }
-template <typename R>
-__global__ __launch_bounds__(64) void k_tri_count(int T, Consts<R> c, const TriD<R>* __restrict__ tris, int* emit) {
-    tri_count_body<R>(blockIdx.x, T, c, tris, emit);
-}
-
-template <typename R>
-__device__ inline void tri_fill_body(int blk, int T, Consts<R> c, const TriD<R>* __restrict__ tris,
-                                     const int* __restrict__ off, const int* __restrict__ pair_n,
-                                     int pair_cap, uint32_t* pair_cell, int* pair_tri, int* overflow) {
-    const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= T) return;
-    if (*pair_n > pair_cap) {
-        if (t == 0) *overflow = 1;
-        return;
+// put(k, cell) for the triangle's emissions k = 0 .. L.count - 1, in any order; every thread of the
+// workgroup calls it with the same triangle
+template <typename R, typename F>
+__device__ inline void march_triangle_block(const Consts<R>& c, const TriD<R>& tr, const R* __restrict__ tab,
+                                            MarchLds<R>& L, F&& put) {
+    const int lane = lane_id(), w = (int)(threadIdx.x >> 6), nw = (int)(blockDim.x >> 6);
+    const R cs = c.cell;
+    const int own = lane % 3;
+    P3<R> V = p3(tr.v[3 * own], tr.v[3 * own + 1], tr.v[3 * own + 2]);
+    int iter = 0, carry = -1;
+    if (threadIdx.x == 0) L.count = 0;
+    bool more = true;
+    while (more) {
+        if (w == 0) {
+            int n = 0;
+            bool go = true;
+            while (go && n < kMarchIters) {
+                if (lane < 3) {
+                    L.v[n][3 * lane] = V.x;
+                    L.v[n][3 * lane + 1] = V.y;
+                    L.v[n][3 * lane + 2] = V.z;
+                }
+                const int ln = (own + 1) % 3, lp = (own + 2) % 3;
+                const P3<R> N = p3(__shfl(V.x, ln, 64), __shfl(V.y, ln, 64), __shfl(V.z, ln, 64));
+                const P3<R> Q = p3(__shfl(V.x, lp, 64), __shfl(V.y, lp, 64), __shfl(V.z, lp, 64));
+                const P3<R> e = psub(N, V);
+                const R m = pmag(e);
+                P3<R> md = padd(e, psub(Q, V));
+                const R mm = pmag(md);
+                if (mm > 0.0) {
+                    md.x /= mm; md.y /= mm; md.z /= mm;
+                    V.x += md.x * cs; V.y += md.y * cs; V.z += md.z * cs;
+                }
+                ++n;
+                go = __all(m >= cs) && ++iter < kMaxShrink;
+            }
+            if (lane == 0) {
+                L.copies = n;
+                L.more = go ? 1 : 0;
+            }
+        }
+        __syncthreads();
+        const int nl = 3 * L.copies;
+        for (int q = w; q < nl; q += nw) {
+            const R* a = L.v[q / 3] + 3 * (q % 3);
+            const R* b = L.v[q / 3] + 3 * ((q + 1) % 3);
+            const P3<R> v = p3(a[0], a[1], a[2]);
+            P3<R> d = psub(p3(b[0], b[1], b[2]), v);
+            const R m = pmag(d);
+            int first = -1, prev = -1;
+            if (m > 0.0) {
+                d.x /= m; d.y /= m; d.z /= m;
+                R next = 0;   // beyond the table: the distance of sample `base`
+                for (int base = 0; base < kMaxLineSteps; base += 64) {
+                    R tb;
+                    if (base < kMarchTab) {
+                        tb = tab[base + lane];
+                        if (base + 64 == kMarchTab) next = __shfl(tb, 63, 64) + cs;
+                    } else {
+                        tb = next;
+                        for (int j = 0; j < lane; ++j) tb += cs;
+                        next = __shfl(tb, 63, 64) + cs;
+                    }
+                    const bool in = base + lane == 0 || tb <= m;
+                    int cid = -1;
+                    if (in) {
+                        int i, j, k;
+                        if (cell_coords(c, v.x + tb * d.x, v.y + tb * d.y, v.z + tb * d.z, i, j, k)) {
+                            const long long id = cell_of(c, i, j, k);
+                            if (id >= 0 && id < c.ncell) cid = (int)id;
+                        }
+                    }
+                    const unsigned long long vm = __ballot(cid >= 0);
+                    const unsigned long long below = vm & ((1ull << lane) - 1ull);
+                    const int pc = __shfl(cid, below ? 63 - __clzll(below) : 0, 64);
+                    bool em = cid >= 0 && cid != (below ? pc : prev);
+                    if (vm) {
+                        if (first < 0) {   // emitted or not by the line before it, below
+                            const int fl = __ffsll(vm) - 1;
+                            first = __shfl(cid, fl, 64);
+                            if (lane == fl) em = false;
+                        }
+                        prev = __shfl(cid, 63 - __clzll(vm), 64);
+                    }
+                    emit_wave(em, cid, L, put);
+                    if (!__shfl((int)in, 63, 64)) break;
+                }
+            }
+            if (lane == 0) {
+                L.first[q] = first;
+                L.last[q] = prev;
+            }
+        }
+        __syncthreads();
+        if (w == 0) {
+            // every line's first cell, against the last cell of the lines before it
+            for (int base = 0; base < nl; base += 64) {
+                const int q = base + lane;
+                const int f = q < nl ? L.first[q] : -1, l = q < nl ? L.last[q] : -1;
+                const unsigned long long vm = __ballot(f >= 0);
+                const unsigned long long below = vm & ((1ull << lane) - 1ull);
+                const int pl = __shfl(l, below ? 63 - __clzll(below) : 0, 64);
+                emit_wave(f >= 0 && f != (below ? pl : carry), f, L, put);
+                if (vm) carry = __shfl(l, 63 - __clzll(vm), 64);
+            }
+        }
+        more = L.more != 0;
+        __syncthreads();
     }
-    const TriD<R> tr = tris[t];
-    int e = off[t];
-    march_triangle(c, tr, [&](int cid) {
-        pair_cell[e] = (uint32_t)cid;
-        pair_tri[e] = t;
-        ++e;
-    });
 }
-template <typename R>
-__global__ __launch_bounds__(64) void k_tri_fill(int T, Consts<R> c, const TriD<R>* __restrict__ tris,
-                                                 const int* __restrict__ off, const int* __restrict__ pair_n,
-                                                 int pair_cap, uint32_t* pair_cell, int* pair_tri, int* overflow) {
-    tri_fill_body<R>(blockIdx.x, T, c, tris, off, pair_n, pair_cap, pair_cell, pair_tri, overflow);
+// workgroups of the march: the triangles in equal runs, one run per workgroup, one triangle per
+// workgroup up to 256 triangles
+inline int march_blocks(int T) { return T <= kMarchBlock ? T : std::max(kMarchBlock, (T + kMarchBlock - 1) / kMarchBlock); }
+__device__ inline int march_run(int T) {
+    const int nb = T <= kMarchBlock ? T : max(kMarchBlock, (T + kMarchBlock - 1) / kMarchBlock);
+    return (T + nb - 1) / nb;
 }
+// FILL: the pairs of the triangles of workgroup blk, at off[t]; else their number per triangle
+template <typename R, bool FILL>
+__device__ inline void tri_march_body(int blk, int T, const Consts<R>& c, const TriD<R>* __restrict__ tris,
+                                      const R* __restrict__ tab, int* __restrict__ emit, const int* __restrict__ off,
+                                      const int* __restrict__ pair_n, int pair_cap, uint32_t* pair_cell,
+                                      int* pair_tri, int* overflow, MarchLds<R>& L) {
+    if constexpr (FILL) {
+        if (*pair_n > pair_cap) {
+            if (blk == 0 && threadIdx.x == 0) *overflow = 1;
+            return;
+        }
+    }
+    const int run = march_run(T), t0 = blk * run, t1 = min(T, t0 + run);
+    if (threadIdx.x == 0) L.nlong = 0;
+    __syncthreads();
+    const int t = t0 + (int)threadIdx.x;
+    if (t < t1) {
+        const TriD<R> tr = tris[t];
+        const P3<R> A = p3(tr.v[0], tr.v[1], tr.v[2]), B = p3(tr.v[3], tr.v[4], tr.v[5]), C = p3(tr.v[6], tr.v[7], tr.v[8]);
+        const R lim = (R)kLongEdge * c.cell;
+        bool fin = true;
+        for (int q = 0; q < 9; ++q) fin = fin && isfinite(tr.v[q]);
+        if (fin && !(pmag(psub(B, A)) <= lim && pmag(psub(C, B)) <= lim && pmag(psub(A, C)) <= lim)) {
+            L.longs[atomicAdd(&L.nlong, 1)] = t;
+        } else if constexpr (FILL) {
+            int e = off[t];
+            march_triangle(c, tr, [&](int cid) {
+                pair_cell[e] = (uint32_t)cid;
+                pair_tri[e] = t;
+                ++e;
+            });
+        } else {
+            int n = 0;
+            march_triangle(c, tr, [&](int) { ++n; });
+            emit[t] = n;
+        }
+    }
+    __syncthreads();
+    const int nlong = L.nlong;
+    for (int q = 0; q < nlong; ++q) {
+        const int tl = L.longs[q];
+        if constexpr (FILL) {
+            const int o = off[tl];
+            march_triangle_block(c, tris[tl], tab, L, [&](int k, int cid) {
+                pair_cell[o + k] = (uint32_t)cid;
+                pair_tri[o + k] = tl;
+            });
+        } else {
+            march_triangle_block(c, tris[tl], tab, L, [&](int, int) {});
+            if (threadIdx.x == 0) emit[tl] = L.count;
+            __syncthreads();
+        }
+    }
+}
+template <typename R, bool FILL>
+__global__ __launch_bounds__(kMarchBlock) void k_tri_march(int T, Consts<R> c, const TriD<R>* __restrict__ tris,
+                                                           const R* __restrict__ tab, int* emit,
+                                                           const int* __restrict__ off, const int* __restrict__ pair_n,
+                                                           int pair_cap, uint32_t* pair_cell, int* pair_tri,
+                                                           int* overflow) {
+    __shared__ MarchLds<R> L;
+    tri_march_body<R, FILL>(blockIdx.x, T, c, tris, tab, emit, off, pair_n, pair_cap, pair_cell, pair_tri, overflow, L);
+}
+template <typename R, bool FILL> static void launch_tri_march(const Dev<R>& d, hipStream_t st) {
+    hipLaunchKernelGGL((k_tri_march<R, FILL>), dim3(march_blocks(d.ntri)), dim3(kMarchBlock), 0, st, d.ntri, d.c, d.tris,
+                       d.march_tab, d.tri_emit, d.tri_off, d.pair_n, d.pair_cap, d.pair_cell, d.pair_tri, d.overflow);
+}
+int tri_march_blocks(int T) { return march_blocks(T); }
 
 // 1 where a sorted pair differs from its predecessor
 __device__ inline void pair_flags_body(int blk, const int* pair_n, int pair_cap, const uint32_t* __restrict__ cell,
@@ -157,7 +335,7 @@ template <typename R> void launch_tri_count_total(Dev<R>& d, hipStream_t st) {
         fill_int(d.pair_n, 0, 1, st);
         return;
     }
-    hipLaunchKernelGGL(k_tri_count<R>, dim3(grid_for(d.ntri, 64)), dim3(64), 0, st, d.ntri, d.c, d.tris, d.tri_emit);
+    launch_tri_march<R, false>(d, st);
     exclusive_scan(d.tri_emit, d.tri_off, nullptr, d.ntri, d.ntri, d.pair_n, d.tsort, st);
 }
 
@@ -356,10 +534,9 @@ template <typename R> void launch_tri_bin(Dev<R>& d, hipStream_t st) {
         return;
     }
     const int T = d.ntri;
-    hipLaunchKernelGGL(k_tri_count<R>, dim3(grid_for(T, 64)), dim3(64), 0, st, T, d.c, d.tris, d.tri_emit);
+    launch_tri_march<R, false>(d, st);
     exclusive_scan(d.tri_emit, d.tri_off, nullptr, T, T, d.pair_n, d.tsort, st);
-    hipLaunchKernelGGL(k_tri_fill<R>, dim3(grid_for(T, 64)), dim3(64), 0, st, T, d.c, d.tris, d.tri_off, d.pair_n,
-                       d.pair_cap, d.pair_cell, d.pair_tri, d.overflow);
+    launch_tri_march<R, true>(d, st);
     const int bits = tri_pair_bits(d.c.ncell);
     const int which = radix_sort_pairs(d.pair_cell, d.pair_tri, d.pair_n, 0, d.pair_cap, bits, d.tsort, st);
     const uint32_t* sc = which ? d.tsort.k1 : d.pair_cell;
@@ -555,20 +732,15 @@ __global__ void k_step_advance(int* ctr) {
 void launch_step_advance(int* ctr, hipStream_t st) { hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, st, ctr); }
 
 // ---- batched forms: one work item = one block of one domain's particles or triangles ---------
-template <typename R> struct OpTriCount {
-    const Dev<R>* dv;
-    __device__ void operator()(int k, int b) const {
-        const Dev<R>& d = dv[k];
-        tri_count_body<R>(b, d.ntri, d.c, d.tris, d.tri_emit);
-    }
-};
-template <typename R> struct OpTriFill {
-    const Dev<R>* dv;
-    __device__ void operator()(int k, int b) const {
-        const Dev<R>& d = dv[k];
-        tri_fill_body<R>(b, d.ntri, d.c, d.tris, d.tri_off, d.pair_n, d.pair_cap, d.pair_cell, d.pair_tri, d.overflow);
-    }
-};
+template <typename R, bool FILL>
+__global__ __launch_bounds__(kMarchBlock) void k_tri_march_b(const Dev<R>* __restrict__ dv,
+                                                             const int2* __restrict__ items) {
+    __shared__ MarchLds<R> L;
+    const int2 w = items[blockIdx.x];
+    const Dev<R>& d = dv[w.x];
+    tri_march_body<R, FILL>(w.y, d.ntri, d.c, d.tris, d.march_tab, d.tri_emit, d.tri_off, d.pair_n, d.pair_cap,
+                            d.pair_cell, d.pair_tri, d.overflow, L);
+}
 // the sorted pairs are where the pair sort's passes left them (radix_sort_pairs' parity)
 template <typename R> struct OpPairs {
     const Dev<R>* dv;
@@ -647,11 +819,13 @@ template <typename R> struct OpStepAdvance {
         if (threadIdx.x == 0 && ctr) ctr[0] = ctr[0] + 1;
     }
 };
-template <typename R> void launch_tri_count_b(const BatchLaunch<R>& b, WorkList t64, hipStream_t st) {
-    launch_batched<64>(OpTriCount<R>{b.devs}, t64, 64, st);
+template <typename R> void launch_tri_count_b(const BatchLaunch<R>& b, WorkList tri, hipStream_t st) {
+    if (tri.n > 0)
+        hipLaunchKernelGGL((k_tri_march_b<R, false>), dim3(tri.n), dim3(kMarchBlock), 0, st, b.devs, tri.items);
 }
-template <typename R> void launch_tri_fill_b(const BatchLaunch<R>& b, WorkList t64, hipStream_t st) {
-    launch_batched<64>(OpTriFill<R>{b.devs}, t64, 64, st);
+template <typename R> void launch_tri_fill_b(const BatchLaunch<R>& b, WorkList tri, hipStream_t st) {
+    if (tri.n > 0)
+        hipLaunchKernelGGL((k_tri_march_b<R, true>), dim3(tri.n), dim3(kMarchBlock), 0, st, b.devs, tri.items);
 }
 template <typename R> void launch_pairs_b(const BatchLaunch<R>& b, int pass, WorkList pairs, hipStream_t st) {
     launch_batched<256>(OpPairs<R>{b.devs, pass}, pairs, 256, st);
