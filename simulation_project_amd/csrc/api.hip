@@ -510,6 +510,15 @@ template <typename R> struct Engine : EngineBase {
         ALLOC(d.keys, cap); ALLOC(d.vals, cap);
         ALLOC(d.cell_start, d.c.ncell); ALLOC(d.cell_end, d.c.ncell);
         ALLOC(d.spos, cap); ALLOC(d.svel, cap); ALLOC(d.spres, cap);
+        d.rel.stride = cap + 32;
+        d.rel.half = cap / 2 + 32;
+        ALLOC(d.rel.x, 4 * (size_t)d.rel.stride); ALLOC(d.rel.w, 2 * d.rel.half);
+        HIPC(hipMemset(d.rel.x, 0, sizeof(float) * 3 * (size_t)d.rel.stride));
+        HIPC(hipMemset(d.rel.w, 0, sizeof(float) * 2 * d.rel.half));
+        {
+            const std::vector<float> one(d.rel.stride, 1.0f);
+            HIPC(hipMemcpy(d.rel.x + 3 * (size_t)d.rel.stride, one.data(), sizeof(float) * one.size(), hipMemcpyHostToDevice));
+        }
         ALLOC(d.stl_mag, cap); ALLOC(d.stl_dir, cap); ALLOC(d.stl_id, cap);
         ALLOC(d.drag_acc, cap); ALLOC(d.drag_temp, cap);
         HIPC(hipMemset(d.drag_acc, 0, sizeof(R4<R>) * cap));
@@ -1225,6 +1234,7 @@ template <typename R> struct BatchGroup {
         const SortJob* jobs = nullptr;
         WorkList tiles, singles;
     };
+    WorkList wnear;                    // blocks of kNearBlock particles
     WorkList wp, wmarch, wt256, wpairs, wone, wdrag, wtherm, wturb, wc256;
     int2* walk_items = nullptr;        // (bucket, cell) of the cell walks, one per cell of the buckets
     int* walk_n = nullptr;
@@ -1236,7 +1246,7 @@ template <typename R> struct BatchGroup {
     const ScanJob* scan_emit = nullptr;
     const ScanJob* scan_flag = nullptr;
     WorkList scan_emit_t, scan_emit_1, scan_flag_t, scan_flag_1;
-    WorkList wp_eos;                   // particle blocks of the buckets with the EOS pressure
+    WorkList wp_eos;                   // kNearBlock blocks of the buckets with the EOS pressure
     PpeBatch<R>* pb = nullptr;         // the PPE buckets' solves (null: none)
 
     ~BatchGroup() {
@@ -1311,7 +1321,7 @@ template <typename R> struct BatchGroup {
             int n;
         };
         auto items_of = [&](const std::vector<int2>& v) { return Ref{put(v.data(), v.size() * sizeof(int2)), (int)v.size()}; };
-        std::vector<int2> p, tmarch, t256, pairs, one, drag, therm, turb, peos, c256;
+        std::vector<int2> p, pnear, tmarch, t256, pairs, one, drag, therm, turb, peos, c256;
         const int n = (int)eng.size();
         size_t ncells = 0;
         for (int k = 0; k < n; ++k) {
@@ -1319,8 +1329,11 @@ template <typename R> struct BatchGroup {
             const int nb = (int)grid_for(d.N, block);
             for (int j = 0; j < nb; ++j) {
                 p.push_back(make_int2(k, j));
-                if (eng[k]->pressure_mode != MPSR_PRESSURE_PPE) peos.push_back(make_int2(k, j));
                 if (d.ndrag > 0) drag.push_back(make_int2(k, j));
+            }
+            for (int j = 0; j < (int)grid_for(d.N, kNearBlock); ++j) {
+                pnear.push_back(make_int2(k, j));
+                if (eng[k]->pressure_mode != MPSR_PRESSURE_PPE) peos.push_back(make_int2(k, j));
                 if (eng[k]->P.bUpdateTemperature) therm.push_back(make_int2(k, j));
                 if (d.c.turb && d.turb_nu) turb.push_back(make_int2(k, j));
             }
@@ -1335,7 +1348,7 @@ template <typename R> struct BatchGroup {
             }
             one.push_back(make_int2(k, 0));
         }
-        const Ref rp = items_of(p), rmarch = items_of(tmarch), r256 = items_of(t256), rpairs = items_of(pairs),
+        const Ref rp = items_of(p), rnear = items_of(pnear), rmarch = items_of(tmarch), r256 = items_of(t256), rpairs = items_of(pairs),
                   rone = items_of(one), rdrag = items_of(drag), rtherm = items_of(therm), rturb = items_of(turb),
                   rpeos = items_of(peos), rc256 = items_of(c256);
         // fills: cell ranges of the particle binning; triangle counts per cell (and the pair count of
@@ -1431,7 +1444,7 @@ template <typename R> struct BatchGroup {
         }
         HIPC(hipMemcpy(tab, img.data(), img.size(), hipMemcpyHostToDevice));
         auto wl = [&](Ref r) { return WorkList{reinterpret_cast<const int2*>(tab + r.off), r.n}; };
-        wp = wl(rp); wmarch = wl(rmarch); wt256 = wl(r256); wpairs = wl(rpairs); wone = wl(rone);
+        wp = wl(rp); wnear = wl(rnear); wmarch = wl(rmarch); wt256 = wl(r256); wpairs = wl(rpairs); wone = wl(rone);
         wdrag = wl(rdrag); wtherm = wl(rtherm); wturb = wl(rturb); wp_eos = wl(rpeos); wc256 = wl(rc256);
         if (ncells > walk_cap) {
             if (walk_items) (void)hipFree(walk_items);
@@ -1465,7 +1478,7 @@ template <typename R> struct BatchGroup {
         if (!solvers.empty()) {
             if (!pb) pb = ppe_batch_create<R>();
             mpsr_status ps = ppe_batch_build(pb, solvers.data(), pdev.data(), host.data(), popt.data(),
-                                             (int)solvers.size(), block);
+                                             (int)solvers.size());
             if (ps != MPSR_NOERR) return fail(ps, "batched step: PPE solver tables");
         }
         sig = sg;
@@ -1503,7 +1516,7 @@ template <typename R> struct BatchGroup {
         launch_drag_b(b, wdrag, st);
         launch_thermal_b(b, wtherm, st);
         launch_turbulence_b(b, wturb, st);
-        launch_explicit_b(b, wp, st);
+        launch_explicit_b(b, wp, wnear, st);
         launch_relocate_b(b, wp, st);
         bin(st);
         launch_stl_distance_b(b, wp, st);

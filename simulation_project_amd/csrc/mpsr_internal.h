@@ -376,6 +376,19 @@ struct NbList {
 // initial lattice at 2.1 l0; rows with more walk the stencil)
 static constexpr int kGradWidth = 64;
 
+// Positions relative to the centre of their cell, sorted order: component k at x[k * stride + t], the
+// fourth component 1; half the square of the length in w, the even t first, the odd ones from w[half]
+// on.  stride = capacity + 32 (rows past the last particle are read, and ignored).
+struct RelPos {
+    float* x = nullptr;
+    float* w = nullptr;
+    int stride = 0, half = 0;
+    __device__ float& half_sq(int t) const { return w[(t & 1 ? half : 0) + (t >> 1)]; }
+};
+
+// threads of a workgroup of the kernels on for_near_mfma
+static constexpr int kNearBlock = 64;
+
 // entries of Dev::march_tab (a multiple of 64)
 static constexpr int kMarchTab = 1024;
 
@@ -395,6 +408,7 @@ template <typename R> struct Dev {
     int* cell_end = nullptr;
     R4<R>* spos = nullptr;
     R4<R>* svel = nullptr;
+    RelPos rel{};
     R* spres = nullptr;
     int key_bits = 0;
     // walls
@@ -512,7 +526,8 @@ template <typename R> void launch_reset_walls(const Dev<R>& d, const TriD<R>* tr
 
 // ---- batched forms of the step kernels ------------------------------------------------------
 // devs: device table of the domains; a work list of (domain, block).  P: blocks of `block`
-// particles; tri: the march's workgroups (tri_march_blocks), T256: blocks of 256 triangles; pairs: blocks of 256 of the pair capacity;
+// particles; near (and the lists of the PND pass, heat conduction and turbulence): blocks of
+// kNearBlock particles; tri: the march's workgroups (tri_march_blocks), T256: blocks of 256 triangles; pairs: blocks of 256 of the pair capacity;
 // one: one item per domain.  Each domain's Dev holds the buffers its last sort left the keys and
 // permutation in (skeys, perm), and for replays its rotation table and step counter.
 template <typename R> struct BatchLaunch {
@@ -521,7 +536,7 @@ template <typename R> struct BatchLaunch {
 };
 template <typename R> void launch_bin_hash_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st);
 template <typename R> void launch_bin_ranges_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st);
-template <typename R> void launch_explicit_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st);
+template <typename R> void launch_explicit_b(const BatchLaunch<R>& b, WorkList p, WorkList near, hipStream_t st);
 template <typename R> void launch_relocate_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st);
 template <typename R> void launch_pnd_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st);   // EOS pressure
 template <typename R> void launch_gradient_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st);

@@ -76,11 +76,13 @@ __global__ __launch_bounds__(kMaxBlock) void k_bin_hash(int N, Consts<R> c, PSta
 }
 
 template <typename R>
-__device__ inline void bin_ranges_body(int blk, int N, int ncell, const uint32_t* __restrict__ sk,
+__device__ inline void bin_ranges_body(int blk, int N, Consts<R> c, const uint32_t* __restrict__ sk,
                                        const int* __restrict__ perm, int* cs, int* ce, PState<R> in,
-                                       R4<R>* __restrict__ spos, R4<R>* __restrict__ svel) {
+                                       R4<R>* __restrict__ spos, R4<R>* __restrict__ svel,
+                                       RelPos rel) {
     const int t = blk * blockDim.x + threadIdx.x;
     if (t >= N) return;
+    const int ncell = c.ncell;
     const uint32_t k = sk[t];
     const uint32_t kp = t > 0 ? sk[t - 1] : 0xffffffffu;
     const uint32_t sent = (uint32_t)ncell;
@@ -90,75 +92,67 @@ __device__ inline void bin_ranges_body(int blk, int N, int ncell, const uint32_t
     }
     if (t == N - 1 && k != sent) ce[k] = N;
     const int s = perm[t];
-    spos[t] = mk4<R>(in.px[s], in.py[s], in.pz[s], R(0));
+    const R x = in.px[s], y = in.py[s], z = in.pz[s];
+    spos[t] = mk4<R>(x, y, z, R(0));
     svel[t] = mk4<R>(in.vx[s], in.vy[s], in.vz[s], R(0));
+    // for the matrix-core walk (for_near_mfma); nothing reads the entry of a slot without a cell
+    float qx = 0, qy = 0, qz = 0;
+    if (k != sent) {
+        const uint32_t gyz = (uint32_t)c.gy * (uint32_t)c.gz, i = k / gyz, r = k - i * gyz, j = r / (uint32_t)c.gz;
+        qx = (float)(x - (c.bminx + ((R)i + (R)0.5) * c.cell));
+        qy = (float)(y - (c.bminy + ((R)j + (R)0.5) * c.cell));
+        qz = (float)(z - (c.bminz + ((R)(r - j * (uint32_t)c.gz) + (R)0.5) * c.cell));
+    }
+    rel.x[t] = qx;
+    rel.x[rel.stride + t] = qy;
+    rel.x[2 * (size_t)rel.stride + t] = qz;
+    rel.half_sq(t) = 0.5f * (qx * qx + qy * qy + qz * qz);
 }
 template <typename R>
-__global__ __launch_bounds__(kMaxBlock) void k_bin_ranges(int N, int ncell, const uint32_t* __restrict__ sk,
+__global__ __launch_bounds__(kMaxBlock) void k_bin_ranges(int N, Consts<R> c, const uint32_t* __restrict__ sk,
                                                      const int* __restrict__ perm, int* cs, int* ce, PState<R> in,
-                                                     R4<R>* __restrict__ spos, R4<R>* __restrict__ svel) {
-    bin_ranges_body<R>(blockIdx.x, N, ncell, sk, perm, cs, ce, in, spos, svel);
+                                                     R4<R>* __restrict__ spos, R4<R>* __restrict__ svel,
+                                                     RelPos rel) {
+    bin_ranges_body<R>(blockIdx.x, N, c, sk, perm, cs, ce, in, spos, svel, rel);
 }
 
 // ---------------------------------------------------------------------------------------------
-template <typename R>
-__device__ inline void explicit_body(int blk, int N, Consts<R> c, const int* __restrict__ perm, PState<R> in,
-                                     PState<R> out, const R4<R>* __restrict__ spos,
-                                     const R4<R>* __restrict__ svel, const int* __restrict__ cs,
-                                     const int* __restrict__ ce, const R* __restrict__ stl_mag,
-                                     const R4<R>* __restrict__ stl_dir, const int* __restrict__ stl_id,
-                                     const R4<R>* __restrict__ drag_acc, const R4<R>* __restrict__ sph_dv,
-                                     const TriD<R>* __restrict__ tris,
-                                     const mpsr_tri_params* __restrict__ models,
-                                     const R* __restrict__ turb_nu) {
-    const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= N) return;
-    const int s = perm[t];
-    if (out.id[s] < 0) return;
-    const R4<R> P = spos[t];
-    const R x = P.x, y = P.y, z = P.z;
-    if (!include(c, x, y, z)) return;
-    const R4<R> V0 = svel[t];
+template <typename R> struct PosVel { R4<R> p, v; };
+// the predictor's sums over the neighbours: viscosity, artificial pressure, collisions
+template <typename R> struct ExplicitSums {
     R lx = 0, ly = 0, lz = 0, ax = 0, ay = 0, az = 0, qx = 0, qy = 0, qz = 0;
-    const R re = c.re_lap, mind = c.mind_lap;
-    // per group of 4 candidates: the distances first, then the velocities of the hits, loaded
-    // together, then the sums in the canonical order
-    for_candidate_groups(c, cs, ce, spos, x, y, z, [&](int t0, const R4<R> (&Q)[4], int m) {
-        R dd[4];
-        bool hit[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            dd[u] = dist3(x, y, z, Q[u].x, Q[u].y, Q[u].z);
-            hit[u] = u < m && t0 + u != t && dd[u] < re;
-        }
-        R4<R> V[4];   // read only where hit[u]
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (hit[u]) V[u] = svel[t0 + u];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (!hit[u]) continue;
-            R d = dd[u];
-            if (d < mind) d = mind;
-            const R w = weight(re, d);
-            const R4<R>& V1 = V[u];
-            lx += (V1.x - V0.x) * w;
-            ly += (V1.y - V0.y) * w;
-            lz += (V1.z - V0.z) * w;
-            if (c.expl) {
-                const R a = c.art_p * w / (d * d);
-                ax = ax + (Q[u].x - x) * a;
-                ay = ay + (Q[u].y - y) * a;
-                az = az + (Q[u].z - z) * a;
-                if (d < c.rc) {
-                    const R cc = (c.rc - d) / d;
-                    qx = qx + (Q[u].x - x) * cc;
-                    qy = qy + (Q[u].y - y) * cc;
-                    qz = qz + (Q[u].z - z) * cc;
-                }
+    // neighbour at distance d0 < re_lap
+    __device__ void add(const Consts<R>& c, R x, R y, R z, const R4<R>& V0, const R4<R>& Q, const R4<R>& V1, R d0) {
+        R d = d0;
+        if (d < c.mind_lap) d = c.mind_lap;
+        const R w = c.re_lap / d - 1;   // weight(re, d) for 0 < d < re
+        lx += (V1.x - V0.x) * w;
+        ly += (V1.y - V0.y) * w;
+        lz += (V1.z - V0.z) * w;
+        if (c.expl) {
+            const R a = c.art_p * w / (d * d);
+            ax = ax + (Q.x - x) * a;
+            ay = ay + (Q.y - y) * a;
+            az = az + (Q.z - z) * a;
+            if (d < c.rc) {
+                const R cc = (c.rc - d) / d;
+                qx = qx + (Q.x - x) * cc;
+                qy = qy + (Q.y - y) * cc;
+                qz = qz + (Q.z - z) * cc;
             }
         }
-    });
+    }
+};
+// the wall terms, the new velocity and position of sorted particle t (slot s)
+template <typename R>
+__device__ inline void explicit_finish(int t, int s, const Consts<R>& c, const PState<R>& in, const PState<R>& out, R x,
+                                       R y, R z, const R4<R>& V0, ExplicitSums<R> S, const R* __restrict__ stl_mag,
+                                       const R4<R>* __restrict__ stl_dir, const int* __restrict__ stl_id,
+                                       const R4<R>* __restrict__ drag_acc, const R4<R>* __restrict__ sph_dv,
+                                       const TriD<R>* __restrict__ tris,
+                                       const mpsr_tri_params* __restrict__ models, const R* __restrict__ turb_nu) {
+    R lx = S.lx, ly = S.ly, lz = S.lz, ax = S.ax, ay = S.ay, az = S.az, qx = S.qx, qy = S.qy, qz = S.qz;
+    const R re = c.re_lap;
     const R dw = stl_mag[t];
     const int tid = stl_id[t];
     if (tid >= 0 && tid < c.ntri) {
@@ -221,20 +215,81 @@ __device__ inline void explicit_body(int blk, int N, Consts<R> c, const int* __r
         out.vx[s] = vx; out.vy[s] = vy; out.vz[s] = vz;
     }
 }
-template <typename R>
-__global__ __launch_bounds__(kMaxBlock) void k_explicit(int N, Consts<R> c, const int* __restrict__ perm, PState<R> in,
-                                                   PState<R> out, const R4<R>* __restrict__ spos,
-                                                   const R4<R>* __restrict__ svel, const int* __restrict__ cs,
-                                                   const int* __restrict__ ce, const R* __restrict__ stl_mag,
-                                                   const R4<R>* __restrict__ stl_dir, const int* __restrict__ stl_id,
-                                                   const R4<R>* __restrict__ drag_acc, const R4<R>* __restrict__ sph_dv,
-                                                   const TriD<R>* __restrict__ tris,
-                                                   const mpsr_tri_params* __restrict__ models,
-                                                   const R* __restrict__ turb_nu) {
+// NEAR: one wave per 64 sorted particles (for_near_mfma), else the plain walk, one lane per particle.
+// The near walk's second phase gathers 32 bytes a neighbour, half of them past L1, and on a full chip it
+// falls behind the plain FP32 walk, whose lanes read the same candidates; an FP64 candidate costs the
+// plain walk twice as much.  Near against plain (start of a drum, without / with the explicit pressure's
+// sums): FP32 107 / 186 us at 4k particles, 165 / 193 and 174 / 238 at 126k, 280 / 257 and 302 / 327 at
+// 245k, 534 / 473 and 570 / 560 at 517k, 928 / 801 and 998 / 968 at 1M; FP64 128 / 289 at 32k, 800 / 1063
+// at 517k, 1154 / 2062 at 1M.
+template <typename R> static bool near_explicit(long long n) { return sizeof(R) == 8 || n <= 200000; }
+template <typename R, bool NEAR>
+__device__ inline void explicit_body(int blk, int N, Consts<R> c, const int* __restrict__ perm,
+                                     PState<R> in, PState<R> out, const R4<R>* __restrict__ spos,
+                                     const R4<R>* __restrict__ svel, RelPos rel,
+                                     const uint32_t* __restrict__ skeys, const int* __restrict__ cs,
+                                     const int* __restrict__ ce, const R* __restrict__ stl_mag,
+                                     const R4<R>* __restrict__ stl_dir, const int* __restrict__ stl_id,
+                                     const R4<R>* __restrict__ drag_acc, const R4<R>* __restrict__ sph_dv,
+                                     const TriD<R>* __restrict__ tris,
+                                     const mpsr_tri_params* __restrict__ models,
+                                     const R* __restrict__ turb_nu, NearLds* Lw) {
+    const int t = blk * (int)blockDim.x + (int)threadIdx.x, t0 = t & ~63;
+    if (t0 >= N) return;   // the whole wave
+    const int s = t < N ? perm[t] : 0;
+    const R4<R> P = spos[t < N ? t : 0];
+    const R x = P.x, y = P.y, z = P.z;
+    const bool live = t < N && out.id[s] >= 0 && include(c, x, y, z);
+    const R4<R> V0 = svel[t < N ? t : 0];
+    const R re = c.re_lap;
+    ExplicitSums<R> S;
+    if constexpr (NEAR) {
+        for_near_mfma(
+            c, cs, ce, rel, skeys, t0, N, live, x, y, z, re, Lw[threadIdx.x >> 6],
+            [&](int q) { return PosVel<R>{spos[q], svel[q]}; },
+            [&](int, const PosVel<R>& r) {
+                const R d = dist3(x, y, z, r.p.x, r.p.y, r.p.z);
+                if (d < re) S.add(c, x, y, z, V0, r.p, r.v, d);
+            });
+    } else if (live) {
+        // per group of 4 candidates: the distances first, then the velocities of the hits, loaded
+        // together, then the sums in the canonical order
+        for_candidate_groups(c, cs, ce, spos, x, y, z, [&](int q0, const R4<R> (&Q)[4], int m) {
+            R dd[4];
+            bool hit[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                dd[u] = dist3(x, y, z, Q[u].x, Q[u].y, Q[u].z);
+                hit[u] = u < m && q0 + u != t && dd[u] < re;
+            }
+            R4<R> V[4];   // read only where hit[u]
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (hit[u]) V[u] = svel[q0 + u];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (hit[u]) S.add(c, x, y, z, V0, Q[u], V[u], dd[u]);
+        });
+    }
+    if (live) explicit_finish<R>(t, s, c, in, out, x, y, z, V0, S, stl_mag, stl_dir, stl_id, drag_acc, sph_dv, tris,
+                                 models, turb_nu);
+}
+template <typename R, bool NEAR>
+__global__ __launch_bounds__(NEAR ? kNearBlock : kMaxBlock, NEAR ? 3 : 1) void k_explicit(
+    int N, Consts<R> c, const int* __restrict__ perm, PState<R> in, PState<R> out, const R4<R>* __restrict__ spos,
+    const R4<R>* __restrict__ svel, RelPos rel, const uint32_t* __restrict__ skeys, const int* __restrict__ cs,
+    const int* __restrict__ ce, const R* __restrict__ stl_mag, const R4<R>* __restrict__ stl_dir,
+    const int* __restrict__ stl_id, const R4<R>* __restrict__ drag_acc, const R4<R>* __restrict__ sph_dv,
+    const TriD<R>* __restrict__ tris, const mpsr_tri_params* __restrict__ models, const R* __restrict__ turb_nu) {
     const int blk = xcd_block(N);
     if (blk < 0) return;
-    explicit_body<R>(blk, N, c, perm, in, out, spos, svel, cs, ce, stl_mag, stl_dir, stl_id, drag_acc, sph_dv, tris,
-                     models, turb_nu);
+    NearLds* L = nullptr;
+    if constexpr (NEAR) {
+        __shared__ NearLds lds[kNearBlock / 64];
+        L = lds;
+    }
+    explicit_body<R, NEAR>(blk, N, c, perm, in, out, spos, svel, rel, skeys, cs, ce, stl_mag, stl_dir, stl_id, drag_acc,
+                           sph_dv, tris, models, turb_nu, L);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -287,111 +342,80 @@ __device__ inline void list_tail(int* nbq, int lbase, int lane, int kept, int q1
 // scanning again; the fill forms their weights again from the positions, with the same operations.
 // Without PPE and with nbq given, the gradient-radius neighbours go to the list instead (nb_width
 // of them, nbn[t] their count, -1 for a skipped row), in walk order, for the corrector.
+// One wave per 64 sorted particles (for_near_mfma).
 template <typename R, bool PPE>
 __device__ inline void pnd_body(int blk, int N, Consts<R> c, int eos, const int* __restrict__ perm, PState<R> in,
-                                PState<R> out, const R4<R>* __restrict__ spos, R* __restrict__ spres,
+                                PState<R> out, const R4<R>* __restrict__ spos, R* __restrict__ spres, RelPos rel,
                                 const int* __restrict__ cs, const int* __restrict__ ce,
                                 const R* __restrict__ stl_mag, const int* __restrict__ stl_id,
                                 const uint32_t* __restrict__ skeys, int* __restrict__ active,
                                 int* __restrict__ rcnt, double* __restrict__ rdiag, int* __restrict__ rdir,
                                 int* __restrict__ nbq, int* __restrict__ nbn,
-                                int nb_width) {
-    const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= N) return;
-    const int s = perm[t];
-    const R4<R> P = spos[t];
+                                int nb_width, NearLds* Lw) {
+    const int t = blk * kNearBlock + (int)threadIdx.x, t0 = t & ~63;
+    if (t0 >= N) return;   // the whole wave
+    const int s = t < N ? perm[t] : 0;
+    const R4<R> P = spos[t < N ? t : 0];
     const R x = P.x, y = P.y, z = P.z;
-    auto dirichlet = [&]() {
-        if constexpr (PPE) {
-            active[t] = 0;
-            rcnt[t] = 0;
-            rdiag[t] = 1.0;
-            rdir[t] = 1;
-            nbn[t] = -1;
-        } else if (nbn) {
-            nbn[t] = -1;
-        }
-    };
-    if (!include(c, x, y, z)) {
-        in.p[s] = 0;
-        spres[t] = out.p[s];
-        dirichlet();
-        return;
-    }
-    int ci, cj, ck;
-    long long cid = -1;
-    if (cell_coords(c, x, y, z, ci, cj, ck)) cid = cell_of(c, ci, cj, ck);
-    if (cid < 0 || cid >= c.ncell) {
-        in.p[s] = 0;
-        spres[t] = out.p[s];
-        dirichlet();
-        return;
+    // a particle outside the zone or the grid has no neighbour sum
+    bool sums = t < N && include(c, x, y, z);
+    if (sums) {
+        int ci, cj, ck;
+        long long cid = -1;
+        if (cell_coords(c, x, y, z, ci, cj, ck)) cid = cell_of(c, ci, cj, ck);
+        sums = cid >= 0 && cid < c.ncell;
     }
     const R re = c.re_grad, mind = c.mind_grad;
     R dens = 0;
     int nl = 0;
     double wl = 0.0;
-    if constexpr (PPE) {
-        const R rl = c.re_lap, mindl = c.mind_lap;
-        const int lbase = (t >> 6) * 64 * nb_width, lane = t & 63;
-        int q0 = 0, q1 = 0, q2 = 0, q3 = 0;
-        // the root only for candidates inside 1.01 times the larger radius (sqrt14 errs by at most
-        // 0.18 %): a wave whose lanes all miss skips it
-        const R reach = (rl > re ? rl : re) * (R)1.01;
-        const R reach2 = reach * reach;
-        for_candidates_rec<8>(c, cs, ce, spos, x, y, z, t, [&](int q, const R4<R>& Q) {
-            const R d2 = (x - Q.x) * (x - Q.x) + (y - Q.y) * (y - Q.y) + (z - Q.z) * (z - Q.z);
-            if (!(d2 < reach2)) return;
-            const R d0 = build_sqrt(d2);
+    const int lbase = (t >> 6) * 64 * nb_width, lane = t & 63;
+    int q0 = 0, q1 = 0, q2 = 0, q3 = 0;
+    auto list = [&](int q) {
+        if (!nbq) return;   // EOS sums of a handle without a list
+        if (nl < nb_width) {
+            q0 = q1; q1 = q2; q2 = q3; q3 = q;
+            if ((nl & 3) == 3) quad_store(nbq + sell_at(lbase, lane, nl - 3), q0, q1, q2, q3);
+        }
+        ++nl;
+    };
+    const R rl = c.re_lap, mindl = c.mind_lap;
+    for_near_mfma(
+        c, cs, ce, rel, skeys, t0, N, sums, x, y, z, PPE && rl > re ? rl : re, Lw[threadIdx.x >> 6],
+        [&](int q) { return spos[q]; },
+        [&](int q, const R4<R>& Q) {
+            const R d0 = dist3(x, y, z, Q.x, Q.y, Q.z);
             if (d0 < re) {
                 R d = d0;
                 if (d < mind) d = mind;
-                dens = dens + weight(re, d);
+                dens = dens + (re / d - 1);   // weight(re, d) for 0 < d < re
+                if constexpr (!PPE) list(q);
             }
-            if (d0 < rl) {
-                R d = d0;
-                if (d < mindl) d = mindl;
-                const R w = weight(rl, d);
-                wl += (double)w;
-                if (nl < nb_width) {
-                    q0 = q1; q1 = q2; q2 = q3; q3 = q;
-                    if ((nl & 3) == 3) {
-                        const int e = sell_at(lbase, lane, nl - 3);
-                        quad_store(nbq + e, q0, q1, q2, q3);
-                    }
+            if constexpr (PPE) {
+                if (d0 < rl) {
+                    R d = d0;
+                    if (d < mindl) d = mindl;
+                    const R w = rl / d - 1;
+                    wl += (double)w;
+                    list(q);
                 }
-                ++nl;
             }
         });
-        list_tail(nbq, lbase, lane, nl < nb_width ? nl : nb_width, q1, q2, q3);
-    } else if (nbq) {
-        const int lbase = (t >> 6) * 64 * nb_width, lane = t & 63;
-        int q0 = 0, q1 = 0, q2 = 0, q3 = 0;
-        for_near_candidates(c, cs, ce, spos, x, y, z, t, re, [&](int q) {
-            const R4<R> Q = spos[q];
-            R d = dist3(x, y, z, Q.x, Q.y, Q.z);
-            if (d < re) {
-                if (d < mind) d = mind;
-                dens = dens + weight(re, d);
-                if (nl < nb_width) {
-                    q0 = q1; q1 = q2; q2 = q3; q3 = q;
-                    if ((nl & 3) == 3) quad_store(nbq + sell_at(lbase, lane, nl - 3), q0, q1, q2, q3);
-                }
-                ++nl;
-            }
-        });
-        list_tail(nbq, lbase, lane, nl < nb_width ? nl : nb_width, q1, q2, q3);
-        nbn[t] = nl;
-    } else {
-        for_candidates_within(c, cs, ce, x, y, z, t, re, [&](int q) {
-            const R4<R> Q = spos[q];
-            R d = dist3(x, y, z, Q.x, Q.y, Q.z);
-            if (d < re) {
-                if (d < mind) d = mind;
-                dens = dens + weight(re, d);
-            }
-        });
+    if (t >= N) return;
+    if (!sums) {
+        in.p[s] = 0;
+        spres[t] = out.p[s];
+        if constexpr (PPE) {
+            active[t] = 0;
+            rcnt[t] = 0;
+            rdiag[t] = 1.0;
+            rdir[t] = 1;
+        }
+        if (nbn) nbn[t] = -1;
+        return;
     }
+    if (nbq) list_tail(nbq, lbase, lane, nl < nb_width ? nl : nb_width, q1, q2, q3);
+    if (!PPE && nbn) nbn[t] = nl;
     const R riw = stl_mag[t];
     R ww = 0;
     const int tid = stl_id[t];
@@ -421,16 +445,19 @@ __device__ inline void pnd_body(int blk, int N, Consts<R> c, int eos, const int*
     spres[t] = pout;
 }
 template <typename R, bool PPE>
-__global__ __launch_bounds__(kMaxBlock) void k_pnd(int N, Consts<R> c, int eos, const int* __restrict__ perm, PState<R> in,
+__global__ __launch_bounds__(kNearBlock, 3) void k_pnd(int N, Consts<R> c, int eos, const int* __restrict__ perm, PState<R> in,
                                               PState<R> out, const R4<R>* __restrict__ spos, R* __restrict__ spres,
-                                              const int* __restrict__ cs, const int* __restrict__ ce,
+                                              RelPos rel, const int* __restrict__ cs, const int* __restrict__ ce,
                                               const R* __restrict__ stl_mag, const int* __restrict__ stl_id,
                                               const uint32_t* __restrict__ skeys, int* __restrict__ active,
                                               int* __restrict__ rcnt, double* __restrict__ rdiag, int* __restrict__ rdir,
                                               int* __restrict__ nbq, int* __restrict__ nbn,
                                               int nb_width) {
-    pnd_body<R, PPE>(blockIdx.x, N, c, eos, perm, in, out, spos, spres, cs, ce, stl_mag, stl_id, skeys, active, rcnt,
-                     rdiag, rdir, nbq, nbn, nb_width);
+    __shared__ NearLds L[kNearBlock / 64];
+    const int blk = xcd_block(N);
+    if (blk < 0) return;
+    pnd_body<R, PPE>(blk, N, c, eos, perm, in, out, spos, spres, rel, cs, ce, stl_mag, stl_id, skeys, active, rcnt,
+                     rdiag, rdir, nbq, nbn, nb_width, L);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -598,47 +625,50 @@ __global__ __launch_bounds__(256) void k_nbr_fill(int N, Consts<R> c, R re, cons
 // [MinWallTemperature, MaxWallTemperature]; the out arrays get T, A T + B and the enthalpy term.
 template <typename R>
 __device__ inline void thermal_body(int blk, int N, Consts<R> c, const int* __restrict__ perm, PState<R> in,
-                                    PState<R> out, const R4<R>* __restrict__ spos,
-                                    const int* __restrict__ cs, const int* __restrict__ ce,
+                                    PState<R> out, const R4<R>* __restrict__ spos, RelPos rel,
+                                    const uint32_t* __restrict__ skeys, const int* __restrict__ cs, const int* __restrict__ ce,
                                     const R* __restrict__ stl_mag, const int* __restrict__ stl_id,
                                     const TriD<R>* __restrict__ tris,
                                     const mpsr_tri_params* __restrict__ models,
                                     const R* __restrict__ drag_temp, const int* __restrict__ step_base,
-                                    const int* __restrict__ step_ctr, int thermal_step) {
+                                    const int* __restrict__ step_ctr, int thermal_step, NearLds* Lw) {
     if (step_ctr && ((*step_base + *step_ctr) % thermal_step) != 0) return;
-    const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= N) return;
-    const int s = perm[t];
-    if (out.id[s] < 0) return;
-    const R4<R> P = spos[t];
-    if (!include(c, P.x, P.y, P.z)) return;
-    int ci, cj, ck;
-    if (!cell_coords(c, P.x, P.y, P.z, ci, cj, ck)) return;
-    const long long cid = cell_of(c, ci, cj, ck);
-    if (cid < 0 || cid >= c.ncell) return;
-    const R t0 = in.temp[s];
+    const int t = blk * kNearBlock + (int)threadIdx.x, t0 = t & ~63;
+    if (t0 >= N) return;   // the whole wave
+    const int s = t < N ? perm[t] : 0;
+    const R4<R> P = spos[t < N ? t : 0];
+    bool live = t < N && out.id[s] >= 0 && include(c, P.x, P.y, P.z);
+    if (live) {
+        int ci, cj, ck;
+        live = cell_coords(c, P.x, P.y, P.z, ci, cj, ck);
+        const long long cid = live ? cell_of(c, ci, cj, ck) : -1;
+        live = cid >= 0 && cid < c.ncell;
+    }
+    const R t0_ = in.temp[s];
     const R re = c.re_temp, mind = c.mind_temp;
     R hf = 0, hw = 0;
-    for_candidates_rec_within<4>(c, cs, ce, spos, P.x, P.y, P.z, t, re, [&](int q, const R4<R>& Q) {
-        R d = dist3(P.x, P.y, P.z, Q.x, Q.y, Q.z);
-        if (d < re) {
+    for_near_mfma(
+        c, cs, ce, rel, skeys, t0, N, live, P.x, P.y, P.z, re, Lw[threadIdx.x >> 6], [&](int q) { return spos[q]; },
+        [&](int q, const R4<R>& Q) {
+            R d = dist3(P.x, P.y, P.z, Q.x, Q.y, Q.z);
+            if (!(d < re)) return;
             if (d < mind) d = mind;
-            const R num = (in.temp[perm[q]] - t0) * weight(re, d);
+            const R num = (in.temp[perm[q]] - t0_) * weight(re, d);
             const R den = d * d * (c.inv_kf + c.rf / d);
             hf = hf + num / den;
-        }
-    });
+        });
+    if (!live) return;
     const R dist = stl_mag[t];
     const int tid = stl_id[t];
     if (tid >= 0 && tid < c.ntri && dist > 0 && dist < re) {
         const mpsr_tri_params& m = models[tris[tid].model];
         const R rw = (R)m.WallThermalResistivity, kw = (R)m.WallThermalConductivity;
         const R k = (R)2 * c.kf * kw / (c.kf + kw);
-        const R num = ((R)m.Temperature - t0) * ztable_eval(kZgrad, dist, c.l0);
+        const R num = ((R)m.Temperature - t0_) * ztable_eval(kZgrad, dist, c.l0);
         const R den = dist * dist * ((R)1 / k + rw / dist);
         hw = num / den;
     }
-    R temp = t0;
+    R temp = t0_;
     if (c.has_drag) temp = temp + drag_temp[t];
     R comb = 0;
     if (fabs(hf) > (R)FLT_EPSILON) comb = comb + hf;
@@ -651,18 +681,19 @@ __device__ inline void thermal_body(int blk, int N, Consts<R> c, const int* __re
     out.solid[s] = c.enth * comb;
 }
 template <typename R>
-__global__ __launch_bounds__(kMaxBlock) void k_thermal(int N, Consts<R> c, const int* __restrict__ perm, PState<R> in,
-                                                    PState<R> out, const R4<R>* __restrict__ spos,
-                                                    const int* __restrict__ cs, const int* __restrict__ ce,
-                                                    const R* __restrict__ stl_mag, const int* __restrict__ stl_id,
-                                                    const TriD<R>* __restrict__ tris,
+__global__ __launch_bounds__(kNearBlock, 3) void k_thermal(int N, Consts<R> c, const int* __restrict__ perm, PState<R> in,
+                                                    PState<R> out, const R4<R>* __restrict__ spos, RelPos rel,
+                                                    const uint32_t* __restrict__ skeys, const int* __restrict__ cs,
+                                                    const int* __restrict__ ce, const R* __restrict__ stl_mag,
+                                                    const int* __restrict__ stl_id, const TriD<R>* __restrict__ tris,
                                                     const mpsr_tri_params* __restrict__ models,
                                                     const R* __restrict__ drag_temp, const int* __restrict__ step_base,
                                                     const int* __restrict__ step_ctr, int thermal_step) {
+    __shared__ NearLds L[kNearBlock / 64];
     const int blk = xcd_block(N);
     if (blk < 0) return;
-    thermal_body<R>(blk, N, c, perm, in, out, spos, cs, ce, stl_mag, stl_id, tris, models, drag_temp, step_base,
-                    step_ctr, thermal_step);
+    thermal_body<R>(blk, N, c, perm, in, out, spos, rel, skeys, cs, ce, stl_mag, stl_id, tris, models, drag_temp,
+                    step_base, step_ctr, thermal_step, L);
 }
 
 template <typename R> void launch_bin_hash(const Dev<R>& d, hipStream_t st) {
@@ -677,8 +708,8 @@ template <typename R> void launch_bin_ranges(Dev<R>& d, hipStream_t st) {
     d.perm = which ? d.sort.v1 : d.vals;
     fill_int(d.cell_start, -1, d.c.ncell, st);
     fill_int(d.cell_end, -1, d.c.ncell, st);
-    hipLaunchKernelGGL(k_bin_ranges<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c.ncell, d.skeys,
-                       d.perm, d.cell_start, d.cell_end, d.in, d.spos, d.svel);
+    hipLaunchKernelGGL(k_bin_ranges<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.skeys,
+                       d.perm, d.cell_start, d.cell_end, d.in, d.spos, d.svel, d.rel);
 }
 // ---------------------------------------------------------------------------------------------
 // CalcTurbulenceViscosity_Kernel (radix DeviceProcess_Kernel.h:1273-1476): the velocity gradient
@@ -692,36 +723,36 @@ template <typename R> void launch_bin_ranges(Dev<R>& d, hipStream_t st) {
 template <typename R>
 __device__ inline void turbulence_body(int blk, int N, Consts<R> c, const int* __restrict__ perm,
                                        PState<R> out, const R4<R>* __restrict__ spos,
-                                       const R4<R>* __restrict__ svel, const int* __restrict__ cs,
+                                       const R4<R>* __restrict__ svel, RelPos rel,
+                                       const uint32_t* __restrict__ skeys, const int* __restrict__ cs,
                                        const int* __restrict__ ce, const R* __restrict__ stl_mag,
-                                       R* __restrict__ turb_nu, R* __restrict__ turb_k) {
-    const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= N) return;
-    const int s = perm[t];
-    if (out.id[s] < 0) return;
-    const R4<R> P = spos[t];
+                                       R* __restrict__ turb_nu, R* __restrict__ turb_k, NearLds* Lw) {
+    const int t = blk * kNearBlock + (int)threadIdx.x, t0 = t & ~63;
+    if (t0 >= N) return;   // the whole wave
+    const int s = t < N ? perm[t] : 0;
+    const bool alive = t < N && out.id[s] >= 0;
+    const R4<R> P = spos[t < N ? t : 0];
     const R x = P.x, y = P.y, z = P.z;
-    if (!include(c, x, y, z)) {
-        turb_nu[s] = 0;
-        return;
+    const bool inside = include(c, x, y, z);
+    bool sums = alive && inside;
+    if (sums) {
+        int ci, cj, ck;
+        long long cid = -1;
+        if (cell_coords(c, x, y, z, ci, cj, ck)) cid = cell_of(c, ci, cj, ck);
+        sums = cid >= 0 && cid < c.ncell;
     }
-    int ci, cj, ck;
-    long long cid = -1;
-    if (cell_coords(c, x, y, z, ci, cj, ck)) cid = cell_of(c, ci, cj, ck);
-    if (cid < 0 || cid >= c.ncell) {
-        turb_nu[s] = 0;
-        turb_k[s] = 0;
-        return;
-    }
-    const R4<R> V0 = svel[t];
+    const R4<R> V0 = svel[t < N ? t : 0];
     R txx = 0, txy = 0, txz = 0, tyx = 0, tyy = 0, tyz = 0, tzx = 0, tzy = 0, tzz = 0;
     const R re = c.re_grad, mind = c.mind_grad;
-    for_candidates_rec_within<4>(c, cs, ce, spos, x, y, z, t, re, [&](int q, const R4<R>& Q) {
-        R d = dist3(x, y, z, Q.x, Q.y, Q.z);
-        if (d < re) {
+    for_near_mfma(
+        c, cs, ce, rel, skeys, t0, N, sums, x, y, z, re, Lw[threadIdx.x >> 6],
+        [&](int q) { return PosVel<R>{spos[q], svel[q]}; },
+        [&](int, const PosVel<R>& r) {
+            const R4<R>&Q = r.p, &V1 = r.v;
+            R d = dist3(x, y, z, Q.x, Q.y, Q.z);
+            if (!(d < re)) return;
             if (d < mind) d = mind;
-            const R w = weight(re, d);
-            const R4<R> V1 = svel[q];
+            const R w = re / d - 1;   // weight(re, d) for 0 < d < re
             const R ux = V1.x - V0.x, uy = V1.y - V0.y, uz = V1.z - V0.z;
             const R rx = Q.x - x, ry = Q.y - y, rz = Q.z - z;
             const R dd = d * d;
@@ -740,8 +771,13 @@ __device__ inline void turbulence_body(int blk, int N, Consts<R> c, const int* _
                 tyx = tyx + uy * rx * w / dd; tyy = tyy + uy * ry * w / dd; tyz = tyz + uy * rz * w / dd;
                 tzx = tzx + uz * rx * w / dd; tzy = tzy + uz * ry * w / dd; tzz = tzz + uz * rz * w / dd;
             }
-        }
-    });
+        });
+    if (!alive) return;
+    if (!sums) {
+        turb_nu[s] = 0;
+        if (inside) turb_k[s] = 0;
+        return;
+    }
     const R g = c.turb_g;
     txx = g * txx; txy = g * txy; txz = g * txz;
     tyx = g * tyx; tyy = g * tyy; tyz = g * tyz;
@@ -761,26 +797,30 @@ __device__ inline void turbulence_body(int blk, int N, Consts<R> c, const int* _
     turb_k[s] = k;
 }
 template <typename R>
-__global__ __launch_bounds__(kMaxBlock) void k_turbulence(int N, Consts<R> c, const int* __restrict__ perm,
+__global__ __launch_bounds__(kNearBlock, 3) void k_turbulence(int N, Consts<R> c, const int* __restrict__ perm,
                                                      PState<R> out, const R4<R>* __restrict__ spos,
-                                                     const R4<R>* __restrict__ svel, const int* __restrict__ cs,
+                                                     const R4<R>* __restrict__ svel, RelPos rel,
+                                                     const uint32_t* __restrict__ skeys, const int* __restrict__ cs,
                                                      const int* __restrict__ ce, const R* __restrict__ stl_mag,
                                                      R* __restrict__ turb_nu, R* __restrict__ turb_k) {
+    __shared__ NearLds L[kNearBlock / 64];
     const int blk = xcd_block(N);
     if (blk < 0) return;
-    turbulence_body<R>(blk, N, c, perm, out, spos, svel, cs, ce, stl_mag, turb_nu, turb_k);
+    turbulence_body<R>(blk, N, c, perm, out, spos, svel, rel, skeys, cs, ce, stl_mag, turb_nu, turb_k, L);
 }
 
 template <typename R> void launch_explicit(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
-    hipLaunchKernelGGL(k_explicit<R>, dim3(xcd_grid(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.perm, d.in, d.out,
-                       d.spos, d.svel, d.cell_start, d.cell_end, d.stl_mag, d.stl_dir, d.stl_id, d.drag_acc, d.sph_dv,
-                       d.tris, d.models, d.turb_nu);
+    const bool near = near_explicit<R>(d.N);
+    const int block = near ? kNearBlock : d.block;
+    hipLaunchKernelGGL((near ? k_explicit<R, true> : k_explicit<R, false>), dim3(xcd_grid(d.N, block)), dim3(block), 0,
+                       st, d.N, d.c, d.perm, d.in, d.out, d.spos, d.svel, d.rel, d.skeys, d.cell_start, d.cell_end,
+                       d.stl_mag, d.stl_dir, d.stl_id, d.drag_acc, d.sph_dv, d.tris, d.models, d.turb_nu);
 }
 template <typename R> void launch_turbulence(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0 || !d.turb_nu) return;
-    hipLaunchKernelGGL(k_turbulence<R>, dim3(xcd_grid(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.perm, d.out,
-                       d.spos, d.svel, d.cell_start, d.cell_end, d.stl_mag, d.turb_nu, d.turb_k);
+    hipLaunchKernelGGL(k_turbulence<R>, dim3(xcd_grid(d.N, kNearBlock)), dim3(kNearBlock), 0, st, d.N, d.c, d.perm, d.out,
+                       d.spos, d.svel, d.rel, d.skeys, d.cell_start, d.cell_end, d.stl_mag, d.turb_nu, d.turb_k);
 }
 template <typename R> void launch_relocate(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
@@ -790,15 +830,15 @@ template <typename R>
 void launch_pnd_ppe(const Dev<R>& d, int* active, int* cnt, double* diag, int* dir, int* nbq, int* nbn,
                     int nb_width, hipStream_t st) {
     if (d.N <= 0) return;
-    hipLaunchKernelGGL((k_pnd<R, true>), dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, 0, d.perm, d.in,
-                       d.out, d.spos, d.spres, d.cell_start, d.cell_end, d.stl_mag, d.stl_id, d.skeys, active, cnt, diag,
+    hipLaunchKernelGGL((k_pnd<R, true>), dim3(xcd_grid(d.N, kNearBlock)), dim3(kNearBlock), 0, st, d.N, d.c, 0, d.perm,
+                       d.in, d.out, d.spos, d.spres, d.rel, d.cell_start, d.cell_end, d.stl_mag, d.stl_id, d.skeys, active, cnt, diag,
                        dir, nbq, nbn, nb_width);
 }
 template <typename R> void launch_pnd(const Dev<R>& d, int eos, hipStream_t st) {
     if (d.N <= 0) return;
-    hipLaunchKernelGGL((k_pnd<R, false>), dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, eos, d.perm, d.in, d.out,
-                       d.spos, d.spres, d.cell_start, d.cell_end, d.stl_mag, d.stl_id, nullptr, nullptr, nullptr,
-                       nullptr, nullptr, d.gnb_q, d.gnb_n, kGradWidth);
+    hipLaunchKernelGGL((k_pnd<R, false>), dim3(xcd_grid(d.N, kNearBlock)), dim3(kNearBlock), 0, st, d.N, d.c, eos, d.perm,
+                       d.in, d.out, d.spos, d.spres, d.rel, d.cell_start, d.cell_end, d.stl_mag, d.stl_id, d.skeys,
+                       nullptr, nullptr, nullptr, nullptr, d.gnb_q, d.gnb_n, kGradWidth);
 }
 template <typename R> void launch_gradient(const Dev<R>& d, hipStream_t st, NbList nb) {
     if (d.N <= 0) return;
@@ -809,8 +849,8 @@ template <typename R> void launch_gradient(const Dev<R>& d, hipStream_t st, NbLi
 template <typename R>
 void launch_thermal(const Dev<R>& d, const int* step_base, const int* step_ctr, int thermal_step, hipStream_t st) {
     if (d.N <= 0) return;
-    hipLaunchKernelGGL(k_thermal<R>, dim3(xcd_grid(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.perm, d.in, d.out,
-                       d.spos, d.cell_start, d.cell_end, d.stl_mag, d.stl_id, d.tris, d.models, d.drag_temp, step_base,
+    hipLaunchKernelGGL(k_thermal<R>, dim3(xcd_grid(d.N, kNearBlock)), dim3(kNearBlock), 0, st, d.N, d.c, d.perm, d.in, d.out,
+                       d.spos, d.rel, d.skeys, d.cell_start, d.cell_end, d.stl_mag, d.stl_id, d.tris, d.models, d.drag_temp, step_base,
                        step_ctr, thermal_step > 0 ? thermal_step : 1);
 }
 template <typename R> void launch_neighbor_count(const Dev<R>& d, R re, int* counts, hipStream_t st) {
@@ -836,15 +876,21 @@ template <typename R> struct OpBinRanges {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
-        bin_ranges_body<R>(b, d.N, d.c.ncell, d.skeys, d.perm, d.cell_start, d.cell_end, d.in, d.spos, d.svel);
+        bin_ranges_body<R>(b, d.N, d.c, d.skeys, d.perm, d.cell_start, d.cell_end, d.in, d.spos, d.svel, d.rel);
     }
 };
-template <typename R> struct OpExplicit {
+template <typename R, bool NEAR> struct OpExplicit {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
-        explicit_body<R>(b, d.N, d.c, d.perm, d.in, d.out, d.spos, d.svel, d.cell_start, d.cell_end, d.stl_mag,
-                         d.stl_dir, d.stl_id, d.drag_acc, d.sph_dv, d.tris, d.models, d.turb_nu);
+        NearLds* L = nullptr;
+        if constexpr (NEAR) {
+            __shared__ NearLds lds[kNearBlock / 64];
+            L = lds;
+        }
+        explicit_body<R, NEAR>(b, d.N, d.c, d.perm, d.in, d.out, d.spos, d.svel, d.rel, d.skeys, d.cell_start,
+                               d.cell_end, d.stl_mag, d.stl_dir, d.stl_id, d.drag_acc, d.sph_dv, d.tris, d.models,
+                               d.turb_nu, L);
     }
 };
 template <typename R> struct OpRelocate {
@@ -858,8 +904,10 @@ template <typename R> struct OpPndEos {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
-        pnd_body<R, false>(b, d.N, d.c, 1, d.perm, d.in, d.out, d.spos, d.spres, d.cell_start, d.cell_end, d.stl_mag,
-                           d.stl_id, nullptr, nullptr, nullptr, nullptr, nullptr, d.gnb_q, d.gnb_n, kGradWidth);
+        __shared__ NearLds L[kNearBlock / 64];
+        pnd_body<R, false>(b, d.N, d.c, 1, d.perm, d.in, d.out, d.spos, d.spres, d.rel, d.cell_start, d.cell_end,
+                           d.stl_mag, d.stl_id, d.skeys, nullptr, nullptr, nullptr, nullptr, d.gnb_q, d.gnb_n,
+                           kGradWidth, L);
     }
 };
 template <typename R> struct OpGradient {
@@ -875,16 +923,18 @@ template <typename R> struct OpThermal {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
-        thermal_body<R>(b, d.N, d.c, d.perm, d.in, d.out, d.spos, d.cell_start, d.cell_end, d.stl_mag, d.stl_id,
-                        d.tris, d.models, d.drag_temp, d.step_base, d.step_ctr, d.thermal_step);
+        __shared__ NearLds L[kNearBlock / 64];
+        thermal_body<R>(b, d.N, d.c, d.perm, d.in, d.out, d.spos, d.rel, d.skeys, d.cell_start, d.cell_end, d.stl_mag,
+                        d.stl_id, d.tris, d.models, d.drag_temp, d.step_base, d.step_ctr, d.thermal_step, L);
     }
 };
 template <typename R> struct OpTurbulence {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
-        turbulence_body<R>(b, d.N, d.c, d.perm, d.out, d.spos, d.svel, d.cell_start, d.cell_end, d.stl_mag,
-                           d.turb_nu, d.turb_k);
+        __shared__ NearLds L[kNearBlock / 64];
+        turbulence_body<R>(b, d.N, d.c, d.perm, d.out, d.spos, d.svel, d.rel, d.skeys, d.cell_start, d.cell_end,
+                           d.stl_mag, d.turb_nu, d.turb_k, L);
     }
 };
 template <typename R> struct OpPndPpe {
@@ -893,12 +943,13 @@ template <typename R> struct OpPndPpe {
     __device__ void operator()(int j, int b) const {
         const PndRows<R>& q = rows[j];
         const Dev<R>& d = dv[q.dev];
-        pnd_body<R, true>(b, d.N, d.c, 0, d.perm, d.in, d.out, d.spos, d.spres, d.cell_start, d.cell_end, d.stl_mag,
-                          d.stl_id, d.skeys, q.active, q.cnt, q.diag, q.dir, q.nbq, q.nbn, q.nb_width);
+        __shared__ NearLds L[kNearBlock / 64];
+        pnd_body<R, true>(b, d.N, d.c, 0, d.perm, d.in, d.out, d.spos, d.spres, d.rel, d.cell_start, d.cell_end,
+                          d.stl_mag, d.stl_id, d.skeys, q.active, q.cnt, q.diag, q.dir, q.nbq, q.nbn, q.nb_width, L);
     }
 };
 template <typename R> void launch_pnd_ppe_b(const BatchLaunch<R>& b, const PndRows<R>* rows, WorkList p, hipStream_t st) {
-    launch_batched<kMaxBlock>(OpPndPpe<R>{b.devs, rows}, p, b.block, st);
+    launch_batched<kNearBlock>(OpPndPpe<R>{b.devs, rows}, p, kNearBlock, st);
 }
 template <typename R> void launch_bin_hash_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
     launch_batched<kMaxBlock>(OpBinHash<R>{b.devs}, p, b.block, st);
@@ -906,23 +957,25 @@ template <typename R> void launch_bin_hash_b(const BatchLaunch<R>& b, WorkList p
 template <typename R> void launch_bin_ranges_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
     launch_batched<kMaxBlock>(OpBinRanges<R>{b.devs}, p, b.block, st);
 }
-template <typename R> void launch_explicit_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
-    launch_batched<kMaxBlock>(OpExplicit<R>{b.devs}, p, b.block, st);
+template <typename R> void launch_explicit_b(const BatchLaunch<R>& b, WorkList p, WorkList near, hipStream_t st) {
+    if (near_explicit<R>((long long)near.n * kNearBlock))
+        launch_batched<kNearBlock>(OpExplicit<R, true>{b.devs}, near, kNearBlock, st);
+    else launch_batched<kMaxBlock>(OpExplicit<R, false>{b.devs}, p, b.block, st);
 }
 template <typename R> void launch_relocate_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
     launch_batched<kMaxBlock>(OpRelocate<R>{b.devs}, p, b.block, st);
 }
 template <typename R> void launch_pnd_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
-    launch_batched<kMaxBlock>(OpPndEos<R>{b.devs}, p, b.block, st);
+    launch_batched<kNearBlock>(OpPndEos<R>{b.devs}, p, kNearBlock, st);
 }
 template <typename R> void launch_gradient_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
     launch_batched<kMaxBlock>(OpGradient<R>{b.devs}, p, b.block, st);
 }
 template <typename R> void launch_thermal_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
-    launch_batched<kMaxBlock>(OpThermal<R>{b.devs}, p, b.block, st);
+    launch_batched<kNearBlock>(OpThermal<R>{b.devs}, p, kNearBlock, st);
 }
 template <typename R> void launch_turbulence_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
-    launch_batched<kMaxBlock>(OpTurbulence<R>{b.devs}, p, b.block, st);
+    launch_batched<kNearBlock>(OpTurbulence<R>{b.devs}, p, kNearBlock, st);
 }
 
 #define MPSR_INSTANTIATE(R)                                                                   \
@@ -939,7 +992,7 @@ template <typename R> void launch_turbulence_b(const BatchLaunch<R>& b, WorkList
     template void launch_neighbor_fill<R>(const Dev<R>&, R, const int*, int*, hipStream_t);   \
     template void launch_bin_hash_b<R>(const BatchLaunch<R>&, WorkList, hipStream_t);         \
     template void launch_bin_ranges_b<R>(const BatchLaunch<R>&, WorkList, hipStream_t);       \
-    template void launch_explicit_b<R>(const BatchLaunch<R>&, WorkList, hipStream_t);         \
+    template void launch_explicit_b<R>(const BatchLaunch<R>&, WorkList, WorkList, hipStream_t); \
     template void launch_relocate_b<R>(const BatchLaunch<R>&, WorkList, hipStream_t);         \
     template void launch_pnd_b<R>(const BatchLaunch<R>&, WorkList, hipStream_t);              \
     template void launch_gradient_b<R>(const BatchLaunch<R>&, WorkList, hipStream_t);         \

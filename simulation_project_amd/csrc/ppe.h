@@ -53,7 +53,7 @@ template <typename R> PpeBatch<R>* ppe_batch_create();
 template <typename R> void ppe_batch_destroy(PpeBatch<R>* b);
 template <typename R>
 mpsr_status ppe_batch_build(PpeBatch<R>* b, PpeSolver<R>* const* solvers, const int* dev, const Dev<R>* host_devs,
-                            const mpsr_ppe_options* opts, int n, int block);
+                            const mpsr_ppe_options* opts, int n);
 template <typename R> void ppe_batch_pnd(PpeBatch<R>* b, const BatchLaunch<R>& bl, hipStream_t st);
 template <typename R> void ppe_batch_head(PpeBatch<R>* b, const BatchLaunch<R>& bl, int iters, hipStream_t st);
 template <typename R> void ppe_batch_iterate(PpeBatch<R>* b, int iters, hipStream_t st);

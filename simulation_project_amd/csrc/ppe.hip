@@ -2921,7 +2921,7 @@ template <typename R> void ppe_batch_destroy(PpeBatch<R>* b) {
 
 template <typename R>
 mpsr_status ppe_batch_build(PpeBatch<R>* b, PpeSolver<R>* const* solvers, const int* dev, const Dev<R>* host_devs,
-                            const mpsr_ppe_options* opts, int n, int block) {
+                            const mpsr_ppe_options* opts, int n) {
     const bool first = b->views == nullptr;
     if (!first && n != b->n) return MPSR_PARAMERR;
     b->n = n;
@@ -2984,7 +2984,7 @@ mpsr_status ppe_batch_build(PpeBatch<R>* b, PpeSolver<R>* const* solvers, const 
         v.flags = b->flags + 2 * j;
         b->hv[j] = v;
         rows[j] = PndRows<R>{dev[j], s->active, s->cnt, s->diag, s->dir, s->nbq, s->nbn, NB_WIDTH};
-        for (int k = 0; k < (int)grid_for(N, block); ++k) pnd.push_back(make_int2(j, k));
+        for (int k = 0; k < (int)grid_for(N, kNearBlock); ++k) pnd.push_back(make_int2(j, k));
         for (int k = 0; k < (int)grid_for((long long)d.c.ncell + 1, PB); ++k) cells.push_back(make_int2(j, k));
         for (int k = 0; k < (int)grid_for(N, SELL_SIGMA); ++k) win.push_back(make_int2(j, k));
         for (int k = 0; k < v.nb; ++k) vec.push_back(make_int2(j, k));
@@ -3129,7 +3129,7 @@ template <typename R> mpsr_status ppe_batch_finish(PpeBatch<R>* b, int* failed, 
     template PpeBatch<R>* ppe_batch_create<R>();                                                                    \
     template void ppe_batch_destroy<R>(PpeBatch<R>*);                                                              \
     template mpsr_status ppe_batch_build<R>(PpeBatch<R>*, PpeSolver<R>* const*, const int*, const Dev<R>*,          \
-                                            const mpsr_ppe_options*, int, int);                                    \
+                                            const mpsr_ppe_options*, int);                                    \
     template void ppe_batch_pnd<R>(PpeBatch<R>*, const BatchLaunch<R>&, hipStream_t);                              \
     template void ppe_batch_head<R>(PpeBatch<R>*, const BatchLaunch<R>&, int, hipStream_t);                        \
     template void ppe_batch_iterate<R>(PpeBatch<R>*, int, hipStream_t);                                            \
