@@ -553,6 +553,7 @@ template <typename R> struct Engine : EngineBase {
         for (int k = 1; k < kMarchTab; ++k) tab[k] = tab[k - 1] + d.c.cell;
         ALLOC(d.march_tab, kMarchTab);
         HIPC(hipMemcpy(d.march_tab, tab.data(), sizeof(R) * kMarchTab, hipMemcpyHostToDevice));
+        ALLOC(d.tri_sph, std::max(1, d.ntri));
         ALLOC(d.tri_emit, d.ntri + 1); ALLOC(d.tri_off, d.ntri + 1);
         ALLOC(d.pair_n, 1); ALLOC(d.uniq_n, 1); ALLOC(d.overflow, 1);
         HIPC(hipMemset(d.overflow, 0, sizeof(int)));
@@ -1512,14 +1513,14 @@ template <typename R> struct BatchGroup {
         const BatchLaunch<R> b = launch();
         bin(st);
         tri(st);
-        launch_stl_distance_b(b, wp, st);
+        launch_stl_distance_b(b, wnear, st);
         launch_drag_b(b, wdrag, st);
         launch_thermal_b(b, wtherm, st);
         launch_turbulence_b(b, wturb, st);
         launch_explicit_b(b, wp, wnear, st);
         launch_relocate_b(b, wp, st);
         bin(st);
-        launch_stl_distance_b(b, wp, st);
+        launch_stl_distance_b(b, wnear, st);
         launch_pnd_b(b, wp_eos, st);
         if (pb) {
             ppe_batch_pnd(pb, b, st);

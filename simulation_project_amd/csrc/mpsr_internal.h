@@ -136,10 +136,14 @@ template <typename R> struct PState {
     R *p, *n, *temp, *nu, *solid;
 };
 
-// most triangles of a per-cell triangle walk (nearest_triangle_listed); a walk entry's key keeps
+// most triangles of a per-cell triangle walk (nearest_triangle_wave); a walk entry's key keeps
 // the walk position in its low 10 bits
 static constexpr int kStencilTris = 1024;
 static constexpr unsigned kWalkPosMask = 1023u;
+// pairs of a wave's nearest-triangle queue beyond which it is tested
+static constexpr int kNearestQueue = 192;
+// longest triangle lists that the lanes of a wave of few points walk each for itself
+static constexpr int kNearestShort = 16;
 
 // Triangle record on the device: three vertices, the stored normal, the model, the model's
 // drag flag.  64 B for float, 112 B for double.
@@ -160,6 +164,12 @@ template <typename R> struct RotCoef {
 
 // ---- wave64 / block primitives --------------------------------------------------------------
 __device__ inline int lane_id() { return (int)(threadIdx.x & 63); }
+
+// orders a wave's LDS accesses before it against those after it (its own only)
+__device__ inline void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 __device__ inline int wave_inclusive_scan(int v) {
     const int lane = lane_id();
@@ -418,6 +428,7 @@ template <typename R> struct Dev {
     RotCoef<R>* rot = nullptr;        // [nmodel] for the current step, or the table base when
     const int* step_ctr = nullptr;    // ... this device step counter picks the row (graph replays)
     R* march_tab = nullptr;           // [kMarchTab] distances of a wall march: 0, then + cell each
+    float4* tri_sph = nullptr;        // [ntri] spheres around the triangles as last binned (tri_sphere)
     int* tri_emit = nullptr;          // [ntri + 1] emitted cell count per triangle
     int* tri_off = nullptr;           // [ntri + 1]
     int* pair_n = nullptr;            // device count of emitted (cell, triangle) pairs

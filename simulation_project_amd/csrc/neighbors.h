@@ -156,9 +156,6 @@ struct NearLds {
     int meta[kNearWords];
 };
 
-// orders a wave's LDS accesses before it against those after it (its own only)
-__device__ inline void wave_lds_sync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
-
 template <typename R, typename Load, typename Use>
 __device__ inline void for_near_mfma(const Consts<R>& c, const int* __restrict__ cs, const int* __restrict__ ce,
                                      const RelPos& rel, const uint32_t* __restrict__ skeys, int t0,

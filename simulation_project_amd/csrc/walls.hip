@@ -214,11 +214,12 @@ __device__ inline int march_run(int T) {
     const int nb = T <= kMarchBlock ? T : max(kMarchBlock, (T + kMarchBlock - 1) / kMarchBlock);
     return (T + nb - 1) / nb;
 }
-// FILL: the pairs of the triangles of workgroup blk, at off[t]; else their number per triangle
+// FILL: the pairs of the triangles of workgroup blk, at off[t]; else their number per triangle, and the
+// triangles' spheres
 template <typename R, bool FILL>
 __device__ inline void tri_march_body(int blk, int T, const Consts<R>& c, const TriD<R>* __restrict__ tris,
-                                      const R* __restrict__ tab, int* __restrict__ emit, const int* __restrict__ off,
-                                      const int* __restrict__ pair_n, int pair_cap, uint32_t* pair_cell,
+                                      const R* __restrict__ tab, float4* __restrict__ sph, int* __restrict__ emit,
+                                      const int* __restrict__ off, const int* __restrict__ pair_n, int pair_cap, uint32_t* pair_cell,
                                       int* pair_tri, int* overflow, MarchLds<R>& L) {
     if constexpr (FILL) {
         if (*pair_n > pair_cap) {
@@ -232,6 +233,7 @@ __device__ inline void tri_march_body(int blk, int T, const Consts<R>& c, const 
     const int t = t0 + (int)threadIdx.x;
     if (t < t1) {
         const TriD<R> tr = tris[t];
+        if constexpr (!FILL) sph[t] = tri_sphere(tr);
         const P3<R> A = p3(tr.v[0], tr.v[1], tr.v[2]), B = p3(tr.v[3], tr.v[4], tr.v[5]), C = p3(tr.v[6], tr.v[7], tr.v[8]);
         const R lim = (R)kLongEdge * c.cell;
         bool fin = true;
@@ -270,16 +272,17 @@ __device__ inline void tri_march_body(int blk, int T, const Consts<R>& c, const 
 }
 template <typename R, bool FILL>
 __global__ __launch_bounds__(kMarchBlock) void k_tri_march(int T, Consts<R> c, const TriD<R>* __restrict__ tris,
-                                                           const R* __restrict__ tab, int* emit,
+                                                           const R* __restrict__ tab, float4* sph, int* emit,
                                                            const int* __restrict__ off, const int* __restrict__ pair_n,
                                                            int pair_cap, uint32_t* pair_cell, int* pair_tri,
                                                            int* overflow) {
     __shared__ MarchLds<R> L;
-    tri_march_body<R, FILL>(blockIdx.x, T, c, tris, tab, emit, off, pair_n, pair_cap, pair_cell, pair_tri, overflow, L);
+    tri_march_body<R, FILL>(blockIdx.x, T, c, tris, tab, sph, emit, off, pair_n, pair_cap, pair_cell, pair_tri, overflow, L);
 }
 template <typename R, bool FILL> static void launch_tri_march(const Dev<R>& d, hipStream_t st) {
     hipLaunchKernelGGL((k_tri_march<R, FILL>), dim3(march_blocks(d.ntri)), dim3(kMarchBlock), 0, st, d.ntri, d.c, d.tris,
-                       d.march_tab, d.tri_emit, d.tri_off, d.pair_n, d.pair_cap, d.pair_cell, d.pair_tri, d.overflow);
+                       d.march_tab, d.tri_sph, d.tri_emit, d.tri_off, d.pair_n, d.pair_cap, d.pair_cell, d.pair_tri,
+                       d.overflow);
 }
 int tri_march_blocks(int T) { return march_blocks(T); }
 
@@ -339,7 +342,7 @@ template <typename R> void launch_tri_count_total(Dev<R>& d, hipStream_t st) {
     exclusive_scan(d.tri_emit, d.tri_off, nullptr, d.ntri, d.ntri, d.pair_n, d.tsort, st);
 }
 
-// The walk of every cell that holds particles, for nearest_triangle_listed, in two passes, into a
+// The walk of every cell that holds particles, for nearest_triangle_wave, in two passes, into a
 // pool shared by the cells (head[cell] = (offset, count); count -1: no walk, the full one is taken).
 // First, per cell: a cell without particles gets -1, one whose stencil lists are all empty gets 0;
 // the others reserve min(total, kStencilTris) pool entries (total: the stencil lists' lengths,
@@ -410,7 +413,7 @@ __global__ __launch_bounds__(256) void k_cell_walk_cells(int ncell, int gy, int 
 // kept when neither the ids kept so far (LDS, read 4 at a time) nor an earlier lane of the same 64
 // holds it: its first meeting.  More than kStencilTris kept ids give -1 (the full walk).  The kept
 // ids are then ordered by tri_box_bound over the cell's box (bitonic sort in LDS), each with its
-// position in the walk, and written at the cell's pool offset for nearest_triangle_listed.
+// position in the walk, and written at the cell's pool offset for nearest_triangle_wave.
 struct WalkLds {
     int off[28], beg[28];
     __align__(16) int kept[kStencilTris];
@@ -555,30 +558,41 @@ template <typename R> __device__ inline R4<R> mk4w(R x, R y, R z);
 template <> __device__ inline float4 mk4w<float>(float x, float y, float z) { return make_float4(x, y, z, 0.f); }
 template <> __device__ inline double4 mk4w<double>(double x, double y, double z) { return make_double4(x, y, z, 0.0); }
 
-template <typename R>
+// largest domain whose wall distances are searched by waves of 16 particles: a fine wall's particles are a
+// long chain for a wave of 64 (119 us against 41 at 62k, 96 against 45 at 126k), and a full chip gains
+// nothing from more waves (79 against 60 at 517k, 72 against 84 at 1M)
+static constexpr int kStlSplitMax = 700000;
+// P particles to a wave of the block (a power of two up to 64; the lanes beyond them only help to test)
+template <typename R, int P_>
 __device__ inline void stl_distance_body(int blk, int N, Consts<R> c, const R4<R>* __restrict__ spos,
                                          const int* __restrict__ tstart, const int* __restrict__ tcount,
                                          const int* __restrict__ tids, const TriD<R>* __restrict__ tris,
                                          R* stl_mag, R4<R>* stl_dir, int* stl_id, const int2* __restrict__ ulist,
-                                         const int2* __restrict__ uhead) {
-    const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= N) return;
-    const R4<R> P = spos[t];
+                                         const int2* __restrict__ uhead, const float4* __restrict__ sph,
+                                         NearestLds<R>* Lw) {
+    const int t = (int)(blk * (blockDim.x >> 6) + (threadIdx.x >> 6)) * P_ + lane_id();
+    const bool mine = lane_id() < P_ && t < N;
+    const R4<R> P = spos[mine ? t : 0];
     R best;
     P3<R> dir;
-    const int bid = nearest_triangle_listed(c, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, 0, &best,
-                                            &dir);
+    const int bid = nearest_triangle_wave(c, mine, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, sph, 0,
+                                          &best, &dir, Lw[threadIdx.x >> 6],
+                                          P_ == 64 ? 2 * kNearestShort : kNearestShort);
+    if (!mine) return;
     stl_mag[t] = best;
     stl_dir[t] = mk4w<R>(dir.x, dir.y, dir.z);
     stl_id[t] = bid;
 }
-template <typename R>
-__global__ __launch_bounds__(kMaxBlock) void k_stl_distance(int N, Consts<R> c, const R4<R>* __restrict__ spos,
+template <typename R, int P_>
+__global__ __launch_bounds__(256) void k_stl_distance(int N, Consts<R> c, const R4<R>* __restrict__ spos,
                                                        const int* __restrict__ tstart, const int* __restrict__ tcount,
                                                        const int* __restrict__ tids, const TriD<R>* __restrict__ tris,
                                                        R* stl_mag, R4<R>* stl_dir, int* stl_id,
-                                                       const int2* __restrict__ ulist, const int2* __restrict__ uhead) {
-    stl_distance_body<R>(blockIdx.x, N, c, spos, tstart, tcount, tids, tris, stl_mag, stl_dir, stl_id, ulist, uhead);
+                                                       const int2* __restrict__ ulist, const int2* __restrict__ uhead,
+                                                       const float4* __restrict__ sph) {
+    __shared__ NearestLds<R> L[4];
+    stl_distance_body<R, P_>(blockIdx.x, N, c, spos, tstart, tcount, tids, tris, stl_mag, stl_dir, stl_id, ulist, uhead, sph,
+                         L);
 }
 
 
@@ -589,16 +603,17 @@ __device__ inline void drag_body(int blk, int N, Consts<R> c, const int* __restr
                                  const int* __restrict__ tids, const TriD<R>* __restrict__ tris,
                                  const mpsr_tri_params* __restrict__ models,
                                  const mpsr_drag_params* __restrict__ drag, R4<R>* drag_acc,
-                                 R* drag_temp, const int2* __restrict__ ulist, const int2* __restrict__ uhead) {
+                                 R* drag_temp, const int2* __restrict__ ulist, const int2* __restrict__ uhead,
+                                 const float4* __restrict__ sph, NearestLds<R>* Lw) {
     const int t = blk * blockDim.x + threadIdx.x;
-    if (t >= N) return;
-    const int s = perm[t];
-    if (out.id[s] < 0) return;
-    const R4<R> P = spos[t];
+    const int s = t < N ? perm[t] : 0;
+    const bool live = t < N && out.id[s] >= 0;
+    const R4<R> P = spos[t < N ? t : 0];
     R best;
     P3<R> dir;
-    const int bid = nearest_triangle_listed(c, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, 1, &best,
-                                            &dir);
+    const int bid = nearest_triangle_wave(c, live, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, sph, 1,
+                                          &best, &dir, Lw[threadIdx.x >> 6]);
+    if (!live) return;
     drag_acc[t] = mk4w<R>(0, 0, 0);
     drag_temp[t] = 0;
     out.type[s] = 0;
@@ -651,9 +666,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_drag(int N, Consts<R> c, const in
                                                const mpsr_tri_params* __restrict__ models,
                                                const mpsr_drag_params* __restrict__ drag, R4<R>* drag_acc,
                                                R* drag_temp, const int2* __restrict__ ulist,
-                                               const int2* __restrict__ uhead) {
+                                               const int2* __restrict__ uhead, const float4* __restrict__ sph) {
+    __shared__ NearestLds<R> L[kMaxBlock / 64];
     drag_body<R>(blockIdx.x, N, c, perm, in, out, spos, svel, tstart, tcount, tids, tris, models, drag, drag_acc,
-                 drag_temp, ulist, uhead);
+                 drag_temp, ulist, uhead, sph, L);
 }
 
 template <typename R>
@@ -704,15 +720,17 @@ __global__ __launch_bounds__(256) void k_rotate(int T, TriD<R>* tris, const RotC
 
 template <typename R> void launch_stl_distance(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
-    hipLaunchKernelGGL(k_stl_distance<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.spos,
+    const bool few = d.N <= kStlSplitMax;
+    hipLaunchKernelGGL((few ? k_stl_distance<R, 16> : k_stl_distance<R, 64>), dim3(grid_for(d.N, few ? 64 : 256)),
+                       dim3(256), 0, st, d.N, d.c, d.spos,
                        d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.stl_mag, d.stl_dir, d.stl_id,
-                       d.cell_utri, d.cell_uhead);
+                       d.cell_utri, d.cell_uhead, d.tri_sph);
 }
 template <typename R> void launch_drag(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
     hipLaunchKernelGGL(k_drag<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.perm, d.in, d.out, d.spos,
                        d.svel, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.models, d.drag, d.drag_acc,
-                       d.drag_temp, d.cell_utri, d.cell_uhead);
+                       d.drag_temp, d.cell_utri, d.cell_uhead, d.tri_sph);
 }
 template <typename R> void launch_translate(const Dev<R>& d, hipStream_t st) {
     if (d.ntri <= 0) return;
@@ -738,8 +756,8 @@ __global__ __launch_bounds__(kMarchBlock) void k_tri_march_b(const Dev<R>* __res
     __shared__ MarchLds<R> L;
     const int2 w = items[blockIdx.x];
     const Dev<R>& d = dv[w.x];
-    tri_march_body<R, FILL>(w.y, d.ntri, d.c, d.tris, d.march_tab, d.tri_emit, d.tri_off, d.pair_n, d.pair_cap,
-                            d.pair_cell, d.pair_tri, d.overflow, L);
+    tri_march_body<R, FILL>(w.y, d.ntri, d.c, d.tris, d.march_tab, d.tri_sph, d.tri_emit, d.tri_off, d.pair_n,
+                            d.pair_cap, d.pair_cell, d.pair_tri, d.overflow, L);
 }
 // the sorted pairs are where the pair sort's passes left them (radix_sort_pairs' parity)
 template <typename R> struct OpPairs {
@@ -756,20 +774,22 @@ template <typename R> struct OpPairs {
         else pair_ranges_body(b, d.uniq_n, d.uniq_cell, d.cell_tri_start, d.cell_tri_count);
     }
 };
-template <typename R> struct OpStl {
+template <typename R, int P_> struct OpStl {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
-        stl_distance_body<R>(b, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.stl_mag,
-                             d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead);
+        __shared__ NearestLds<R> L[4];
+        stl_distance_body<R, P_>(b, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.stl_mag,
+                             d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, L);
     }
 };
 template <typename R> struct OpDrag {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
+        __shared__ NearestLds<R> L[kMaxBlock / 64];
         drag_body<R>(b, d.N, d.c, d.perm, d.in, d.out, d.spos, d.svel, d.cell_tri_start, d.cell_tri_count, d.uniq_tri,
-                     d.tris, d.models, d.drag, d.drag_acc, d.drag_temp, d.cell_utri, d.cell_uhead);
+                     d.tris, d.models, d.drag, d.drag_acc, d.drag_temp, d.cell_utri, d.cell_uhead, d.tri_sph, L);
     }
 };
 // the walks of the batched step: (bucket, block of 256 cells) items sort the cells as
@@ -836,8 +856,9 @@ void launch_cell_walks_b(const BatchLaunch<R>& b, WorkList c256, int2* work, int
     launch_batched<256>(OpCellWalkCells<R>{b.devs, work, nwork}, c256, 256, st);
     hipLaunchKernelGGL(k_cell_walks_b<R>, dim3(2048), dim3(64), 0, st, b.devs, work, nwork);
 }
-template <typename R> void launch_stl_distance_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
-    launch_batched<kMaxBlock>(OpStl<R>{b.devs}, p, b.block, st);
+template <typename R> void launch_stl_distance_b(const BatchLaunch<R>& b, WorkList near, hipStream_t st) {
+    static_assert(kNearBlock == 64, "four waves of 16 particles to an item");
+    launch_batched<256>(OpStl<R, 16>{b.devs}, near, 256, st);
 }
 template <typename R> void launch_drag_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
     launch_batched<kMaxBlock>(OpDrag<R>{b.devs}, p, b.block, st);
