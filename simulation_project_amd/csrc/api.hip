@@ -17,8 +17,10 @@
 // All launches go to one HIP stream; there is no host synchronisation inside a step (the
 // reference synchronises every step, MultiGPUHandler.cpp:1009-1018), so mpsr_step_many queues
 // `count` steps back to back and waits once.
+#include <atomic>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 #include <algorithm>
 #include "mpsr_internal.h"
@@ -251,6 +253,10 @@ template <typename R> struct Engine : EngineBase {
     ~Engine() override {
         if (ppe) ppe_destroy(ppe);
         if (bk_dead_h) (void)hipHostFree(bk_dead_h);
+        for (char* p : frame_pin)
+            if (p) (void)hipHostFree(p);
+        for (hipEvent_t e : frame_ev)
+            if (e) (void)hipEventDestroy(e);
         for (void* p : allocs) (void)hipFree(p);
         for (hipEvent_t e : pev) (void)hipEventDestroy(e);
         if (ev_a) (void)hipEventDestroy(ev_a);
@@ -512,13 +518,10 @@ template <typename R> struct Engine : EngineBase {
         ALLOC(d.spos, cap); ALLOC(d.svel, cap); ALLOC(d.spres, cap);
         d.rel.stride = cap + 32;
         d.rel.half = cap / 2 + 32;
-        ALLOC(d.rel.x, 4 * (size_t)d.rel.stride); ALLOC(d.rel.w, 2 * d.rel.half);
-        HIPC(hipMemset(d.rel.x, 0, sizeof(float) * 3 * (size_t)d.rel.stride));
-        HIPC(hipMemset(d.rel.w, 0, sizeof(float) * 2 * d.rel.half));
-        {
-            const std::vector<float> one(d.rel.stride, 1.0f);
-            HIPC(hipMemcpy(d.rel.x + 3 * (size_t)d.rel.stride, one.data(), sizeof(float) * one.size(), hipMemcpyHostToDevice));
-        }
+        ALLOC(d.rel.x, 4 * (size_t)d.rel.stride + 2 * d.rel.half);
+        d.rel.w = d.rel.x + 4 * (size_t)d.rel.stride;
+        fill_int(reinterpret_cast<int*>(d.rel.x), 0, 4 * (long long)d.rel.stride + 2 * d.rel.half, st);
+        fill_int(reinterpret_cast<int*>(d.rel.x + 3 * (size_t)d.rel.stride), 0x3f800000, d.rel.stride, st);   // 1.0f
         ALLOC(d.stl_mag, cap); ALLOC(d.stl_dir, cap); ALLOC(d.stl_id, cap);
         ALLOC(d.drag_acc, cap); ALLOC(d.drag_temp, cap);
         HIPC(hipMemset(d.drag_acc, 0, sizeof(R4<R>) * cap));
@@ -549,11 +552,9 @@ template <typename R> struct Engine : EngineBase {
         HIPC(hipMemcpy(d.tris, th.data(), sizeof(TriD<R>) * std::max(1, d.ntri), hipMemcpyHostToDevice));
         ALLOC(tris0, std::max(1, d.ntri));
         HIPC(hipMemcpy(tris0, th.data(), sizeof(TriD<R>) * std::max(1, d.ntri), hipMemcpyHostToDevice));
-        std::vector<R> tab(kMarchTab, R(0));
-        for (int k = 1; k < kMarchTab; ++k) tab[k] = tab[k - 1] + d.c.cell;
-        ALLOC(d.march_tab, kMarchTab);
-        HIPC(hipMemcpy(d.march_tab, tab.data(), sizeof(R) * kMarchTab, hipMemcpyHostToDevice));
-        ALLOC(d.tri_sph, std::max(1, d.ntri));
+        ALLOC(d.tri_sph, std::max(1, d.ntri) + kMarchTab * sizeof(R) / sizeof(float4));   // with the march table
+        d.march_tab = reinterpret_cast<R*>(d.tri_sph + std::max(1, d.ntri));
+        launch_march_tab(d, st);
         ALLOC(d.tri_emit, d.ntri + 1); ALLOC(d.tri_off, d.ntri + 1);
         ALLOC(d.pair_n, 1); ALLOC(d.uniq_n, 1); ALLOC(d.overflow, 1);
         HIPC(hipMemset(d.overflow, 0, sizeof(int)));
@@ -1052,29 +1053,96 @@ template <typename R> struct Engine : EngineBase {
         return MPSR_NOERR;
     }
 
+    // Frames leave in chunks of kFrameChunk particles through two pinned slots: a kernel packs a chunk's
+    // fields (vectors interleaved), one copy brings it to the host, and a few threads widen it into the
+    // caller's arrays while the next chunk is under way.  Thirteen copies into fresh pageable memory and
+    // one thread took 12 ms of a 1M-particle frame (and most of that in the first touches of the pages,
+    // its own and the caller's).  The slots are allocated by the first frame and kept.
+    static constexpr int kFrameChunk = 1 << 16;
+    char* frame_dev[2] = {nullptr, nullptr};
+    char* frame_pin[2] = {nullptr, nullptr};
+    hipEvent_t frame_ev[2] = {nullptr, nullptr};
+
     mpsr_status get_particles(int which, mpsr_particles* o) override {
+        HIPC(hipSetDevice(device));
         HIPC(hipStreamSynchronize(st));
         const PState<R>& S = which ? d.out : d.in;
         const int n = std::min(o->n, d.N);
-        std::vector<int> ids, type;
-        std::vector<R> f[11];
-        D2H(ids, S.id, n); D2H(type, S.type, n);
-        const R* src[11] = {S.px, S.py, S.pz, S.vx, S.vy, S.vz, S.p, S.n, S.temp, S.nu, S.solid};
-        for (int a = 0; a < 11; ++a) D2H(f[a], src[a], n);
-        for (int s = 0; s < n; ++s) {
-            if (o->id) o->id[s] = ids[s];
-            if (o->type) o->type[s] = type[s];
-            for (int a = 0; a < 3; ++a) {
-                if (o->position) o->position[3 * s + a] = (double)f[a][s];
-                if (o->velocity) o->velocity[3 * s + a] = (double)f[3 + a][s];
-            }
-            if (o->pressure) o->pressure[s] = f[6][s];
-            if (o->density) o->density[s] = f[7][s];
-            if (o->temperature) o->temperature[s] = f[8][s];
-            if (o->kinetic_viscosity) o->kinetic_viscosity[s] = f[9][s];
-            if (o->solid_phase_rate) o->solid_phase_rate[s] = f[10][s];
+        if (n <= 0) return MPSR_NOERR;
+        constexpr size_t row = 11 * sizeof(R) + 2 * sizeof(int);
+        const int chunk = std::min(kFrameChunk, std::max(1, d.cap)), chunks = (n + chunk - 1) / chunk;
+        for (int k = 0; k < 2; ++k) {
+            if (!frame_dev[k]) ALLOC(frame_dev[k], row * chunk);
+            if (!frame_pin[k]) HIPC(hipHostMalloc((void**)&frame_pin[k], row * chunk));
+            if (!frame_ev[k]) HIPC(hipEventCreateWithFlags(&frame_ev[k], hipEventDisableTiming));
         }
-        return MPSR_NOERR;
+        auto queue = [&](int c) -> mpsr_status {
+            const int first = c * chunk, m = std::min(chunk, n - first), k = c & 1;
+            launch_pack_frame(S, first, m, reinterpret_cast<R*>(frame_dev[k]), st);
+            HIPC(hipGetLastError());
+            HIPC(hipMemcpyAsync(frame_pin[k], frame_dev[k], row * m, hipMemcpyDeviceToHost, st));
+            HIPC(hipEventRecord(frame_ev[k], st));
+            return MPSR_NOERR;
+        };
+        // part w of nw of chunk c
+        auto widen = [&](int c, int w, int nw) {
+            const int first = c * chunk, m = std::min(chunk, n - first);
+            const int i0 = (int)((long long)m * w / nw), i1 = (int)((long long)m * (w + 1) / nw);
+            const R* f = reinterpret_cast<const R*>(frame_pin[c & 1]);
+            const int* q = reinterpret_cast<const int*>(f + 11 * (size_t)m);
+            auto put = [&](double* dst, const R* src, int width) {
+                if (dst)
+                    for (size_t i = (size_t)i0 * width; i < (size_t)i1 * width; ++i) dst[(size_t)first * width + i] = (double)src[i];
+            };
+            put(o->position, f, 3);
+            put(o->velocity, f + 3 * (size_t)m, 3);
+            double* const scalars[5] = {o->pressure, o->density, o->temperature, o->kinetic_viscosity, o->solid_phase_rate};
+            for (int a = 0; a < 5; ++a) put(scalars[a], f + (6 + a) * (size_t)m, 1);
+            if (o->id) std::memcpy(o->id + first + i0, q + i0, sizeof(int) * (i1 - i0));
+            if (o->type) std::memcpy(o->type + first + i0, q + m + i0, sizeof(int) * (i1 - i0));
+        };
+        for (int c = 0; c < std::min(2, chunks); ++c) {
+            const mpsr_status s = queue(c);
+            if (s != MPSR_NOERR) return s;
+        }
+        // one thread per 8k particles, at most eight; the calling thread is one of them
+        std::atomic<int> ready{0}, done{0}, stop{0};
+        std::vector<std::thread> helpers;
+        const int want = std::min(8, n / 8192);
+        std::atomic<int> nw{0};                       // 0 until all helpers that could be had are there
+        auto help = [&](int w) {
+            while (nw.load(std::memory_order_acquire) == 0) std::this_thread::yield();
+            for (int c = 0; c < chunks; ++c) {
+                while (ready.load(std::memory_order_acquire) <= c) {
+                    if (stop.load(std::memory_order_acquire)) return;
+                    std::this_thread::yield();
+                }
+                widen(c, w, nw.load(std::memory_order_relaxed));
+                done.fetch_add(1, std::memory_order_acq_rel);
+            }
+        };
+        try {
+            helpers.reserve(std::max(0, want - 1));
+            for (int w = 1; w < want; ++w) helpers.emplace_back(help, w);
+        } catch (...) {                                // fewer helpers, or none
+        }
+        const int all = (int)helpers.size() + 1;
+        nw.store(all, std::memory_order_release);
+        mpsr_status s = MPSR_NOERR;
+        for (int c = 0; c < chunks && s == MPSR_NOERR; ++c) {
+            if (hipEventSynchronize(frame_ev[c & 1]) != hipSuccess) {
+                s = fail(MPSR_GPUERR, "reading the particles back");
+                break;
+            }
+            ready.store(c + 1, std::memory_order_release);
+            widen(c, 0, all);
+            while (done.load(std::memory_order_acquire) < (all - 1) * (c + 1)) std::this_thread::yield();
+            if (c + 2 < chunks) s = queue(c + 2);     // the slot is free again
+        }
+        stop.store(1, std::memory_order_release);
+        for (std::thread& t : helpers) t.join();
+        if (s != MPSR_NOERR) (void)hipStreamSynchronize(st);
+        return s;
     }
     mpsr_status set_particles(const mpsr_particles* p) override {
         if (!p || p->n < 0 || p->n > d.cap) return fail(MPSR_PARAMERR, "particle count exceeds the allocated slots");

@@ -479,6 +479,9 @@ template <typename R> void launch_bin_hash(const Dev<R>& d, hipStream_t st);
 template <typename R> void launch_bin_ranges(Dev<R>& d, hipStream_t st);
 template <typename R> void launch_explicit(const Dev<R>& d, hipStream_t st);
 template <typename R> void launch_relocate(const Dev<R>& d, hipStream_t st);
+// slots first .. first + m - 1 of s packed for the host: positions and velocities interleaved [3m] each,
+// pressure, density, temperature, viscosity and solid rate [m] each, then (ints) id and type [m] each
+template <typename R> void launch_pack_frame(const PState<R>& s, int first, int m, R* out, hipStream_t st);
 template <typename R> void launch_pnd(const Dev<R>& d, int eos, hipStream_t st);
 // PND on the PPE path, with each Poisson row's active flag, neighbour bound, diagonal and
 // Dirichlet flag from the same neighbour pass, and its first nb_width Laplacian-radius neighbours
@@ -500,6 +503,7 @@ template <typename R> void launch_turbulence(const Dev<R>& d, hipStream_t st);
 template <typename R> void launch_neighbor_count(const Dev<R>& d, R re, int* counts, hipStream_t st);
 template <typename R> void launch_neighbor_fill(const Dev<R>& d, R re, const int* offsets, int* nbr, hipStream_t st);
 // walls.hip
+template <typename R> void launch_march_tab(const Dev<R>& d, hipStream_t st);   // fills march_tab
 template <typename R> void launch_tri_bin(Dev<R>& d, hipStream_t st);
 // key bits of the (cell, triangle) pair sort of a grid of ncell cells
 __host__ __device__ inline int tri_pair_bits(long long ncell) {

@@ -318,6 +318,34 @@ __global__ __launch_bounds__(kMaxBlock) void k_relocate(int N, Consts<R> c, PSta
 }
 
 // ---------------------------------------------------------------------------------------------
+// a frame's chunk in the layout the host widens (launch_pack_frame)
+template <typename R>
+__global__ __launch_bounds__(256) void k_pack_frame(PState<R> S, int first, int m, R* __restrict__ out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m) return;
+    const int s = first + i;
+    out[3 * i] = S.px[s];
+    out[3 * i + 1] = S.py[s];
+    out[3 * i + 2] = S.pz[s];
+    R* v = out + 3 * (size_t)m;
+    v[3 * i] = S.vx[s];
+    v[3 * i + 1] = S.vy[s];
+    v[3 * i + 2] = S.vz[s];
+    R* f = v + 3 * (size_t)m;
+    f[i] = S.p[s];
+    f[m + i] = S.n[s];
+    f[2 * (size_t)m + i] = S.temp[s];
+    f[3 * (size_t)m + i] = S.nu[s];
+    f[4 * (size_t)m + i] = S.solid[s];
+    int* q = reinterpret_cast<int*>(f + 5 * (size_t)m);
+    q[i] = S.id[s];
+    q[m + i] = S.type[s];
+}
+template <typename R> void launch_pack_frame(const PState<R>& s, int first, int m, R* out, hipStream_t st) {
+    hipLaunchKernelGGL(k_pack_frame<R>, dim3(grid_for(m, 256)), dim3(256), 0, st, s, first, m, out);
+}
+
+// ---------------------------------------------------------------------------------------------
 // the last, partial group of a row's neighbour list, padded with its last index
 __device__ inline void list_tail(int* nbq, int lbase, int lane, int kept, int q1, int q2, int q3) {
     if (kept & 3) {
@@ -983,6 +1011,7 @@ template <typename R> void launch_turbulence_b(const BatchLaunch<R>& b, WorkList
     template void launch_bin_ranges<R>(Dev<R>&, hipStream_t);                                 \
     template void launch_explicit<R>(const Dev<R>&, hipStream_t);                             \
     template void launch_relocate<R>(const Dev<R>&, hipStream_t);                             \
+    template void launch_pack_frame<R>(const PState<R>&, int, int, R*, hipStream_t);          \
     template void launch_pnd<R>(const Dev<R>&, int, hipStream_t);                             \
     template void launch_pnd_ppe<R>(const Dev<R>&, int*, int*, double*, int*, int*, int*, int, hipStream_t); \
     template void launch_gradient<R>(const Dev<R>&, hipStream_t, NbList);                     \

@@ -333,6 +333,18 @@ __global__ __launch_bounds__(256) void k_pair_ranges(const int* uniq_n, const ui
     pair_ranges_body(blockIdx.x, uniq_n, ucell, cstart, ccount);
 }
 
+template <typename R> __global__ void k_march_tab(R cell, R* tab) {
+    if (threadIdx.x != 0) return;
+    R t = 0;
+    for (int k = 0; k < kMarchTab; ++k) {
+        tab[k] = t;
+        t += cell;
+    }
+}
+template <typename R> void launch_march_tab(const Dev<R>& d, hipStream_t st) {
+    hipLaunchKernelGGL(k_march_tab<R>, dim3(1), dim3(64), 0, st, d.c.cell, d.march_tab);
+}
+
 template <typename R> void launch_tri_count_total(Dev<R>& d, hipStream_t st) {
     if (d.ntri <= 0) {
         fill_int(d.pair_n, 0, 1, st);
@@ -875,6 +887,7 @@ template <typename R> void launch_step_advance_b(const BatchLaunch<R>& b, WorkLi
 
 #define MPSR_INSTANTIATE_W(R)                                               \
     template void launch_tri_bin<R>(Dev<R>&, hipStream_t);                  \
+    template void launch_march_tab<R>(const Dev<R>&, hipStream_t);          \
     template void launch_tri_count_total<R>(Dev<R>&, hipStream_t);          \
     template void launch_stl_distance<R>(const Dev<R>&, hipStream_t);       \
     template void launch_drag<R>(const Dev<R>&, hipStream_t);               \
