@@ -431,7 +431,7 @@ mpsr_status mpsr_get_binning(mpsr_handle *h, int *sorted_keys, int *perm, int *c
  *   cell_start, cell_end  device [cell_capacity >= cells of gb]: first / end sorted index, -1 empty
  *   stream      a hipStream_t (NULL: the null stream); the call only queues work on it
  * The sort's scratch is a fixed device area inside the library (MPSR_NOALLOC_MAX_PARTICLES
- * particles, about 9 MB per GPU, held until the process ends): n above it is MPSR_PARAMERR.  No
+ * particles, about 10 MB per GPU, held until the process ends): n above it is MPSR_PARAMERR.  No
  * hipMalloc, hipFree or other allocation happens in this call.  Every call on one GPU shares that
  * GPU's scratch: calls that overlap on one GPU race. */
 #define MPSR_NOALLOC_MAX_PARTICLES (1 << 20)

@@ -1301,7 +1301,7 @@ template <typename R> struct BatchGroup {
     long long sig = -1;                // launch shape and optional phases the tables were built for
     struct Pass {
         const SortJob* jobs = nullptr;
-        WorkList tiles, singles;
+        WorkList tiles, rows;
     };
     WorkList wnear;                    // blocks of kNearBlock particles
     WorkList wp, wmarch, wt256, wpairs, wone, wdrag, wtherm, wturb, wc256;
@@ -1463,13 +1463,13 @@ template <typename R> struct BatchGroup {
         // have that many passes
         struct PassImg {
             size_t jobs;
-            Ref tiles, singles;
+            Ref tiles, rows;
         };
         auto passes = [&](bool pairs_sort, std::vector<PassImg>& out) {
             const int tile = radix_tile(pairs_sort ? 8 : items);
             for (int pass = 0;; ++pass) {
                 std::vector<SortJob> jobs;
-                std::vector<int2> tiles, singles;
+                std::vector<int2> tiles, rows;
                 for (int k = 0; k < n; ++k) {
                     const Dev<R>& d = host[k];
                     const int bits = pairs_sort ? tri_pair_bits(d.c.ncell) : d.key_bits;
@@ -1493,10 +1493,10 @@ template <typename R> struct BatchGroup {
                     const int j = (int)jobs.size();
                     jobs.push_back(q);
                     for (int b = 0; b < (int)grid_for(cap, tile); ++b) tiles.push_back(make_int2(j, b));
-                    singles.push_back(make_int2(j, 0));
+                    for (int b = 0; b < kRowBlocks; ++b) rows.push_back(make_int2(j, b));
                 }
                 if (jobs.empty()) break;
-                out.push_back(PassImg{put(jobs.data(), jobs.size() * sizeof(SortJob)), items_of(tiles), items_of(singles)});
+                out.push_back(PassImg{put(jobs.data(), jobs.size() * sizeof(SortJob)), items_of(tiles), items_of(rows)});
             }
         };
         std::vector<PassImg> pp, tp;
@@ -1532,8 +1532,8 @@ template <typename R> struct BatchGroup {
         scan_emit_t = wl(rse_t); scan_emit_1 = wl(rse_1); scan_flag_t = wl(rsf_t); scan_flag_1 = wl(rsf_1);
         psort.clear();
         tsort.clear();
-        for (const PassImg& q : pp) psort.push_back(Pass{reinterpret_cast<const SortJob*>(tab + q.jobs), wl(q.tiles), wl(q.singles)});
-        for (const PassImg& q : tp) tsort.push_back(Pass{reinterpret_cast<const SortJob*>(tab + q.jobs), wl(q.tiles), wl(q.singles)});
+        for (const PassImg& q : pp) psort.push_back(Pass{reinterpret_cast<const SortJob*>(tab + q.jobs), wl(q.tiles), wl(q.rows)});
+        for (const PassImg& q : tp) tsort.push_back(Pass{reinterpret_cast<const SortJob*>(tab + q.jobs), wl(q.tiles), wl(q.rows)});
         // the PPE buckets' solver tables
         std::vector<PpeSolver<R>*> solvers;
         std::vector<int> pdev;
@@ -1558,7 +1558,7 @@ template <typename R> struct BatchGroup {
         const BatchLaunch<R> b = launch();
         fill_int_batched(fill_bin, fill_bin_w, st);
         launch_bin_hash_b(b, wp, st);
-        for (const Pass& q : psort) radix_pass_batched(items, q.jobs, q.tiles, q.singles, st);
+        for (const Pass& q : psort) radix_pass_batched(items, q.jobs, q.tiles, q.rows, st);
         launch_bin_ranges_b(b, wp, st);
     }
     void tri(hipStream_t st) {
@@ -1567,7 +1567,7 @@ template <typename R> struct BatchGroup {
         launch_tri_count_b(b, wmarch, st);
         exclusive_scan_batched(scan_emit, scan_emit_t, scan_emit_1, st);
         launch_tri_fill_b(b, wmarch, st);
-        for (const Pass& q : tsort) radix_pass_batched(8, q.jobs, q.tiles, q.singles, st);
+        for (const Pass& q : tsort) radix_pass_batched(8, q.jobs, q.tiles, q.rows, st);
         launch_pairs_b(b, 0, wpairs, st);
         exclusive_scan_batched(scan_flag, scan_flag_t, scan_flag_1, st);
         launch_pairs_b(b, 1, wpairs, st);

@@ -303,7 +303,8 @@ size_t scan_tmp_ints(int n_cap);
 // Stable LSD radix sort of (key, value) pairs on `bits` low key bits.  n is *d_n when d_n is
 // non-null (device-resident count, n_cap bounds it), else n_host.  The result ends in (k0, v0)
 // or in (s.k1, s.v1); the return value says which (0 or 1).
-// `items` (4, 8 or 16) sets the tile of 256 * items keys; every tile gives the same result.
+// `items` (4, 8 or 16) sets the tile of 256 * items keys (4 up to 200k keys); every tile gives the same
+// result.
 int radix_sort_pairs(uint32_t* k0, int* v0, const int* d_n, int n_host, int n_cap, int bits,
                      const SortScratch& s, hipStream_t st, int items = 8);
 bool radix_items_valid(int items);
@@ -353,7 +354,7 @@ struct FillJob {
 };
 int radix_tile(int items);                  // keys per sort tile
 // passes of radix_sort_pairs over `bits` key bits (an odd count leaves the result in the scratch)
-__host__ __device__ inline int radix_passes_dev(int bits) { return bits > 0 ? (bits + 7) / 8 : 0; }
+__host__ __device__ inline int radix_passes_dev(int bits) { return bits > 0 ? (bits + 8) / 9 : 0; }
 int radix_passes(int bits);
 int radix_pass_bits(int bits, int pass, int* shift);
 int scan_tile();                            // ints per tile of the exclusive scan
@@ -362,8 +363,10 @@ constexpr int kScanBlock = 1024;            // threads of the scan kernels
 void fill_int_batched(const FillJob* jobs, WorkList blocks, hipStream_t st);
 // exclusive scans: tiles = (job, tile of scan_tile() ints), singles = (job, 0)
 void exclusive_scan_batched(const ScanJob* jobs, WorkList tiles, WorkList singles, hipStream_t st);
-// one radix pass of several sorts: tiles = (job, tile of radix_tile(items) keys), singles = (job, 0)
-void radix_pass_batched(int items, const SortJob* jobs, WorkList tiles, WorkList singles, hipStream_t st);
+// one radix pass of several sorts: tiles = (job, tile of radix_tile(items) keys), rows = (job, 0 ..
+// kRowBlocks - 1)
+constexpr int kRowBlocks = 32;
+void radix_pass_batched(int items, const SortJob* jobs, WorkList tiles, WorkList rows, hipStream_t st);
 
 }  // namespace mpsr
 

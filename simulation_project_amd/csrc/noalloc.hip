@@ -20,7 +20,7 @@ namespace mpsr {
 
 static constexpr size_t NA_MAX = MPSR_NOALLOC_MAX_PARTICLES;
 // radix_hist_ints(NA_MAX) and scan_tmp_ints(NA_MAX), checked against sort.hip at set-up
-static constexpr size_t NA_HIST = (size_t)256 * ((NA_MAX + 1023) / 1024 + 1);
+static constexpr size_t NA_HIST = (size_t)512 * ((NA_MAX + 1023) / 1024 + 2);
 static constexpr size_t NA_SCAN = (NA_MAX + 4095) / 4096 + 2 + 64;
 static constexpr size_t NA_INTS = 2 * NA_MAX + NA_HIST + NA_SCAN;
 static constexpr int NA_DEVICES = 64;
@@ -47,8 +47,11 @@ static hipError_t scratch_address(int device, int** out) {
 // RegisterParticleTopology's key per slot (the same bin_key as k_bin_hash), value = slot
 __global__ __launch_bounds__(256) void k_na_keys(int N, Consts<float> c, const int* __restrict__ id,
                                                  const float* __restrict__ px, const float* __restrict__ py,
-                                                 const float* __restrict__ pz, uint32_t* keys, int* vals) {
+                                                 const float* __restrict__ pz, uint32_t* keys, int* vals, int* cs,
+                                                 int* ce) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    // the cells are empty until k_na_ranges finds their particles
+    for (int i = s; i < c.ncell; i += gridDim.x * blockDim.x) cs[i] = ce[i] = -1;
     if (s >= N) return;
     keys[s] = bin_key(c, id[s], px[s], py[s], pz[s]);
     vals[s] = s;
@@ -118,11 +121,12 @@ extern "C" mpsr_status mpsr_register_particle_topology_noalloc(const mpsr_gridbo
     ss.hist_cap = (int)NA_HIST;
     ss.scan_tmp = base + 2 * NA_MAX + NA_HIST;
     ss.scan_tmp_cap = (int)NA_SCAN;
-    fill_int(cell_start, -1, ncell, st);
-    fill_int(cell_end, -1, ncell, st);
-    if (n > 0) {
+    if (n == 0) {
+        fill_int(cell_start, -1, ncell, st);
+        fill_int(cell_end, -1, ncell, st);
+    } else {
         hipLaunchKernelGGL(k_na_keys, dim3(grid_for(n, 256)), dim3(256), 0, st, n, c, id, px, py, pz,
-                           (uint32_t*)sorted_keys, perm);
+                           (uint32_t*)sorted_keys, perm, cell_start, cell_end);
         const int which = radix_sort_pairs((uint32_t*)sorted_keys, perm, nullptr, n, n, bits, ss, st, 8);
         if (which)
             hipLaunchKernelGGL(k_na_copy, dim3(grid_for(n, 256)), dim3(256), 0, st, n, ss.k1, ss.v1,

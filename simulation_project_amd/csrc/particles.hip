@@ -71,7 +71,9 @@ __device__ inline void bin_hash_body(int blk, int N, Consts<R> c, PState<R> in, 
 }
 template <typename R>
 __global__ __launch_bounds__(kMaxBlock) void k_bin_hash(int N, Consts<R> c, PState<R> in, PState<R> out, uint32_t* keys,
-                                                   int* vals) {
+                                                   int* vals, int* cs, int* ce) {
+    // the cells are empty until k_bin_ranges finds their particles
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < c.ncell; i += gridDim.x * blockDim.x) cs[i] = ce[i] = -1;
     bin_hash_body<R>(blockIdx.x, N, c, in, out, keys, vals);
 }
 
@@ -727,15 +729,13 @@ __global__ __launch_bounds__(kNearBlock, 3) void k_thermal(int N, Consts<R> c, c
 template <typename R> void launch_bin_hash(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
     hipLaunchKernelGGL(k_bin_hash<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.in, d.out, d.keys,
-                       d.vals);
+                       d.vals, d.cell_start, d.cell_end);
 }
 template <typename R> void launch_bin_ranges(Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
     const int which = radix_sort_pairs(d.keys, d.vals, nullptr, d.N, d.N, d.key_bits, d.sort, st, d.sort_items);
     d.skeys = which ? d.sort.k1 : d.keys;
     d.perm = which ? d.sort.v1 : d.vals;
-    fill_int(d.cell_start, -1, d.c.ncell, st);
-    fill_int(d.cell_end, -1, d.c.ncell, st);
     hipLaunchKernelGGL(k_bin_ranges<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.skeys,
                        d.perm, d.cell_start, d.cell_end, d.in, d.spos, d.svel, d.rel);
 }
