@@ -823,15 +823,109 @@ __global__ __launch_bounds__(PB) void k_resid_first(int N, int nslices, const in
                                      part, nullptr, nullptr, nullptr, 0, 0, nullptr, 0);
 }
 
-// x += alpha p; r -= alpha q; z = r / diag; partial r.z and r.r
-template <typename V>
+enum { RED_START = 0, RED_ALPHA = 1, RED_BETA = 2, RED_RESID = 3 };
+
+// the scalars of a step of the PCG from its sums
+struct PcgStep {
+    double done;   // S_DONE after it
+    double coef;   // alpha or beta
+};
+__device__ inline PcgStep pcg_step(int mode, double s0, double s1, const double* scal) {
+    if (mode == RED_ALPHA) {
+        if (!(s0 > 0.0) || !isfinite(s0)) return {3.0, 0.0};
+        return {0.0, scal[S_RZ] / s0};
+    }
+    double done = 0.0;
+    if (!isfinite(s1)) done = 3.0;
+    else if (s1 <= scal[S_TARGET]) done = 1.0;
+    else if (scal[S_ITERS] + 1.0 >= scal[S_MAXIT]) done = 2.0;
+    return {done, s0 / scal[S_RZ]};
+}
+__device__ inline void pcg_write(int mode, double s0, double s1, PcgStep w, double* scal) {
+    scal[S_DONE] = w.done;
+    if (mode == RED_ALPHA) {
+        if (w.done != 0.0) return;
+        scal[S_PQ] = s0;
+        scal[S_ALPHA] = w.coef;
+    } else {
+        scal[S_ITERS] += 1.0;
+        scal[S_BETA] = w.coef;
+        scal[S_RZ] = s0;
+        scal[S_RR] = s1;
+    }
+}
+
+// The sums of k_pcg_reduce formed again by every workgroup that needs them, for solves of at most
+// kFoldMax partials (262,144 rows: one partial a thread of k_pcg_reduce, so the waves' sums and their
+// order are the same).  Two launches of 3.3-4.5 us an iteration go; at 62k particles their readers take
+// 4.5 us for 4.0 (k_cell_pre), 3.6 for 1.9 (k_pcg_direction), 4.5 for 4.1 (k_pcg_update), and 327 launches a
+// step are left of 390.  With more partials every workgroup would read 31 KB and more (1M rows) against
+// 4.7 us of the one workgroup.  The scalars alternate between two copies: alpha's readers take scal and
+// write scal + S_COUNT, beta's the other way round, so no workgroup reads what another of its launch
+// writes.
+static constexpr int kFoldMax = 1024;
+// the step's scalars for the whole workgroup, workgroup 0 writing them to `out`; false when the solve has
+// stopped (before this step or by it)
+__device__ inline bool pcg_fold(int blk, int mode, const double* __restrict__ part, int nb,
+                                const double* __restrict__ in, double* __restrict__ out, double* coef) {
+    const bool write = blk == 0 && threadIdx.x == 0;
+    if (write)
+        for (int i = 0; i < S_COUNT; ++i) out[i] = in[i];
+    if (in[S_DONE] != 0.0) return false;
+    __shared__ double w0[16], w1[16];
+    const int lane = lane_id(), w = (int)(threadIdx.x >> 6);
+    constexpr int W = PB / 64, U = 16 / W;   // waves, and waves of k_pcg_reduce that each stands for
+    double a[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int i = (u * W + w) * 64 + lane;
+        a[u] = b[u] = 0.0;
+        if (i < nb) {
+            if (mode == RED_ALPHA) {
+                a[u] += part[i];
+            } else {
+                a[u] += part[2 * i];
+                b[u] += part[2 * i + 1];
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if ((u * W + w) * 64 < nb) {   // the whole wave: sums of zeros are left out
+            a[u] = wave_sum(a[u]);
+            if (mode != RED_ALPHA) b[u] = wave_sum(b[u]);
+        }
+        if (lane == 0) {
+            w0[u * W + w] = a[u];
+            w1[u * W + w] = b[u];
+        }
+    }
+    __syncthreads();
+    const double s0 = wave_sum(lane < 16 ? w0[lane] : 0.0);   // as block_sum<16>, in every wave
+    const double s1 = wave_sum(lane < 16 ? w1[lane] : 0.0);
+    const PcgStep st = pcg_step(mode, s0, s1, in);
+    if (write) pcg_write(mode, s0, s1, st, out);
+    *coef = st.coef;
+    return st.done == 0.0;
+}
+
+// x += alpha p; r -= alpha q; z = r / diag; partial r.z and r.r (to part; FOLD: alpha from the nb sums in
+// pq, another array: other workgroups may still read those)
+template <typename V, bool FOLD>
 __device__ inline void pcg_update_body(int blk, int N, V* x, V* r, V* z, const V* __restrict__ p,
                                        const V* __restrict__ q, const double* __restrict__ diag,
-                                       const double* __restrict__ scal, double* part) {
-    if (scal[S_DONE] != 0.0) return;
+                                       const double* __restrict__ scal, double* part, const double* __restrict__ pq,
+                                       int nb, double* scal_out) {
+    double al;
+    if constexpr (FOLD) {
+        if (!pcg_fold(blk, RED_ALPHA, pq, nb, scal, scal_out, &al)) return;
+    } else {
+        if (scal[S_DONE] != 0.0) return;
+        al = scal[S_ALPHA];
+    }
     __shared__ double lds[PB / 64];
     const int t = blk * blockDim.x + threadIdx.x;
-    const V alpha = (V)scal[S_ALPHA];
+    const V alpha = (V)al;
     double rz = 0.0, rr = 0.0;
     if (t < N) {
         x[t] = x[t] + alpha * p[t];
@@ -849,28 +943,35 @@ __device__ inline void pcg_update_body(int blk, int N, V* x, V* r, V* z, const V
         part[2 * blk + 1] = rr;
     }
 }
-template <typename V>
+template <typename V, bool FOLD>
 __global__ __launch_bounds__(PB) void k_pcg_update(int N, V* x, V* r, V* z, const V* __restrict__ p,
                                                     const V* __restrict__ q, const double* __restrict__ diag,
-                                                    const double* __restrict__ scal, double* part) {
-    pcg_update_body<V>(blockIdx.x, N, x, r, z, p, q, diag, scal, part);
+                                                    const double* __restrict__ scal, double* part,
+                                                    const double* __restrict__ pq, int nb, double* scal_out) {
+    pcg_update_body<V, FOLD>(blockIdx.x, N, x, r, z, p, q, diag, scal, part, pq, nb, scal_out);
 }
 
-// p = z + beta p (after the beta reduction; skipped once the solve has converged)
-template <typename V>
+// p = z + beta p (after the beta reduction or, FOLD, with it; skipped once the solve has converged)
+template <typename V, bool FOLD>
 __device__ inline void pcg_direction_body(int blk, int N, const V* __restrict__ z, V* p,
-                                          const double* __restrict__ scal) {
-    if (scal[S_DONE] != 0.0) return;
+                                          const double* __restrict__ scal, const double* __restrict__ part, int nb,
+                                          double* scal_out) {
+    double beta;
+    if constexpr (FOLD) {
+        if (!pcg_fold(blk, RED_BETA, part, nb, scal, scal_out, &beta)) return;
+    } else {
+        if (scal[S_DONE] != 0.0) return;
+        beta = scal[S_BETA];
+    }
     const int t = blk * blockDim.x + threadIdx.x;
-    if (t < N) p[t] = z[t] + (V)scal[S_BETA] * p[t];
+    if (t < N) p[t] = z[t] + (V)beta * p[t];
 }
-template <typename V>
+template <typename V, bool FOLD>
 __global__ __launch_bounds__(PB) void k_pcg_direction(int N, const V* __restrict__ z, V* p,
-                                                       const double* __restrict__ scal) {
-    pcg_direction_body<V>(blockIdx.x, N, z, p, scal);
+                                                       const double* __restrict__ scal, const double* __restrict__ part,
+                                                       int nb, double* scal_out) {
+    pcg_direction_body<V, FOLD>(blockIdx.x, N, z, p, scal, part, nb, scal_out);
 }
-
-enum { RED_START = 0, RED_ALPHA = 1, RED_BETA = 2, RED_RESID = 3 };
 
 // one workgroup: sums the block partials (1 or 2 interleaved sums) and advances the scalars
 __device__ inline void pcg_reduce_body(int blk, const double* __restrict__ part, int nb, int nsum, double* scal,
@@ -897,21 +998,8 @@ __device__ inline void pcg_reduce_body(int blk, const double* __restrict__ part,
         scal[S_BETA] = 0.0;
         scal[S_ITERS] = 0.0;
         scal[S_DONE] = (s1 <= scal[S_TARGET]) ? 1.0 : 0.0;
-    } else if (mode == RED_ALPHA) {
-        if (!(s0 > 0.0) || !isfinite(s0)) {
-            scal[S_DONE] = 3.0;
-            return;
-        }
-        scal[S_PQ] = s0;
-        scal[S_ALPHA] = scal[S_RZ] / s0;
-    } else if (mode == RED_BETA) {
-        scal[S_ITERS] += 1.0;
-        scal[S_BETA] = s0 / scal[S_RZ];
-        scal[S_RZ] = s0;
-        scal[S_RR] = s1;
-        if (!isfinite(s1)) scal[S_DONE] = 3.0;
-        else if (s1 <= scal[S_TARGET]) scal[S_DONE] = 1.0;
-        else if (scal[S_ITERS] >= scal[S_MAXIT]) scal[S_DONE] = 2.0;
+    } else if (mode == RED_ALPHA || mode == RED_BETA) {
+        pcg_write(mode, s0, s1, pcg_step(mode, s0, s1, scal), scal);
     } else {  // RED_RESID: residual norm and rhs norm of an FP64 residual pass
         scal[S_RR] = s0;
         scal[S_BB] = s1;
@@ -1558,16 +1646,23 @@ __global__ __launch_bounds__(PB) void k_cell_sym(int ncell, AggGeom g, float* op
 }
 // rc1 = P1^T r (r - alpha q with upd, as k_zcomp then writes it) and e = omega rc1 / diag Ac1:
 // eight lanes per cell striding over its contiguous rows, summed in a fixed lane order
-template <typename V>
+template <typename V, bool FOLD>
 __global__ __launch_bounds__(PB) void k_cell_pre(int ncell, const int* __restrict__ cs, const int* __restrict__ ce,
                                                   const int* __restrict__ dir, const V* __restrict__ r,
                                                   const V* __restrict__ q, int upd, const float* __restrict__ dinv,
                                                   double* rc, double* e, const double* __restrict__ scal,
-                                                  int check_done) {
-    if (check_done && scal[S_DONE] != 0.0) return;
+                                                  int check_done, const double* __restrict__ pq, int nb,
+                                                  double* scal_out) {
+    double al = 0.0;
+    if constexpr (FOLD) {   // with upd only
+        if (!pcg_fold(blockIdx.x, RED_ALPHA, pq, nb, scal, scal_out, &al)) return;
+    } else {
+        if (check_done && scal[S_DONE] != 0.0) return;
+        if (upd) al = scal[S_ALPHA];
+    }
     const int g8 = blockIdx.x * blockDim.x + threadIdx.x;
     const int I = g8 >> 3, sub = g8 & 7;
-    const V alpha = upd ? (V)scal[S_ALPHA] : (V)0;
+    const V alpha = (V)al;
     double acc = 0.0;
     const int a0 = I < ncell ? cs[I] : -1;
     if (a0 >= 0) {
@@ -1755,7 +1850,7 @@ PpeSolver<R>* ppe_create(const Dev<R>& d, const mpsr_params& P, const mpsr_ppe_o
           dev_alloc(&s->q, rows);
     ok &= dev_alloc(&s->rf, rows) && dev_alloc(&s->zf, rows) && dev_alloc(&s->p0f, rows) && dev_alloc(&s->p1f, rows) &&
           dev_alloc(&s->qf, rows) && dev_alloc(&s->ef, rows);
-    ok &= dev_alloc(&s->part, 2 * nb + 2) && dev_alloc(&s->scal, S_COUNT);
+    ok &= dev_alloc(&s->part, 3 * nb + 2) && dev_alloc(&s->scal, 2 * S_COUNT);
     s->scan.scan_tmp_cap = (int)scan_tmp_ints(s->nslices + 1);
     ok &= dev_alloc(&s->scan.scan_tmp, s->scan.scan_tmp_cap);
     ok &= hipHostMalloc((void**)&s->scal_h, sizeof(double) * S_COUNT) == hipSuccess;
@@ -1772,7 +1867,7 @@ PpeSolver<R>* ppe_create(const Dev<R>& d, const mpsr_params& P, const mpsr_ppe_o
         return nullptr;
     }
     (void)hipMemset(s->prev, 0, sizeof(double) * rows);
-    (void)hipMemset(s->scal, 0, sizeof(double) * S_COUNT);
+    (void)hipMemset(s->scal, 0, sizeof(double) * 2 * S_COUNT);
     s->mixed = opt.solver == MPSR_PCG_MIXED;
     // two-level preconditioner geometry and buffers
     s->agg_edge = opt.coarse_cells > 0 ? opt.coarse_cells : 2;
@@ -1930,17 +2025,17 @@ static void launch_spmv(PpeSolver<R>* s, const VA* vals, const V* p, V* q, hipSt
         if (s->c16 && s->wcap > 0) {
             hipLaunchKernelGGL((k_pcg_spmv<VA, V, true, true>), dim3(nb), dim3(PB), sizeof(V) * (size_t)s->wcap, st,
                                s->nslices, s->rowp, s->cnt, s->slice_off, s->slice_w, s->cols, vals, s->diag, p, q,
-                               s->scal, s->part, s->cols16, s->skeys, s->first_ge, s->gz, s->gygz, s->wbox, s->wcap);
+                               s->scal, s->part + 2 * (size_t)nb, s->cols16, s->skeys, s->first_ge, s->gz, s->gygz, s->wbox, s->wcap);
             return;
         }
     }
     if (s->c16)
         hipLaunchKernelGGL((k_pcg_spmv<VA, V, true, false>), dim3(nb), dim3(PB), 0, st, s->nslices, s->rowp, s->cnt,
-                           s->slice_off, s->slice_w, s->cols, vals, s->diag, p, q, s->scal, s->part, s->cols16,
+                           s->slice_off, s->slice_w, s->cols, vals, s->diag, p, q, s->scal, s->part + 2 * (size_t)nb, s->cols16,
                            s->skeys, s->first_ge, s->gz, s->gygz, (const int*)nullptr, 0);
     else
         hipLaunchKernelGGL((k_pcg_spmv<VA, V, false, false>), dim3(nb), dim3(PB), 0, st, s->nslices, s->rowp, s->cnt,
-                           s->slice_off, s->slice_w, s->cols, vals, s->diag, p, q, s->scal, s->part,
+                           s->slice_off, s->slice_w, s->cols, vals, s->diag, p, q, s->scal, s->part + 2 * (size_t)nb,
                            (const uint16_t*)nullptr, (const uint32_t*)nullptr, (const int*)nullptr, 0, 0,
                            (const int*)nullptr, 0);
 }
@@ -1953,6 +2048,18 @@ static int chunk_len(int it, int hint, int probe) {
     if (hint <= 0) return CHUNK;
     if (it == 0) return std::max(CHUNK_TAIL, hint - 1);
     return CHUNK_TAIL;
+}
+
+// beta's sums and p = z + beta p
+template <typename V, typename R>
+static void launch_direction(PpeSolver<R>* s, int N, const V* z, V* p, int nb, bool fold, hipStream_t st) {
+    if (fold) {
+        hipLaunchKernelGGL((k_pcg_direction<V, true>), dim3(nb), dim3(PB), 0, st, N, z, p, s->scal + S_COUNT, s->part, nb,
+                           s->scal);
+    } else {
+        hipLaunchKernelGGL(k_pcg_reduce, dim3(1), dim3(1024), 0, st, s->part, nb, 2, s->scal, (int)RED_BETA);
+        hipLaunchKernelGGL((k_pcg_direction<V, false>), dim3(nb), dim3(PB), 0, st, N, z, p, s->scal, nullptr, 0, nullptr);
+    }
 }
 
 template <typename R, typename VA, typename V>
@@ -1978,21 +2085,29 @@ static int run_pcg2(PpeSolver<R>* s, const Dev<R>& d, int N, const VA* vals, V* 
     // correction cc, or with the V-cycle the cell correction c_ef
     const bool vc = s->vcycle != 0;
     const int ncell = s->ncell;
+    const bool fold = vc && nb <= kFoldMax;   // without the V-cycle alpha's first reader has one wave a workgroup
+    double* const pq = s->part + 2 * (size_t)nb;   // q's partial sums, which are read while z's are written
     auto coarse = [&](int upd, int check) {
+        const double* const scal = fold && upd ? s->scal + S_COUNT : s->scal;
         if (vc) {
-            hipLaunchKernelGGL(k_cell_pre<V>, dim3(grid_for((long long)ncell * 8, PB)), dim3(PB), 0, st, ncell,
-                               d.cell_start, d.cell_end, s->dir, r, q, upd, s->c_dinv, s->c_rc, s->c_e, s->scal, check);
+            const dim3 grid(grid_for((long long)ncell * 8, PB));
+            if (fold && upd)
+                hipLaunchKernelGGL((k_cell_pre<V, true>), grid, dim3(PB), 0, st, ncell, d.cell_start, d.cell_end, s->dir,
+                                   r, q, upd, s->c_dinv, s->c_rc, s->c_e, s->scal, check, pq, nb, s->scal + S_COUNT);
+            else
+                hipLaunchKernelGGL((k_cell_pre<V, false>), grid, dim3(PB), 0, st, ncell, d.cell_start, d.cell_end, s->dir,
+                                   r, q, upd, s->c_dinv, s->c_rc, s->c_e, s->scal, check, nullptr, 0, nullptr);
             hipLaunchKernelGGL(k_cell_agg, dim3(nc), dim3(64), 0, st, nc, g, s->agg_full, s->c_op, s->c_rc, s->c_e,
-                               s->rc, s->scal, check);
+                               s->rc, scal, check);
         } else {
             hipLaunchKernelGGL(k_restrict<V>, dim3(nc), dim3(64), 0, st, nc, stacks, s->agg_rng, s->dir, r, q, upd,
                                s->rc, s->scal, check);
         }
-        if (f32) hipLaunchKernelGGL(k_coarse_mv<float>, dim3(nc), dim3(64), 0, st, nc, s->Af, s->rc, s->cc, s->scal, check);
-        else hipLaunchKernelGGL(k_coarse_mv<double>, dim3(nc), dim3(64), 0, st, nc, s->Ac, s->rc, s->cc, s->scal, check);
+        if (f32) hipLaunchKernelGGL(k_coarse_mv<float>, dim3(nc), dim3(64), 0, st, nc, s->Af, s->rc, s->cc, scal, check);
+        else hipLaunchKernelGGL(k_coarse_mv<double>, dim3(nc), dim3(64), 0, st, nc, s->Ac, s->rc, s->cc, scal, check);
         if (vc)
             hipLaunchKernelGGL(k_cell_post, dim3(grid_for((long long)ncell * 8, PB)), dim3(PB), 0, st, ncell, g, s->c_agg, s->c_op,
-                               s->c_dinv, s->c_rc, s->c_e, s->cc, s->c_ef, s->scal, check);
+                               s->c_dinv, s->c_rc, s->c_e, s->cc, s->c_ef, scal, check);
     };
     const int* zrow = vc ? s->cell_of_row : s->agg_of_row;
     const double* zcor = vc ? s->c_ef : s->cc;
@@ -2015,12 +2130,12 @@ static int run_pcg2(PpeSolver<R>* s, const Dev<R>& d, int N, const VA* vals, V* 
                 (void)hipEventRecord(s->ev[s->ev_used + 1], st);
                 s->ev_used += 2;
             }
-            hipLaunchKernelGGL(k_pcg_reduce, dim3(1), dim3(1024), 0, st, s->part, nb, 1, s->scal, (int)RED_ALPHA);
+            if (!fold)
+                hipLaunchKernelGGL(k_pcg_reduce, dim3(1), dim3(1024), 0, st, pq, nb, 1, s->scal, (int)RED_ALPHA);
             coarse(1, 1);
             hipLaunchKernelGGL(k_zcomp<V>, dim3(nb), dim3(PB), 0, st, N, r, s->pdiag, zrow, zcor, z, p, 0, x, q, 1,
-                               s->part, s->scal, 1);
-            hipLaunchKernelGGL(k_pcg_reduce, dim3(1), dim3(1024), 0, st, s->part, nb, 2, s->scal, (int)RED_BETA);
-            hipLaunchKernelGGL(k_pcg_direction<V>, dim3(nb), dim3(PB), 0, st, N, z, p, s->scal);
+                               s->part, fold ? s->scal + S_COUNT : s->scal, 1);
+            launch_direction<V>(s, N, z, p, nb, fold, st);
         }
         if (read_scal(s, st) != hipSuccess) {
             std::snprintf(s->why, sizeof(s->why), "device error while reading the PCG scalars");
@@ -2090,6 +2205,8 @@ static int run_pcg(PpeSolver<R>* s, int N, const VA* vals, V* x, V* r, V* z, V* 
     const int zero_x = std::is_same<V, float>::value ? 1 : 0;
     hipLaunchKernelGGL(k_pcg_start<V>, dim3(nb), dim3(PB), 0, st, N, r0, s->pdiag, r, z, pa, x, zero_x, s->part);
     hipLaunchKernelGGL(k_pcg_reduce, dim3(1), dim3(1024), 0, st, s->part, nb, 2, s->scal, (int)RED_START);
+    const bool fold = nb <= kFoldMax;
+    double* const pq = s->part + 2 * (size_t)nb;
     int done_iters = 0;
     const int probe = s->probe_at;
     s->probe_at = 0;
@@ -2109,11 +2226,15 @@ static int run_pcg(PpeSolver<R>* s, int N, const VA* vals, V* x, V* r, V* z, V* 
                 (void)hipEventRecord(s->ev[s->ev_used + 1], st);
                 s->ev_used += 2;
             }
-            hipLaunchKernelGGL(k_pcg_reduce, dim3(1), dim3(1024), 0, st, s->part, nb, 1, s->scal, (int)RED_ALPHA);
-            hipLaunchKernelGGL(k_pcg_update<V>, dim3(nb), dim3(PB), 0, st, N, x, r, z, pa, q, s->pdiag, s->scal,
-                               s->part);
-            hipLaunchKernelGGL(k_pcg_reduce, dim3(1), dim3(1024), 0, st, s->part, nb, 2, s->scal, (int)RED_BETA);
-            hipLaunchKernelGGL(k_pcg_direction<V>, dim3(nb), dim3(PB), 0, st, N, z, pa, s->scal);
+            if (fold) {
+                hipLaunchKernelGGL((k_pcg_update<V, true>), dim3(nb), dim3(PB), 0, st, N, x, r, z, pa, q, s->pdiag,
+                                   s->scal, s->part, pq, nb, s->scal + S_COUNT);
+            } else {
+                hipLaunchKernelGGL(k_pcg_reduce, dim3(1), dim3(1024), 0, st, pq, nb, 1, s->scal, (int)RED_ALPHA);
+                hipLaunchKernelGGL((k_pcg_update<V, false>), dim3(nb), dim3(PB), 0, st, N, x, r, z, pa, q, s->pdiag,
+                                   s->scal, s->part, nullptr, 0, nullptr);
+            }
+            launch_direction<V>(s, N, z, pa, nb, fold, st);
         }
         if (read_scal(s, st) != hipSuccess) {
             std::snprintf(s->why, sizeof(s->why), "device error while reading the PCG scalars");
@@ -2812,7 +2933,10 @@ template <typename R> struct OpPReduce {
             }
             return;
         }
-        pcg_reduce_body(b, v.part, v.nb, mode == RED_ALPHA ? 1 : 2, v.scal, mode);
+        if (mode == RED_ALPHA || mode == RED_BETA)
+            if (v.nb <= kFoldMax) return;   // their readers form the sums
+        pcg_reduce_body(b, mode == RED_ALPHA ? v.part + 2 * (size_t)v.nb : v.part, v.nb, mode == RED_ALPHA ? 1 : 2,
+                        v.scal, mode);
     }
 };
 // the decisions ppe_solve takes on the host after the first residual: the target, the iteration
@@ -2844,22 +2968,29 @@ template <typename R> struct OpPSpmv {
     __device__ void operator()(int j, int b) const {
         const PpeView<R>& v = pv[j];
         pcg_spmv_body<double, double, false, false>(b, v.nslices, v.rowp, v.cnt, v.slice_off, v.slice_w, v.cols,
-                                                    v.vals, v.diag, v.p, v.q, v.scal, v.part, nullptr, nullptr,
-                                                    nullptr, 0, 0, nullptr, 0);
+                                                    v.vals, v.diag, v.p, v.q, v.scal, v.part + 2 * (size_t)v.nb,
+                                                    nullptr, nullptr, nullptr, 0, 0, nullptr, 0);
     }
 };
 template <typename R> struct OpPUpdate {
     const PpeView<R>* pv;
     __device__ void operator()(int j, int b) const {
         const PpeView<R>& v = pv[j];
-        pcg_update_body<double>(b, v.N, v.x, v.r, v.z, v.p, v.q, v.diag, v.scal, v.part);
+        if (v.nb <= kFoldMax)
+            pcg_update_body<double, true>(b, v.N, v.x, v.r, v.z, v.p, v.q, v.diag, v.scal, v.part,
+                                          v.part + 2 * (size_t)v.nb, v.nb, v.scal + S_COUNT);
+        else
+            pcg_update_body<double, false>(b, v.N, v.x, v.r, v.z, v.p, v.q, v.diag, v.scal, v.part, nullptr, 0, nullptr);
     }
 };
 template <typename R> struct OpPDirection {
     const PpeView<R>* pv;
     __device__ void operator()(int j, int b) const {
         const PpeView<R>& v = pv[j];
-        pcg_direction_body<double>(b, v.N, v.z, v.p, v.scal);
+        if (v.nb <= kFoldMax)
+            pcg_direction_body<double, true>(b, v.N, v.z, v.p, v.scal + S_COUNT, v.part, v.nb, v.scal);
+        else
+            pcg_direction_body<double, false>(b, v.N, v.z, v.p, v.scal, nullptr, 0, nullptr);
     }
 };
 // ppe_solve's checks of the final residual: no breakdown, a finite relative residual, and the
@@ -3036,11 +3167,13 @@ template <typename R> void ppe_batch_pnd(PpeBatch<R>* b, const BatchLaunch<R>& b
     launch_pnd_ppe_b(bl, b->pnd, b->wpnd, st);
 }
 template <typename R> void ppe_batch_iterate(PpeBatch<R>* b, int iters, hipStream_t st) {
+    bool big = false;   // a bucket whose reductions are not folded
+    for (const PpeView<R>& v : b->hv) big |= v.nb > kFoldMax;
     for (int k = 0; k < iters; ++k) {
         launch_batched<PB>(OpPSpmv<R>{b->views}, b->wvec, PB, st);
-        launch_batched<1024>(OpPReduce<R>{b->views, RED_ALPHA}, b->wone, 1024, st);
+        if (big) launch_batched<1024>(OpPReduce<R>{b->views, RED_ALPHA}, b->wone, 1024, st);
         launch_batched<PB>(OpPUpdate<R>{b->views}, b->wvec, PB, st);
-        launch_batched<1024>(OpPReduce<R>{b->views, RED_BETA}, b->wone, 1024, st);
+        if (big) launch_batched<1024>(OpPReduce<R>{b->views, RED_BETA}, b->wone, 1024, st);
         launch_batched<PB>(OpPDirection<R>{b->views}, b->wvec, PB, st);
     }
 }
