@@ -362,7 +362,8 @@ mpsr_status mpsr_rotate_triangle_position(mpsr_handle *h, int analysis_step); /*
 /* ---- state in and out ---------------------------------------------------------------------- */
 
 /* which = 0: the "in" arrays (c_daParticle*), 1: the "out" arrays (c_daOutputParticle*).
- * = CCellSet::ParticleDeviceToHost (CGPUCellSet.cpp:833-892). */
+ * = CCellSet::ParticleDeviceToHost (CGPUCellSet.cpp:833-892).  Several threads may read one handle
+ * at once; where the staging memory of a frame cannot be had, the fields are copied one by one. */
 mpsr_status mpsr_get_particles(mpsr_handle *h, int which, mpsr_particles *out);
 /* = ParticleHostToDevice + ParticleNumberToConst (CGPUCellSet.cpp:893-952, DeviceProcess.cu:265-271). */
 mpsr_status mpsr_set_particles(mpsr_handle *h, const mpsr_particles *in);

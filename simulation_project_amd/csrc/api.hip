@@ -19,6 +19,7 @@
 // `count` steps back to back and waits once.
 #include <atomic>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -253,10 +254,7 @@ template <typename R> struct Engine : EngineBase {
     ~Engine() override {
         if (ppe) ppe_destroy(ppe);
         if (bk_dead_h) (void)hipHostFree(bk_dead_h);
-        for (char* p : frame_pin)
-            if (p) (void)hipHostFree(p);
-        for (hipEvent_t e : frame_ev)
-            if (e) (void)hipEventDestroy(e);
+        free_frame_slots();
         for (void* p : allocs) (void)hipFree(p);
         for (hipEvent_t e : pev) (void)hipEventDestroy(e);
         if (ev_a) (void)hipEventDestroy(ev_a);
@@ -1057,11 +1055,58 @@ template <typename R> struct Engine : EngineBase {
     // fields (vectors interleaved), one copy brings it to the host, and a few threads widen it into the
     // caller's arrays while the next chunk is under way.  Thirteen copies into fresh pageable memory and
     // one thread took 12 ms of a 1M-particle frame (and most of that in the first touches of the pages,
-    // its own and the caller's).  The slots are allocated by the first frame and kept.
+    // its own and the caller's).  The slots are allocated by the first frame and kept.  They serve one
+    // frame at a time: a second thread that reads the handle meanwhile, or a frame whose slots cannot be
+    // had, copies field by field into memory of its own.
     static constexpr int kFrameChunk = 1 << 16;
+    std::mutex frame_mutex;                 // holds the slots
     char* frame_dev[2] = {nullptr, nullptr};
     char* frame_pin[2] = {nullptr, nullptr};
     hipEvent_t frame_ev[2] = {nullptr, nullptr};
+
+    void free_frame_slots() {
+        for (int k = 0; k < 2; ++k) {
+            if (frame_dev[k]) (void)hipFree(frame_dev[k]);
+            if (frame_pin[k]) (void)hipHostFree(frame_pin[k]);
+            if (frame_ev[k]) (void)hipEventDestroy(frame_ev[k]);
+            frame_dev[k] = frame_pin[k] = nullptr;
+            frame_ev[k] = nullptr;
+        }
+    }
+    bool frame_slots(size_t bytes) {
+        bool ok = true;
+        for (int k = 0; k < 2 && ok; ++k)
+            ok = (frame_dev[k] || hipMalloc((void**)&frame_dev[k], bytes) == hipSuccess) &&
+                 (frame_pin[k] || hipHostMalloc((void**)&frame_pin[k], bytes) == hipSuccess) &&
+                 (frame_ev[k] || hipEventCreateWithFlags(&frame_ev[k], hipEventDisableTiming) == hipSuccess);
+        if (!ok) {
+            free_frame_slots();
+            (void)hipGetLastError();
+        }
+        return ok;
+    }
+    mpsr_status get_particles_plain(const PState<R>& S, int n, mpsr_particles* o) {
+        std::vector<int> q;
+        std::vector<R> f;
+        if (o->id) {
+            D2H(q, S.id, n);
+            std::copy(q.begin(), q.end(), o->id);
+        }
+        if (o->type) {
+            D2H(q, S.type, n);
+            std::copy(q.begin(), q.end(), o->type);
+        }
+        const R* const src[11] = {S.px, S.py, S.pz, S.vx, S.vy, S.vz, S.p, S.n, S.temp, S.nu, S.solid};
+        double* const dst[11] = {o->position, o->position, o->position, o->velocity, o->velocity, o->velocity,
+                                 o->pressure, o->density, o->temperature, o->kinetic_viscosity, o->solid_phase_rate};
+        for (int a = 0; a < 11; ++a) {
+            if (!dst[a]) continue;
+            D2H(f, src[a], n);
+            const int width = a < 6 ? 3 : 1, at = a < 6 ? a % 3 : 0;
+            for (int s = 0; s < n; ++s) dst[a][(size_t)s * width + at] = (double)f[s];
+        }
+        return MPSR_NOERR;
+    }
 
     mpsr_status get_particles(int which, mpsr_particles* o) override {
         HIPC(hipSetDevice(device));
@@ -1071,11 +1116,8 @@ template <typename R> struct Engine : EngineBase {
         if (n <= 0) return MPSR_NOERR;
         constexpr size_t row = 11 * sizeof(R) + 2 * sizeof(int);
         const int chunk = std::min(kFrameChunk, std::max(1, d.cap)), chunks = (n + chunk - 1) / chunk;
-        for (int k = 0; k < 2; ++k) {
-            if (!frame_dev[k]) ALLOC(frame_dev[k], row * chunk);
-            if (!frame_pin[k]) HIPC(hipHostMalloc((void**)&frame_pin[k], row * chunk));
-            if (!frame_ev[k]) HIPC(hipEventCreateWithFlags(&frame_ev[k], hipEventDisableTiming));
-        }
+        const std::unique_lock<std::mutex> slots(frame_mutex, std::try_to_lock);
+        if (!slots.owns_lock() || !frame_slots(row * chunk)) return get_particles_plain(S, n, o);
         auto queue = [&](int c) -> mpsr_status {
             const int first = c * chunk, m = std::min(chunk, n - first), k = c & 1;
             launch_pack_frame(S, first, m, reinterpret_cast<R*>(frame_dev[k]), st);

@@ -1,6 +1,9 @@
 """The particle read-back leaves in chunks of 65,536 through pinned slots, widened by up to eight threads:
 every field of a state that was set must come back as it was set, at sizes around a chunk, around the
-size that brings in the next thread, and for a count below the handle's."""
+size that brings in the next thread, and for a count below the handle's.  Threads that read one handle at
+once each get the whole frame, whichever of them holds the slots."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -32,3 +35,29 @@ def test_frame_comes_back_as_it_was_set(n, precision):
     got = s.get_particles(0)
     for f in FIELDS:
         np.testing.assert_array_equal(getattr(got, f), getattr(pa, f)[: s.n])
+
+
+@pytest.mark.parametrize("precision", [abi.MPSR_FP32, abi.MPSR_FP64])
+def test_threads_read_one_handle(precision):
+    n, readers, frames = 150001, 4, 6
+    s = Solver(cases.small_box(load_library(), nx=4, ny=4, nz=4), precision=precision, max_particles=n)
+    rng = np.random.default_rng(5)
+    pa = abi.ParticleArrays(n)
+    for f in FIELDS:
+        a = getattr(pa, f)
+        a[...] = rng.integers(-1, 1 << 20, a.shape) if a.dtype == np.int32 else rng.standard_normal(a.shape).astype(np.float32)
+    s.set_particles(pa)
+    start, wrong = threading.Barrier(readers), []
+
+    def read(k):
+        start.wait()
+        for _ in range(frames):
+            got = s.get_particles(k % 2)
+            wrong.extend((k, f) for f in FIELDS if not np.array_equal(getattr(got, f), getattr(pa, f)))
+
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(readers)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
