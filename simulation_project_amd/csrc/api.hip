@@ -469,6 +469,7 @@ template <typename R> struct Engine : EngineBase {
                 d.N += B.count - used;
             }
             launch_reset_walls(d, tris0, step, st);
+            d.walls_moved = 1;
             ++B.added;
         }
         return MPSR_NOERR;
@@ -646,6 +647,7 @@ template <typename R> struct Engine : EngineBase {
     void do_tri() {
         mark_begin(PH_TRI);
         launch_tri_bin(d, st);
+        d.walls_moved = 0;
         mark_end();
     }
     void do_stl() {
@@ -741,6 +743,7 @@ template <typename R> struct Engine : EngineBase {
         if (translate) launch_translate(d, st);
         d.rot = rot_table + (size_t)k * std::max(1, d.nmodel);
         launch_rotate(d, st);
+        d.walls_moved = 1;
         mark_end();
     }
 
@@ -894,6 +897,7 @@ template <typename R> struct Engine : EngineBase {
         if (s != MPSR_NOERR) return s;
         fill_int(step_ctr_buf, 0, 1, st);
         fill_int(step_base_buf, first, 1, st);
+        d.walls_moved = 1;                // by the batched steps
         HIPC(hipStreamSynchronize(st));   // rot_host is refilled by the next call
         return MPSR_NOERR;
     }
@@ -928,8 +932,12 @@ template <typename R> struct Engine : EngineBase {
             if (restore) HIPC(hipMemcpyAsync(f[i].first, snap[i], f[i].second, hipMemcpyDeviceToDevice, st));
             else HIPC(hipMemcpyAsync(snap[i], f[i].first, f[i].second, hipMemcpyDeviceToDevice, st));
         }
-        if (restore) d.N = snap_n;
-        else snap_n = d.N;
+        if (restore) {
+            d.N = snap_n;
+            d.walls_moved = 1;
+        } else {
+            snap_n = d.N;
+        }
         HIPC(hipStreamSynchronize(st));
         return MPSR_NOERR;
     }
@@ -1010,10 +1018,17 @@ template <typename R> struct Engine : EngineBase {
                     s = fail(s, std::string("PPE solve failed: ") + (ppe_why(ppe)[0] ? ppe_why(ppe) : "device error"));
                 break;
             case 8: do_gradient(); break;
-            case 9: launch_translate(d, st); break;
+            case 9:
+                launch_translate(d, st);
+                d.walls_moved = 1;
+                break;
             case 10:
                 s = upload_rot(arg, 1);
-                if (s == MPSR_NOERR) { d.rot = rot_table; launch_rotate(d, st); }
+                if (s == MPSR_NOERR) {
+                    d.rot = rot_table;
+                    launch_rotate(d, st);
+                    d.walls_moved = 1;
+                }
                 break;
             case 11: do_spheres(); break;
             case 12: launch_thermal(d, nullptr, nullptr, P.ThermalStep, st); break;

@@ -432,6 +432,7 @@ template <typename R> struct Dev {
     const int* step_ctr = nullptr;    // ... this device step counter picks the row (graph replays)
     R* march_tab = nullptr;           // [kMarchTab] distances of a wall march: 0, then + cell each
     float4* tri_sph = nullptr;        // [ntri] spheres around the triangles as last binned (tri_sphere)
+    int walls_moved = 0;              // 1: the triangles moved since; spheres and walk bounds do not hold
     int* tri_emit = nullptr;          // [ntri + 1] emitted cell count per triangle
     int* tri_off = nullptr;           // [ntri + 1]
     int* pair_n = nullptr;            // device count of emitted (cell, triangle) pairs

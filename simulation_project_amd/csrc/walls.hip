@@ -646,13 +646,13 @@ __device__ inline void stl_distance_body(int blk, int N, Consts<R> c, const R4<R
                                          const int* __restrict__ tids, const TriD<R>* __restrict__ tris,
                                          R* stl_mag, R4<R>* stl_dir, int* stl_id, const int2* __restrict__ ulist,
                                          const int2* __restrict__ uhead, const float4* __restrict__ sph,
-                                         NearestLds<R>* Lw) {
+                                         int moved, NearestLds<R>* Lw) {
     const int t = (int)(blk * (blockDim.x >> 6) + (threadIdx.x >> 6)) * P_ + lane_id();
     const bool mine = lane_id() < P_ && t < N;
     const R4<R> P = spos[mine ? t : 0];
     R best;
     P3<R> dir;
-    const int bid = nearest_triangle_wave(c, mine, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, sph, 0,
+    const int bid = nearest_triangle_wave(c, mine, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, sph, 0, moved,
                                           &best, &dir, Lw[threadIdx.x >> 6],
                                           P_ == 64 ? 2 * kNearestShort : kNearestShort);
     if (!mine) return;
@@ -666,10 +666,10 @@ __global__ __launch_bounds__(256) void k_stl_distance(int N, Consts<R> c, const 
                                                        const int* __restrict__ tids, const TriD<R>* __restrict__ tris,
                                                        R* stl_mag, R4<R>* stl_dir, int* stl_id,
                                                        const int2* __restrict__ ulist, const int2* __restrict__ uhead,
-                                                       const float4* __restrict__ sph) {
+                                                       const float4* __restrict__ sph, int moved) {
     __shared__ NearestLds<R> L[4];
     stl_distance_body<R, P_>(blockIdx.x, N, c, spos, tstart, tcount, tids, tris, stl_mag, stl_dir, stl_id, ulist, uhead, sph,
-                         L);
+                         moved, L);
 }
 
 
@@ -681,14 +681,14 @@ __device__ inline void drag_body(int blk, int N, Consts<R> c, const int* __restr
                                  const mpsr_tri_params* __restrict__ models,
                                  const mpsr_drag_params* __restrict__ drag, R4<R>* drag_acc,
                                  R* drag_temp, const int2* __restrict__ ulist, const int2* __restrict__ uhead,
-                                 const float4* __restrict__ sph, NearestLds<R>* Lw) {
+                                 const float4* __restrict__ sph, int moved, NearestLds<R>* Lw) {
     const int t = blk * blockDim.x + threadIdx.x;
     const int s = t < N ? perm[t] : 0;
     const bool live = t < N && out.id[s] >= 0;
     const R4<R> P = spos[t < N ? t : 0];
     R best;
     P3<R> dir;
-    const int bid = nearest_triangle_wave(c, live, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, sph, 1,
+    const int bid = nearest_triangle_wave(c, live, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, sph, 1, moved,
                                           &best, &dir, Lw[threadIdx.x >> 6]);
     if (!live) return;
     drag_acc[t] = mk4w<R>(0, 0, 0);
@@ -743,10 +743,11 @@ __global__ __launch_bounds__(kMaxBlock) void k_drag(int N, Consts<R> c, const in
                                                const mpsr_tri_params* __restrict__ models,
                                                const mpsr_drag_params* __restrict__ drag, R4<R>* drag_acc,
                                                R* drag_temp, const int2* __restrict__ ulist,
-                                               const int2* __restrict__ uhead, const float4* __restrict__ sph) {
+                                               const int2* __restrict__ uhead, const float4* __restrict__ sph,
+                                               int moved) {
     __shared__ NearestLds<R> L[kMaxBlock / 64];
     drag_body<R>(blockIdx.x, N, c, perm, in, out, spos, svel, tstart, tcount, tids, tris, models, drag, drag_acc,
-                 drag_temp, ulist, uhead, sph, L);
+                 drag_temp, ulist, uhead, sph, moved, L);
 }
 
 template <typename R>
@@ -801,13 +802,13 @@ template <typename R> void launch_stl_distance(const Dev<R>& d, hipStream_t st) 
     hipLaunchKernelGGL((few ? k_stl_distance<R, 16> : k_stl_distance<R, 64>), dim3(grid_for(d.N, few ? 64 : 256)),
                        dim3(256), 0, st, d.N, d.c, d.spos,
                        d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.stl_mag, d.stl_dir, d.stl_id,
-                       d.cell_utri, d.cell_uhead, d.tri_sph);
+                       d.cell_utri, d.cell_uhead, d.tri_sph, d.walls_moved);
 }
 template <typename R> void launch_drag(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
     hipLaunchKernelGGL(k_drag<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.perm, d.in, d.out, d.spos,
                        d.svel, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.models, d.drag, d.drag_acc,
-                       d.drag_temp, d.cell_utri, d.cell_uhead, d.tri_sph);
+                       d.drag_temp, d.cell_utri, d.cell_uhead, d.tri_sph, d.walls_moved);
 }
 template <typename R> void launch_translate(const Dev<R>& d, hipStream_t st) {
     if (d.ntri <= 0) return;
@@ -851,13 +852,14 @@ template <typename R> struct OpPairs {
         else pair_ranges_body(b, d.uniq_n, d.uniq_cell, d.cell_tri_start, d.cell_tri_count);
     }
 };
+// (a batched step searches the walls it has just binned)
 template <typename R, int P_> struct OpStl {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
         __shared__ NearestLds<R> L[4];
         stl_distance_body<R, P_>(b, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.stl_mag,
-                             d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, L);
+                             d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, 0, L);
     }
 };
 template <typename R> struct OpDrag {
@@ -866,7 +868,7 @@ template <typename R> struct OpDrag {
         const Dev<R>& d = dv[k];
         __shared__ NearestLds<R> L[kMaxBlock / 64];
         drag_body<R>(b, d.N, d.c, d.perm, d.in, d.out, d.spos, d.svel, d.cell_tri_start, d.cell_tri_count, d.uniq_tri,
-                     d.tris, d.models, d.drag, d.drag_acc, d.drag_temp, d.cell_utri, d.cell_uhead, d.tri_sph, L);
+                     d.tris, d.models, d.drag, d.drag_acc, d.drag_temp, d.cell_utri, d.cell_uhead, d.tri_sph, 0, L);
     }
 };
 // the walks of the batched step: (bucket, block of 256 cells) items sort the cells as

@@ -185,6 +185,9 @@ template <typename R> __device__ inline float4 tri_sphere(const TriD<R>& t) {
 // -1: no particles when the lists were written, or more than kStencilTris triangles) takes the
 // full walk.
 //
+// Both bounds are those of the walls as they were binned: where the triangles have moved since (`moved`),
+// every lane walks its whole list.
+//
 // One wave, a point per lane (`want` lanes only; every lane of the wave calls it).  A full distance is a
 // chain of about 250 instructions, and a particle near a fine wall has 70-130 listed triangles, of which a
 // few are near it.  So the points with a list are taken eight at a time, eight lanes to a point (lane
@@ -209,7 +212,7 @@ __device__ inline int nearest_triangle_wave(const Consts<R>& c, bool want, R x, 
                                             const int2* __restrict__ uhead, const int* __restrict__ tstart,
                                             const int* __restrict__ tcount, const int* __restrict__ tids,
                                             const TriD<R>* __restrict__ tris, const float4* __restrict__ sph,
-                                            int want_drag, R* best, P3<R>* bdir, NearestLds<R>& L,
+                                            int want_drag, int moved, R* best, P3<R>* bdir, NearestLds<R>& L,
                                             int short_list = kNearestShort) {
     const int lane = lane_id();
     *best = (R)1e8;
@@ -220,10 +223,10 @@ __device__ inline int nearest_triangle_wave(const Consts<R>& c, bool want, R x, 
     const int2 h = (cid >= 0 && cid < c.ncell) ? uhead[cid] : make_int2(0, -1);
     const R slack = c.cell * (R)0.005;
     const R lox = c.bminx + (R)ci * c.cell, loy = c.bminy + (R)cj * c.cell, loz = c.bminz + (R)ck * c.cell;
-    const int cut = x >= lox - slack && x <= lox + c.cell + slack && y >= loy - slack &&
+    const int cut = !moved && x >= lox - slack && x <= lox + c.cell + slack && y >= loy - slack &&
                     y <= loy + c.cell + slack && z >= loz - slack && z <= loz + c.cell + slack;
     const bool listed = want && h.y > 0;
-    if (!__any(listed && h.y > short_list)) {
+    if (moved || !__any(listed && h.y > short_list)) {
         // short lists (walls of a few large triangles): each lane walks its own
         int bid = -1, bpos = 0;
         const P3<R> p = p3(x, y, z);

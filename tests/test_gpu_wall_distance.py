@@ -55,3 +55,27 @@ def test_distance_and_drag_among_each_other(precision, token):
         a, b = g.get_particles(which), o.get_particles(which)
         for f in a.FIELDS:
             np.testing.assert_array_equal(getattr(a, f), getattr(b, f))
+
+
+@pytest.mark.parametrize("precision", [abi.MPSR_FP32, abi.MPSR_FP64])
+@pytest.mark.parametrize("motion", ["rotate", "translate"])
+@pytest.mark.parametrize("turns", [1, 4])
+def test_distance_after_the_walls_moved(precision, motion, turns):
+    """The walls move after they were binned: the lists are the binning's, the distances the moved walls'."""
+    lib = load_library()
+    case = cases.drum(lib, l0=8e-3, n_r=16, n_x=36, rpm=2000, dt=1e-3)      # 12 degrees a turn
+    case.models[0].Velocity = abi.Float3(9.0, -6.0, 14.0)                   # up to 14 mm a move
+    g, o = Solver(case, precision=precision), Oracle(case, precision=precision)
+    for s in (g, o):
+        s.RegisterParticleTopology()
+        s.RegisterTriangleTopology()
+        for k in range(turns):
+            s.RotateTrianglePosition(k) if motion == "rotate" else s.UpdateTrianglePosition()
+        s.CalcSTLDistance()
+    for a, b in zip(g.stl_distance(), o.stl_distance()):
+        np.testing.assert_array_equal(a, b)
+    for s in (g, o):                                                        # and binned again
+        s.RegisterTriangleTopology()
+        s.CalcSTLDistance()
+    for a, b in zip(g.stl_distance(), o.stl_distance()):
+        np.testing.assert_array_equal(a, b)
