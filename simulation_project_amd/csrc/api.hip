@@ -18,6 +18,8 @@
 // reference synchronises every step, MultiGPUHandler.cpp:1009-1018), so mpsr_step_many queues
 // `count` steps back to back and waits once.
 #include <atomic>
+#include <cfloat>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -103,6 +105,12 @@ template <typename R> static Consts<R> make_consts(const mpsr_params& P, const m
     c.gy = gb.m_GridSize.y;
     c.gz = gb.m_GridSize.z;
     c.ncell = c.gx * c.gy * c.gz;
+    const double lo[3] = {(double)c.bminx, (double)c.bminy, (double)c.bminz};
+    const int cells[3] = {c.gx, c.gy, c.gz};
+    double far = 0;
+    for (int a = 0; a < 3; ++a)
+        far = std::max(far, std::max(std::fabs(lo[a]), std::fabs(lo[a] + cells[a] * (double)c.cell)));
+    c.far_eps = (float)(far * FLT_EPSILON);
     c.tol = (R)P.Tolerance;
     c.l0 = (R)P.InitialParticleDistance;
     c.dt = (R)P.Dt;

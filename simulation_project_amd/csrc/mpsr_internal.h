@@ -61,6 +61,7 @@ template <typename R> struct Consts {
     R bminx, bminy, bminz;
     R cminx, cminy, cminz, cmaxx, cmaxy, cmaxz;
     R cell;
+    float far_eps;     // 2^-23 times the grid's largest coordinate: what a coordinate's rounding to float moves it
     int gx, gy, gz, ncell;
     R tol, l0, dt;
     // explicit predictor, Kern :283-441

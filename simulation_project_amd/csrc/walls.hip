@@ -556,7 +556,7 @@ __device__ inline void cell_walk_wave(long long cell, const Consts<R>& c, const 
     const R lox = c.bminx + (R)ci * c.cell, loy = c.bminy + (R)cj * c.cell, loz = c.bminz + (R)ck * c.cell;
     for (int q = lane; q < n2; q += 64) {
         unsigned key = 0xffffffffu;
-        if (q < n) key = (__float_as_uint(tri_box_bound(tris[L.kept[q]], lox, loy, loz, c.cell)) & ~kWalkPosMask) | (unsigned)q;
+        if (q < n) key = (__float_as_uint(tri_box_bound(tris[L.kept[q]], lox, loy, loz, c.cell, c.far_eps)) & ~kWalkPosMask) | (unsigned)q;
         L.key[q] = key;
     }
     __syncthreads();

@@ -119,7 +119,11 @@ __device__ inline int nearest_triangle(const Consts<R>& c, R x, R y, R z, const 
 // cos(theta) >= 0.2 the result is at least 0.975 times the bound, and at most 1.005 times |p - centroid|
 // + rad.  tri_tilt is 1 / cos(theta), infinite where no bound is drawn: a larger tilt or a degenerate
 // triangle (twice its area below 1 % of the longest edge squared), whose barycentric coordinates say
-// little.  The margins, 1 % of the cell size and of rad, are for the rounding of the rest.
+// little.  The margins, 1 % of the cell size and of rad, are for the rounding of the rest, and kFarRounding
+// coordinate roundings (Consts::far_eps) for that of the coordinates themselves, which outgrows them far
+// from the origin: the dot products of the normal with the point and the centroid err by up to 9, the
+// point's way to float, the box's corner and the points of the edges by 2 each.
+static constexpr float kFarRounding = 16.0f;
 template <typename R> __device__ inline double tri_tilt(const TriD<R>& t) {
     const double ax = t.v[0], ay = t.v[1], az = t.v[2], bx = t.v[3], by = t.v[4], bz = t.v[5], cx = t.v[6],
                  cy = t.v[7], cz = t.v[8];
@@ -147,7 +151,7 @@ template <typename R> __device__ inline double tri_centre(const TriD<R>& t, floa
 // drawn), as a float no larger than the bound: the distance between the box and the triangle's bounding
 // box, less the margins and what the tilt takes P off the triangle.
 template <typename R>
-__device__ inline float tri_box_bound(const TriD<R>& t, R lox, R loy, R loz, R size) {
+__device__ inline float tri_box_bound(const TriD<R>& t, R lox, R loy, R loz, R size, float far_eps) {
     const double sz = (double)size, tilt = tri_tilt(t);
     if (!(tilt < 1e3)) return 0.0f;
     float cc[3];
@@ -159,12 +163,13 @@ __device__ inline float tri_box_bound(const TriD<R>& t, R lox, R loy, R loz, R s
     };
     const double dx = gap(t.v[0], t.v[3], t.v[6], lx), dy = gap(t.v[1], t.v[4], t.v[7], ly),
                  dz = gap(t.v[2], t.v[5], t.v[8], lz);
-    const double lb = 0.975 * (sqrt(dx * dx + dy * dy + dz * dz) - rad * (0.01 + sqrt(tilt * tilt - 1.0))) - 0.01 * sz;
+    const double lb = 0.975 * (sqrt(dx * dx + dy * dy + dz * dz) - rad * (0.01 + sqrt(tilt * tilt - 1.0))) - 0.01 * sz -
+                      kFarRounding * far_eps;
     if (!(lb > 0.0)) return 0.0f;
     return (float)(lb * 0.999999);
 }
 // A sphere around every point tri_distance can end on: |p - centre| less its radius, times 0.975, less 1 %
-// of the cell size is a lower bound.  The radius is infinite where no bound is drawn, and negated for a
+// of the cell size and the coordinates' rounding, is a lower bound.  The radius is infinite where no bound is drawn, and negated for a
 // drag triangle.
 template <typename R> __device__ inline float4 tri_sphere(const TriD<R>& t) {
     float cc[3];
@@ -296,7 +301,7 @@ __device__ inline int nearest_triangle_wave(const Consts<R>& c, bool want, R x, 
         const float px = (float)__shfl(x, src, 64), py = (float)__shfl(y, src, 64), pz = (float)__shfl(z, src, 64);
         const int off = __shfl(h.x, src, 64), n0 = __shfl(h.y, src, 64), cutq = __shfl(cut, src, 64);
         const int n = g + q < count ? n0 : 0;
-        const float margin = 0.01f * (float)c.cell;
+        const float margin = 0.01f * (float)c.cell + kFarRounding * c.far_eps;
         const int2* const list = ulist + off;
         // f(on, e, sphere) for this lane's entries, four at a time (their loads are issued together: a
         // round waits for two loads, one after the other), until the list ends or, for a point inside its
