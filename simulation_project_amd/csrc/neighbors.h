@@ -124,8 +124,12 @@ __device__ inline void for_candidate_groups(const Consts<R>& c, const int* __res
 // the test.  The binning writes q' (an array per component, as a load costs a cycle for every lane that
 // is not next to its neighbour) and |q'|^2 / 2, the accumulator, which is the same for all particles.  Each lane shifts the signs of its 8 results of a run of 32 candidates into a byte
 // of the particle's bit word in LDS (one VALU instruction per 64 pairs, against nine).
-// T holds 1.008 reach^2 + 1e-4 cell^2: the build's root errs by at most 0.18 %, and the product, of
-// values up to 6 cells, by less than 1e-4 cell^2, so every neighbour within reach has its bit.
+// T holds (1.004 reach + e)^2 + 1e-4 cell^2: the build's root errs by at most 0.18 %, and the product, of
+// values up to 6 cells, by less than 1e-4 cell^2.  e = 6 far_eps is for the centres: a float centre is off by
+// up to 1.5 far_eps an axis (the product with the cell size and the sum are rounded), so the particle's and
+// the candidate's leave X - D - q' off by up to 3 an axis; far from the origin that outgrows the rest (l0 =
+// 10 mm, 10 km out: 2 mm, with which a tenth of the pressures went wrong).  So every neighbour within
+// reach has its bit.
 //
 // Phase 2 runs over each lane's own bits in walk order, f(q, record) with the record of the next one
 // loaded ahead; f tests the exact distance, so the sums are those of the plain walk.
@@ -164,7 +168,8 @@ __device__ inline void for_near_mfma(const Consts<R>& c, const int* __restrict__
     const int gz = c.gz, gyz = c.gy * c.gz;
     const uint32_t key = t < N ? skeys[t] : (uint32_t)c.ncell;
     const float cell = (float)c.cell;
-    const float T = (float)((double)reach * (double)reach * 1.008 + 1e-4 * (double)c.cell * (double)c.cell);
+    const double rt = 1.004 * (double)reach + 6.0 * (double)c.far_eps;
+    const float T = (float)(rt * rt + 1e-4 * (double)c.cell * (double)c.cell);
     bool mine = false, walk = false;
     if (want) {
         int ci, cj, ck;

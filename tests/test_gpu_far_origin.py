@@ -1,6 +1,6 @@
 """Domains far from the origin of their coordinates, against the oracle bit for bit: there a coordinate's
-rounding is no longer small against a cell, so the margins of the wall search (float positions, rounded
-distances) have to grow with the coordinate."""
+rounding is no longer small against a cell, so the walks' margins (cell centres in the neighbour test on the
+matrix cores, float positions and rounded distances in the wall search) have to grow with the coordinate."""
 import numpy as np
 import pytest
 
@@ -30,6 +30,21 @@ def test_wall_distance_far_from_the_origin(distance, precision):
             getattr(s, phase)()
     for a, b in zip(g.stl_distance(), o.stl_distance()):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", [abi.MPSR_FP32, abi.MPSR_FP64])
+@pytest.mark.parametrize("distance", [30.0, 1e3, 3e3, 1e4, 1e5, 1e6])
+def test_neighbour_sums_far_from_the_origin(distance, precision):
+    case = moved(cases.small_box(load_library(), nx=16, ny=14, nz=15, velocity_jitter=0.05), distance * DIRECTION, precision)
+    g, o = Solver(case, precision=precision), Oracle(case, precision=precision)
+    for s in (g, o):
+        for phase in ("RegisterParticleTopology", "RegisterTriangleTopology", "CalcSTLDistance", "CalcExplicitly",
+                      "CalcPressureExplicit"):
+            getattr(s, phase)()
+    for which in (0, 1):
+        a, b = g.get_particles(which), o.get_particles(which)
+        for f in a.FIELDS:
+            np.testing.assert_array_equal(getattr(a, f), getattr(b, f), err_msg=f"{which}.{f}")
 
 
 # a triangle, another a little farther from the point, the point; in units of a float's spacing
