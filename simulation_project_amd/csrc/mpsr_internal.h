@@ -163,6 +163,11 @@ template <typename R> struct RotCoef {
     int active;
 };
 
+// f(i) for every cell i, by all threads of the launch (unsigned: a grid may have close to 2^31 cells)
+template <typename F> __device__ inline void for_cells(int ncell, F&& f) {
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < (unsigned)ncell; i += gridDim.x * blockDim.x) f(i);
+}
+
 // ---- wave64 / block primitives --------------------------------------------------------------
 __device__ inline int lane_id() { return (int)(threadIdx.x & 63); }
 

@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void k_na_keys(int N, Consts<float> c, const i
                                                  int* ce) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     // the cells are empty until k_na_ranges finds their particles
-    for (int i = s; i < c.ncell; i += gridDim.x * blockDim.x) cs[i] = ce[i] = -1;
+    for_cells(c.ncell, [&](unsigned i) { cs[i] = ce[i] = -1; });
     if (s >= N) return;
     keys[s] = bin_key(c, id[s], px[s], py[s], pz[s]);
     vals[s] = s;

@@ -73,7 +73,7 @@ template <typename R>
 __global__ __launch_bounds__(kMaxBlock) void k_bin_hash(int N, Consts<R> c, PState<R> in, PState<R> out, uint32_t* keys,
                                                    int* vals, int* cs, int* ce) {
     // the cells are empty until k_bin_ranges finds their particles
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < c.ncell; i += gridDim.x * blockDim.x) cs[i] = ce[i] = -1;
+    for_cells(c.ncell, [&](unsigned i) { cs[i] = ce[i] = -1; });
     bin_hash_body<R>(blockIdx.x, N, c, in, out, keys, vals);
 }
 

@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kMarchBlock) void k_tri_march(int T, Consts<R> c, c
                                                            int* overflow, int* cell_count, int* work_n) {
     __shared__ MarchLds<R> L;
     if constexpr (!FILL) {   // what the passes after it count in
-        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < c.ncell; i += gridDim.x * blockDim.x) cell_count[i] = 0;
+        for_cells(c.ncell, [&](unsigned i) { cell_count[i] = 0; });
         if (blockIdx.x == 0 && threadIdx.x < 2) work_n[threadIdx.x] = 0;
     }
     tri_march_body<R, FILL>(blockIdx.x, T, c, tris, tab, sph, emit, off, pair_n, pair_cap, pair_cell, pair_tri, overflow, L);

@@ -119,3 +119,42 @@ def test_noalloc_rejects_more_particles_than_its_scratch(lib, hip):
     assert st == abi.MPSR_PARAMERR
     hip.free_all()
 
+
+def test_grid_of_almost_2_31_cells(lib):
+    """The largest grid the call takes (2^31 - 2 cells): an index that steps past it by the launch's threads
+    leaves the ints."""
+    gb = abi.GridBox()
+    sides = np.array([1386, 4681, 331])
+    gb.m_GridSize.x, gb.m_GridSize.y, gb.m_GridSize.z = (int(v) for v in sides)
+    gb.m_CellSize = 0.5
+    cells = gb.cells()
+    assert cells == 2 ** 31 - 2
+    n = 300
+    rng = np.random.default_rng(2)
+    c = np.stack([rng.integers(0, v, n) for v in sides], axis=1)
+    c[-1] = sides - 1                                           # the last cell
+    k = (c[:, 0] * sides[1] + c[:, 1]) * sides[2] + c[:, 2]
+    order = np.argsort(k, kind="stable")
+    cell, first, count = np.unique(k[order], return_index=True, return_counts=True)
+    hip = Hip()
+    try:
+        x, y, z = (hip.upload((0.5 * c[:, a] + 0.25).astype(np.float32)) for a in range(3))
+        keys, perm, start, end = hip.alloc(4 * n), hip.alloc(4 * n), hip.alloc(4 * cells), hip.alloc(4 * cells)
+        st = lib.mpsr_register_particle_topology_noalloc(C.byref(gb), n, hip.upload(np.arange(n, dtype=np.int32)), x, y,
+                                                          z, keys, perm, start, end, cells, 0, None)
+        assert st == abi.MPSR_NOERR
+        assert hip.rt.hipDeviceSynchronize() == 0
+        np.testing.assert_array_equal(hip.download(perm, n, np.int32), order)
+        np.testing.assert_array_equal(hip.download(keys, n, np.int32), k[order])
+        buf = np.empty(1 << 28, np.int32)
+        for got, want in ((start, first), (end, first + count)):
+            for at in range(0, cells, len(buf)):
+                m = min(len(buf), cells - at)
+                src = C.c_void_p(got.value + 4 * at)
+                assert hip.rt.hipMemcpy(buf.ctypes.data_as(C.c_void_p), src, 4 * m, 2) == 0
+                here = (cell >= at) & (cell < at + m)
+                np.testing.assert_array_equal(buf[cell[here] - at], want[here])
+                buf[cell[here] - at] = -1
+                assert int(buf[:m].min()) == -1 and int(buf[:m].max()) == -1
+    finally:
+        hip.free_all()
