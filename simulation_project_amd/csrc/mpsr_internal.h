@@ -225,6 +225,15 @@ template <int NW> __device__ inline int block_exclusive_scan(int v, int* lds, in
 // ---- launch helpers shared by the translation units ------------------------------------------
 inline unsigned grid_for(long long n, int block) { return (unsigned)((n + block - 1) / block); }
 
+// Workgroups of a launch over n items that also clears the grid's cells (for_cells): four cells a thread
+// at most up to a million threads, which fill the chip.  With the items' threads alone the two binnings of a
+// step of 1,000 particles in 29 M cells took 1,977 us, so 147 (234 by fills before each binning).
+inline unsigned grid_clearing(long long n, int ncell, int block) {
+    const unsigned items = grid_for(n, block), full = (1u << 20) / (unsigned)block;
+    const unsigned cells = grid_for(ncell, 4 * block);
+    return items > cells || items > full ? items : (cells < full ? cells : full);
+}
+
 // XCD-contiguous workgroup order for the neighbour kernels.  The GPU deals the workgroups of a
 // launch to its 8 XCDs in turn (workgroup b runs on XCD b % 8) and every XCD has its own L2, so in
 // launch order each L2 sees every eighth block of sorted particles and fetches nearly the whole

@@ -125,7 +125,7 @@ extern "C" mpsr_status mpsr_register_particle_topology_noalloc(const mpsr_gridbo
         fill_int(cell_start, -1, ncell, st);
         fill_int(cell_end, -1, ncell, st);
     } else {
-        hipLaunchKernelGGL(k_na_keys, dim3(grid_for(n, 256)), dim3(256), 0, st, n, c, id, px, py, pz,
+        hipLaunchKernelGGL(k_na_keys, dim3(grid_clearing(n, ncell, 256)), dim3(256), 0, st, n, c, id, px, py, pz,
                            (uint32_t*)sorted_keys, perm, cell_start, cell_end);
         const int which = radix_sort_pairs((uint32_t*)sorted_keys, perm, nullptr, n, n, bits, ss, st, 8);
         if (which)

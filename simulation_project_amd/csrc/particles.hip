@@ -728,7 +728,7 @@ __global__ __launch_bounds__(kNearBlock, 3) void k_thermal(int N, Consts<R> c, c
 
 template <typename R> void launch_bin_hash(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
-    hipLaunchKernelGGL(k_bin_hash<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.in, d.out, d.keys,
+    hipLaunchKernelGGL(k_bin_hash<R>, dim3(grid_clearing(d.N, d.c.ncell, d.block)), dim3(d.block), 0, st, d.N, d.c, d.in, d.out, d.keys,
                        d.vals, d.cell_start, d.cell_end);
 }
 template <typename R> void launch_bin_ranges(Dev<R>& d, hipStream_t st) {

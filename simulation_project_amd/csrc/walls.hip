@@ -281,10 +281,13 @@ __global__ __launch_bounds__(kMarchBlock) void k_tri_march(int T, Consts<R> c, c
         for_cells(c.ncell, [&](unsigned i) { cell_count[i] = 0; });
         if (blockIdx.x == 0 && threadIdx.x < 2) work_n[threadIdx.x] = 0;
     }
+    // (the workgroups beyond the triangles' have none)
     tri_march_body<R, FILL>(blockIdx.x, T, c, tris, tab, sph, emit, off, pair_n, pair_cap, pair_cell, pair_tri, overflow, L);
 }
 template <typename R, bool FILL> static void launch_tri_march(const Dev<R>& d, hipStream_t st) {
-    hipLaunchKernelGGL((k_tri_march<R, FILL>), dim3(march_blocks(d.ntri)), dim3(kMarchBlock), 0, st, d.ntri, d.c, d.tris,
+    const long long items = (long long)march_blocks(d.ntri) * kMarchBlock;
+    const unsigned grid = FILL ? march_blocks(d.ntri) : grid_clearing(items, d.c.ncell, kMarchBlock);
+    hipLaunchKernelGGL((k_tri_march<R, FILL>), dim3(grid), dim3(kMarchBlock), 0, st, d.ntri, d.c, d.tris,
                        d.march_tab, d.tri_sph, d.tri_emit, d.tri_off, d.pair_n, d.pair_cap, d.pair_cell, d.pair_tri,
                        d.overflow, d.cell_tri_count, d.cell_work_n);
 }

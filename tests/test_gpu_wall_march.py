@@ -52,3 +52,21 @@ def test_large_triangles_listed_as_the_serial_march(precision, cells, count):
         s.RegisterTriangleTopology()
     for x, y in zip(g.triangle_cells(), o.triangle_cells()):
         np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("side", [20, 66])
+def test_few_triangles_in_a_large_grid(side):
+    """The count pass clears the cells' counts: with workgroups of its own where the grid has more cells than
+    the triangles' threads take (66^3 cells, 12 triangles), and again when the walls have moved."""
+    case = cases.moving_plate_box(load_library(), plate_velocity=(-30.0, 0.0, 10.0), tank_velocity=(0.0, 0.0, 5.0))
+    lo, hi = case.zone.m_MinBound, case.zone.m_MaxBound
+    hi.x, hi.y, hi.z = (b + side * 3.1 * case.meta["l0"] for b in (lo.x, lo.y, lo.z))
+    g, o = Solver(case), Oracle(case)
+    for k in range(3):
+        for s in (g, o):
+            s.RegisterParticleTopology()
+            s.RegisterTriangleTopology()
+            for _ in range(4):
+                s.UpdateTrianglePosition()
+        for x, y in zip(g.triangle_cells(), o.triangle_cells()):
+            np.testing.assert_array_equal(x, y)
