@@ -67,7 +67,7 @@ template <typename R, typename F> __device__ inline void march_triangle(const Co
     } while (mBC >= cs && mAB >= cs && mCA >= cs && ++iter < kMaxShrink);
 }
 
-// A triangle whose longest edge exceeds kLongEdge cells is marched by its whole workgroup: a wall of
+// A large triangle is marched by its whole workgroup: a wall of
 // a few large triangles is one long serial chain per triangle otherwise, with as many lanes of the
 // GPU at work as there are triangles (the reference's 14-triangle deck: 595 us a pass with one lane
 // per triangle, 28.7 us so; a 12-triangle FP64 tank 409 and 28.0 us).  The shrinking alone is a chain, and only of the vertices: one wave walks it, lane l
@@ -79,7 +79,14 @@ template <typename R, typename F> __device__ inline void march_triangle(const Co
 // What remains is the chain of the copies.  Shorter edges (a finely meshed drum: 2-3 samples a line)
 // leave most of a wave idle in that form and stay with one lane per triangle (10k such triangles:
 // 7.2 us a pass).
+// Between them it is the workgroup's choice: with a longest edge of m cells a triangle takes the workgroup
+// 1 + 0.47 m us, one after the other, and a lane 7 + 0.25 m + 0.18 m^2 us, all lanes at once (300 triangles,
+// two to a workgroup, m = 6.4 to 34: 12-39 us a pass by workgroups, 20-224 us by lanes).  So the triangles
+// above 4 cells are counted in classes of m by doubling, and the class from which on the workgroup marches
+// is the one of the least sum of the two.  With every triangle above 4 cells marched by the workgroup,
+// 10k triangles of m = 7, 40 to a workgroup, took 467 us a binning, so 152 (197 with lanes only).
 static constexpr int kLongEdge = 4;
+static constexpr int kMarchClasses = 10;
 static constexpr int kMarchIters = 32;
 static constexpr int kMarchBlock = 256;
 template <typename R> struct MarchLds {
@@ -87,6 +94,7 @@ template <typename R> struct MarchLds {
     int first[3 * kMarchIters], last[3 * kMarchIters];   // first and last cell of each line, -1: none
     int copies, more, count, nlong;
     int longs[kMarchBlock];
+    int by_block[kMarchClasses], by_lane[kMarchClasses];   // the classes' costs, 0.1 us: summed, and the largest
 };
 // the next slots of the triangle for the lanes that emit; every lane of the wave calls it
 template <typename R, typename F> __device__ inline void emit_wave(bool em, int cid, MarchLds<R>& L, F&& put) {
@@ -229,16 +237,49 @@ __device__ inline void tri_march_body(int blk, int T, const Consts<R>& c, const 
     }
     const int run = march_run(T), t0 = blk * run, t1 = min(T, t0 + run);
     if (threadIdx.x == 0) L.nlong = 0;
+    if (threadIdx.x < kMarchClasses) L.by_block[threadIdx.x] = L.by_lane[threadIdx.x] = 0;
     __syncthreads();
     const int t = t0 + (int)threadIdx.x;
+    TriD<R> tr{};
+    int cls = -1;   // the triangle's class, -1: marched by its lane
     if (t < t1) {
-        const TriD<R> tr = tris[t];
+        tr = tris[t];
         if constexpr (!FILL) sph[t] = tri_sphere(tr);
         const P3<R> A = p3(tr.v[0], tr.v[1], tr.v[2]), B = p3(tr.v[3], tr.v[4], tr.v[5]), C = p3(tr.v[6], tr.v[7], tr.v[8]);
-        const R lim = (R)kLongEdge * c.cell;
         bool fin = true;
         for (int q = 0; q < 9; ++q) fin = fin && isfinite(tr.v[q]);
-        if (fin && !(pmag(psub(B, A)) <= lim && pmag(psub(C, B)) <= lim && pmag(psub(A, C)) <= lim)) {
+        const R ab = pmag(psub(B, A)), bc = pmag(psub(C, B)), ca = pmag(psub(A, C));
+        const R lim = (R)kLongEdge * c.cell;
+        if (fin && !(ab <= lim && bc <= lim && ca <= lim)) {
+            cls = 0;
+            if (run > 1) {
+                const float e = (float)fmax(ab, fmax(bc, ca)) / (float)c.cell;
+                const float m = e < 16384.0f ? e : 16384.0f;   // (also where an edge's length overflows)
+                cls = min(kMarchClasses - 1, max(0, (int)log2f(m / (float)kLongEdge)));
+                atomicAdd(&L.by_block[cls], 10 + (int)(4.7f * m));
+                atomicMax(&L.by_lane[cls], 70 + (int)(2.5f * m + 1.8f * m * m));
+            }
+        }
+    }
+    int from = 0;
+    if (run > 1) {   // one large triangle alone is the workgroup's
+        __syncthreads();
+        int block = 0, lane = 0;
+#pragma unroll
+        for (int q = 0; q < kMarchClasses; ++q) block += L.by_block[q];
+        int least = block;
+#pragma unroll
+        for (int q = 0; q < kMarchClasses; ++q) {
+            block -= L.by_block[q];
+            lane = max(lane, L.by_lane[q]);
+            if (lane + block < least) {
+                least = lane + block;
+                from = q + 1;
+            }
+        }
+    }
+    if (t < t1) {
+        if (cls >= from) {
             L.longs[atomicAdd(&L.nlong, 1)] = t;
         } else if constexpr (FILL) {
             int e = off[t];

@@ -1,6 +1,7 @@
 """The triangle binning of large triangles, which a whole workgroup marches, against the oracle's
 serial march: the cells' triangle lists are equal, entry for entry.  The sizes (longest edge in
-cells) sit on both sides of the rule (4 cells), of the copies one batch holds (32 copies: about
+cells) sit on both sides of the rule (4 cells, and from there the workgroup's choice by the sizes of all
+its triangles: 2 to 16 of them), of the copies one batch holds (32 copies: about
 58 cells) and of the table of distances (1,024 samples a line); the triangles are scattered over and
 beyond the grid, so lines start, end and run outside it, and short ones share workgroups with long
 ones (300 triangles: two to a workgroup)."""
@@ -17,6 +18,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("precision", [abi.MPSR_FP32, abi.MPSR_FP64])
 @pytest.mark.parametrize("cells,count", [((0.5, 3.9), 20), ((3.9, 4.1), 40), ((0.5, 30.0), 300), ((50.0, 70.0), 12),
+                                         ((4.2, 9.0), 3000), ((0.5, 40.0), 4000),
                                          ((1000.0, 1300.0), 3)])
 def test_large_triangles_listed_as_the_serial_march(precision, cells, count):
     lib = load_library()
