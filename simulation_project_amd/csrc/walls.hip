@@ -240,20 +240,20 @@ __device__ inline void tri_march_body(int blk, int T, const Consts<R>& c, const 
     if (threadIdx.x < kMarchClasses) L.by_block[threadIdx.x] = L.by_lane[threadIdx.x] = 0;
     __syncthreads();
     const int t = t0 + (int)threadIdx.x;
-    TriD<R> tr{};
     int cls = -1;   // the triangle's class, -1: marched by its lane
     if (t < t1) {
-        tr = tris[t];
+        const TriD<R> tr = tris[t];
         if constexpr (!FILL) sph[t] = tri_sphere(tr);
         const P3<R> A = p3(tr.v[0], tr.v[1], tr.v[2]), B = p3(tr.v[3], tr.v[4], tr.v[5]), C = p3(tr.v[6], tr.v[7], tr.v[8]);
         bool fin = true;
         for (int q = 0; q < 9; ++q) fin = fin && isfinite(tr.v[q]);
-        const R ab = pmag(psub(B, A)), bc = pmag(psub(C, B)), ca = pmag(psub(A, C));
+        const P3<R> ab = psub(B, A), bc = psub(C, B), ca = psub(A, C);
+        const R e2 = fmax(pdot(ab, ab), fmax(pdot(bc, bc), pdot(ca, ca)));
         const R lim = (R)kLongEdge * c.cell;
-        if (fin && !(ab <= lim && bc <= lim && ca <= lim)) {
+        if (fin && !(e2 <= lim * lim)) {
             cls = 0;
             if (run > 1) {
-                const float e = (float)fmax(ab, fmax(bc, ca)) / (float)c.cell;
+                const float e = sqrtf((float)e2) / (float)c.cell;
                 const float m = e < 16384.0f ? e : 16384.0f;   // (also where an edge's length overflows)
                 cls = min(kMarchClasses - 1, max(0, (int)log2f(m / (float)kLongEdge)));
                 atomicAdd(&L.by_block[cls], 10 + (int)(4.7f * m));
@@ -283,14 +283,14 @@ __device__ inline void tri_march_body(int blk, int T, const Consts<R>& c, const 
             L.longs[atomicAdd(&L.nlong, 1)] = t;
         } else if constexpr (FILL) {
             int e = off[t];
-            march_triangle(c, tr, [&](int cid) {
+            march_triangle(c, tris[t], [&](int cid) {
                 pair_cell[e] = (uint32_t)cid;
                 pair_tri[e] = t;
                 ++e;
             });
         } else {
             int n = 0;
-            march_triangle(c, tr, [&](int) { ++n; });
+            march_triangle(c, tris[t], [&](int) { ++n; });
             emit[t] = n;
         }
     }
