@@ -148,6 +148,72 @@ __device__ inline void for_candidate_groups(const Consts<R>& c, const int* __res
 // over 4 cells from its cell (aliased by the truncating cell index) or whose key is not its cell (a dead
 // slot) take the plain walk, as do those of a stencil plane of more than kNearWords words; the candidates
 // of a stencil cell that the cell index wraps to the other side of the grid all get their bit.
+// The cells of a wave are tested one after the other, so a wave of many cells (a spray, the rim of the
+// fluid) takes the plain walk too, its lanes side by side, where that is shorter: a cell of W words costs
+// 2 + W / 4 us, a plain walk of S candidates 20 + S / 5 us (waves alone on a SIMD).  Above kNearCells cells a
+// wave compares them, with the stencils of its first and last particle's cells, and above kNearCellsMost it
+// does not ask.  (Counted for every lane, S and W took 10 us; with S / 10 dense fluids lost 15-50 % at their
+// rims.)  PND pass of particles strewn at random, without the rule / with it: 264 / 34 us at 64k and one a
+// cell, 181 / 59 at four, 108 / 97 at eight, 91 / 93 at fifteen, 1,149 / 117 at 500k and one a cell; predictor
+// in FP64 1,213 / 213 there.  (Plain kernels, whose waves have no bit words to hold, take 45, 64, 82, 108,
+// 133 and 206.)
+static constexpr int kNearCells = 7, kNearCellsMost = 16;
+// g(q0, Q, m) for runs of up to 4 candidates as for_candidate_groups, over the stencil cells within `reach`
+// (as for_candidates_within, its margin with the cell boxes' rounding, up to 1.5 far_eps an axis, and the
+// offsets' own), the ranges of a row of cells loaded together
+static constexpr float kCullRounding = 5.0f;
+template <typename R, typename F>
+__device__ inline void for_candidates_sparse(const Consts<R>& c, const int* __restrict__ cs, const int* __restrict__ ce,
+                                             const R4<R>* __restrict__ spos, R x, R y, R z, R reach, F&& g) {
+    int ci, cj, ck;
+    if (!cell_coords(c, x, y, z, ci, cj, ck)) return;
+    const long long cid = cell_of(c, ci, cj, ck);
+    if (cid < 0 || cid >= c.ncell) return;
+    const R m = reach * (R)1.01 + (R)(kCullRounding * c.far_eps);
+    const R m2 = m * m;
+    const R lx = c.bminx + (R)ci * c.cell, ly = c.bminy + (R)cj * c.cell, lz = c.bminz + (R)ck * c.cell;
+    const R xm = x - lx, xp = lx + c.cell - x, ym = y - ly, yp = ly + c.cell - y, zm = z - lz, zp = lz + c.cell - z;
+    const R dx2[3] = {xm * xm, (R)0, xp * xp};
+    const bool inside = m < c.cell && cj >= 0 && cj < c.gy && ck >= 0 && ck < c.gz;   // and worth it
+    for (int k = -1; k <= 1; ++k) {
+        const R dz2 = k < 0 ? zm * zm : (k > 0 ? zp * zp : (R)0);
+        for (int j = -1; j <= 1; ++j) {
+            const R dyz2 = dz2 + (j < 0 ? ym * ym : (j > 0 ? yp * yp : (R)0));
+            // a cell that the index wraps to the other side of the grid is not where its offset says
+            const bool cull = inside && cj + j >= 0 && cj + j < c.gy && ck + k >= 0 && ck + k < c.gz;
+            if (cull && dyz2 > m2) continue;
+            int a[3], b[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const long long n = cell_of(c, ci + i - 1, cj + j, ck + k);
+                const bool in = n >= 0 && n < c.ncell && !(cull && dyz2 + dx2[i] > m2);
+                a[i] = in ? cs[n] : -1;
+                b[i] = in ? ce[n] : -1;
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                if (a[i] < 0) continue;
+                const int last = b[i] - 1;
+                for (int q = a[i]; q <= last; q += 4) {
+                    R4<R> Q[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) Q[u] = spos[min(q + u, last)];
+                    g(q, Q, min(4, last + 1 - q));
+                }
+            }
+        }
+    }
+}
+
+// f(q, Q) for each candidate of a run but `self`
+template <typename R, typename F> __device__ inline auto each_of(int self, F f) {
+    return [=](int q0, const R4<R> (&Q)[4], int m) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (u < m && q0 + u != self) f(q0 + u, Q[u]);
+    };
+}
+
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v2fu __attribute__((ext_vector_type(2), aligned(4)));
 typedef float v4fu __attribute__((ext_vector_type(4), aligned(4)));
@@ -160,10 +226,13 @@ struct NearLds {
     int meta[kNearWords];
 };
 
-template <typename R, typename Load, typename Use>
+// use(q, load(q)) for the neighbours by their bits; plain(q0, Q, m) for the candidates of a plain walk, in
+// runs (for_candidate_groups: self among them).  Both test the exact distance.
+template <typename R, typename Load, typename Use, typename Plain>
 __device__ inline void for_near_mfma(const Consts<R>& c, const int* __restrict__ cs, const int* __restrict__ ce,
                                      const RelPos& rel, const uint32_t* __restrict__ skeys, int t0,
-                                     int N, bool want, R x, R y, R z, R reach, NearLds& L, Load&& load, Use&& use) {
+                                     int N, bool want, const R4<R>* __restrict__ spos, R x, R y, R z, R reach, NearLds& L,
+                                     Load&& load, Use&& use, Plain&& plain) {
     const int lane = lane_id(), t = t0 + lane;
     const int gz = c.gz, gyz = c.gy * c.gz;
     const uint32_t key = t < N ? skeys[t] : (uint32_t)c.ncell;
@@ -208,6 +277,28 @@ __device__ inline void for_near_mfma(const Consts<R>& c, const int* __restrict__
     if (left) {
         K = __builtin_amdgcn_readlane((int)key, __ffsll(left) - 1);
         range(K, ca, cb);
+    }
+    const int cells = __popcll(__ballot(lane == 0 || (int)key != __shfl_up((int)key, 1, 64)));
+    if (left && cells > kNearCells) {
+        bool strewn = cells > kNearCellsMost;
+        if (!strewn) {
+            const int K1 = __builtin_amdgcn_readlane((int)key, 63 - __clzll(left));
+            int a1, b1;
+            range(K1, a1, b1);
+            // candidates in the low 17 bits, words above them
+            auto count = [&](int len) {
+                const int l = min(len, 4095);
+                return __builtin_amdgcn_readlane(wave_inclusive_scan(l | (((l + 31) >> 5) << 17)), 63);
+            };
+            const int n0 = count(length(K, ca, cb)), n1 = count(length(K1, a1, b1));
+            const int S = max(n0 & 0x1ffff, n1 & 0x1ffff), W = (n0 >> 17) + (n1 >> 17);   // W of both
+            strewn = cells * (80 + 5 * W) > 800 + 8 * S;
+        }
+        if (strewn) {
+            walk = walk || mine;
+            mine = false;
+            left = 0;
+        }
     }
     while (left) {
         int nw = 0, tab = 0, at = 0;
@@ -365,7 +456,7 @@ __device__ inline void for_near_mfma(const Consts<R>& c, const int* __restrict__
         }
         wave_lds_sync();
     }
-    if (walk) for_candidates(c, cs, ce, x, y, z, t, [&](int qq) { use(qq, load(qq)); });
+    if (walk) for_candidates_sparse(c, cs, ce, spos, x, y, z, reach, plain);
 }
 
 }  // namespace mpsr

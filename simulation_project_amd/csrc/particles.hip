@@ -245,33 +245,35 @@ __device__ inline void explicit_body(int blk, int N, Consts<R> c, const int* __r
     const R4<R> V0 = svel[t < N ? t : 0];
     const R re = c.re_lap;
     ExplicitSums<R> S;
+    // a plain walk's run of up to 4 candidates: the distances first, then the velocities of the hits, loaded
+    // together, then the sums in the canonical order
+    auto group = [&](int q0, const R4<R> (&Q)[4], int m) {
+        R dd[4];
+        bool hit[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            dd[u] = dist3(x, y, z, Q[u].x, Q[u].y, Q[u].z);
+            hit[u] = u < m && q0 + u != t && dd[u] < re;
+        }
+        R4<R> V[4];   // read only where hit[u]
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (hit[u]) V[u] = svel[q0 + u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (hit[u]) S.add(c, x, y, z, V0, Q[u], V[u], dd[u]);
+    };
     if constexpr (NEAR) {
         for_near_mfma(
-            c, cs, ce, rel, skeys, t0, N, live, x, y, z, re, Lw[threadIdx.x >> 6],
+            c, cs, ce, rel, skeys, t0, N, live, spos, x, y, z, re, Lw[threadIdx.x >> 6],
             [&](int q) { return PosVel<R>{spos[q], svel[q]}; },
             [&](int, const PosVel<R>& r) {
                 const R d = dist3(x, y, z, r.p.x, r.p.y, r.p.z);
                 if (d < re) S.add(c, x, y, z, V0, r.p, r.v, d);
-            });
+            },
+            group);
     } else if (live) {
-        // per group of 4 candidates: the distances first, then the velocities of the hits, loaded
-        // together, then the sums in the canonical order
-        for_candidate_groups(c, cs, ce, spos, x, y, z, [&](int q0, const R4<R> (&Q)[4], int m) {
-            R dd[4];
-            bool hit[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                dd[u] = dist3(x, y, z, Q[u].x, Q[u].y, Q[u].z);
-                hit[u] = u < m && q0 + u != t && dd[u] < re;
-            }
-            R4<R> V[4];   // read only where hit[u]
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (hit[u]) V[u] = svel[q0 + u];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (hit[u]) S.add(c, x, y, z, V0, Q[u], V[u], dd[u]);
-        });
+        for_candidate_groups(c, cs, ce, spos, x, y, z, group);
     }
     if (live) explicit_finish<R>(t, s, c, in, out, x, y, z, V0, S, stl_mag, stl_dir, stl_id, drag_acc, sph_dv, tris,
                                  models, turb_nu);
@@ -410,27 +412,27 @@ __device__ inline void pnd_body(int blk, int N, Consts<R> c, int eos, const int*
         ++nl;
     };
     const R rl = c.re_lap, mindl = c.mind_lap;
-    for_near_mfma(
-        c, cs, ce, rel, skeys, t0, N, sums, x, y, z, PPE && rl > re ? rl : re, Lw[threadIdx.x >> 6],
-        [&](int q) { return spos[q]; },
-        [&](int q, const R4<R>& Q) {
-            const R d0 = dist3(x, y, z, Q.x, Q.y, Q.z);
-            if (d0 < re) {
+    auto add = [&](int q, const R4<R>& Q) {
+        const R d0 = dist3(x, y, z, Q.x, Q.y, Q.z);
+        if (d0 < re) {
+            R d = d0;
+            if (d < mind) d = mind;
+            dens = dens + (re / d - 1);   // weight(re, d) for 0 < d < re
+            if constexpr (!PPE) list(q);
+        }
+        if constexpr (PPE) {
+            if (d0 < rl) {
                 R d = d0;
-                if (d < mind) d = mind;
-                dens = dens + (re / d - 1);   // weight(re, d) for 0 < d < re
-                if constexpr (!PPE) list(q);
+                if (d < mindl) d = mindl;
+                const R w = rl / d - 1;
+                wl += (double)w;
+                list(q);
             }
-            if constexpr (PPE) {
-                if (d0 < rl) {
-                    R d = d0;
-                    if (d < mindl) d = mindl;
-                    const R w = rl / d - 1;
-                    wl += (double)w;
-                    list(q);
-                }
-            }
-        });
+        }
+    };
+    for_near_mfma(
+        c, cs, ce, rel, skeys, t0, N, sums, spos, x, y, z, PPE && rl > re ? rl : re, Lw[threadIdx.x >> 6],
+        [&](int q) { return spos[q]; }, add, each_of<R>(t, add));
     if (t >= N) return;
     if (!sums) {
         in.p[s] = 0;
@@ -677,16 +679,17 @@ __device__ inline void thermal_body(int blk, int N, Consts<R> c, const int* __re
     const R t0_ = in.temp[s];
     const R re = c.re_temp, mind = c.mind_temp;
     R hf = 0, hw = 0;
+    auto add = [&](int q, const R4<R>& Q) {
+        R d = dist3(P.x, P.y, P.z, Q.x, Q.y, Q.z);
+        if (!(d < re)) return;
+        if (d < mind) d = mind;
+        const R num = (in.temp[perm[q]] - t0_) * weight(re, d);
+        const R den = d * d * (c.inv_kf + c.rf / d);
+        hf = hf + num / den;
+    };
     for_near_mfma(
-        c, cs, ce, rel, skeys, t0, N, live, P.x, P.y, P.z, re, Lw[threadIdx.x >> 6], [&](int q) { return spos[q]; },
-        [&](int q, const R4<R>& Q) {
-            R d = dist3(P.x, P.y, P.z, Q.x, Q.y, Q.z);
-            if (!(d < re)) return;
-            if (d < mind) d = mind;
-            const R num = (in.temp[perm[q]] - t0_) * weight(re, d);
-            const R den = d * d * (c.inv_kf + c.rf / d);
-            hf = hf + num / den;
-        });
+        c, cs, ce, rel, skeys, t0, N, live, spos, P.x, P.y, P.z, re, Lw[threadIdx.x >> 6], [&](int q) { return spos[q]; },
+        add, each_of<R>(t, add));
     if (!live) return;
     const R dist = stl_mag[t];
     const int tid = stl_id[t];
@@ -772,34 +775,39 @@ __device__ inline void turbulence_body(int blk, int N, Consts<R> c, const int* _
     const R4<R> V0 = svel[t < N ? t : 0];
     R txx = 0, txy = 0, txz = 0, tyx = 0, tyy = 0, tyz = 0, tzx = 0, tzy = 0, tzz = 0;
     const R re = c.re_grad, mind = c.mind_grad;
+    auto add = [&](R d, const R4<R>& Q, const R4<R>& V1) {
+        if (d < mind) d = mind;
+        const R w = re / d - 1;   // weight(re, d) for 0 < d < re
+        const R ux = V1.x - V0.x, uy = V1.y - V0.y, uz = V1.z - V0.z;
+        const R rx = Q.x - x, ry = Q.y - y, rz = Q.z - z;
+        const R dd = d * d;
+        if constexpr (sizeof(R) == 4) {
+            // nine quotients by one divisor: n / dd == (float)((double)n * RN(1 / (double)dd)) bit
+            // for bit.  The double product is within 2^-51 of n / dd, and a quotient of two
+            // 24-bit floats that is not a float midpoint (none is) lies more than 2^-48 of its
+            // size from every midpoint, so both round to the same float.
+            const double yd = 1.0 / (double)dd;
+            auto qt = [&](R n) { return (R)((double)n * yd); };
+            txx = txx + qt(ux * rx * w); txy = txy + qt(ux * ry * w); txz = txz + qt(ux * rz * w);
+            tyx = tyx + qt(uy * rx * w); tyy = tyy + qt(uy * ry * w); tyz = tyz + qt(uy * rz * w);
+            tzx = tzx + qt(uz * rx * w); tzy = tzy + qt(uz * ry * w); tzz = tzz + qt(uz * rz * w);
+        } else {
+            txx = txx + ux * rx * w / dd; txy = txy + ux * ry * w / dd; txz = txz + ux * rz * w / dd;
+            tyx = tyx + uy * rx * w / dd; tyy = tyy + uy * ry * w / dd; tyz = tyz + uy * rz * w / dd;
+            tzx = tzx + uz * rx * w / dd; tzy = tzy + uz * ry * w / dd; tzz = tzz + uz * rz * w / dd;
+        }
+    };
     for_near_mfma(
-        c, cs, ce, rel, skeys, t0, N, sums, x, y, z, re, Lw[threadIdx.x >> 6],
+        c, cs, ce, rel, skeys, t0, N, sums, spos, x, y, z, re, Lw[threadIdx.x >> 6],
         [&](int q) { return PosVel<R>{spos[q], svel[q]}; },
         [&](int, const PosVel<R>& r) {
-            const R4<R>&Q = r.p, &V1 = r.v;
-            R d = dist3(x, y, z, Q.x, Q.y, Q.z);
-            if (!(d < re)) return;
-            if (d < mind) d = mind;
-            const R w = re / d - 1;   // weight(re, d) for 0 < d < re
-            const R ux = V1.x - V0.x, uy = V1.y - V0.y, uz = V1.z - V0.z;
-            const R rx = Q.x - x, ry = Q.y - y, rz = Q.z - z;
-            const R dd = d * d;
-            if constexpr (sizeof(R) == 4) {
-                // nine quotients by one divisor: n / dd == (float)((double)n * RN(1 / (double)dd)) bit
-                // for bit.  The double product is within 2^-51 of n / dd, and a quotient of two
-                // 24-bit floats that is not a float midpoint (none is) lies more than 2^-48 of its
-                // size from every midpoint, so both round to the same float.
-                const double yd = 1.0 / (double)dd;
-                auto qt = [&](R n) { return (R)((double)n * yd); };
-                txx = txx + qt(ux * rx * w); txy = txy + qt(ux * ry * w); txz = txz + qt(ux * rz * w);
-                tyx = tyx + qt(uy * rx * w); tyy = tyy + qt(uy * ry * w); tyz = tyz + qt(uy * rz * w);
-                tzx = tzx + qt(uz * rx * w); tzy = tzy + qt(uz * ry * w); tzz = tzz + qt(uz * rz * w);
-            } else {
-                txx = txx + ux * rx * w / dd; txy = txy + ux * ry * w / dd; txz = txz + ux * rz * w / dd;
-                tyx = tyx + uy * rx * w / dd; tyy = tyy + uy * ry * w / dd; tyz = tyz + uy * rz * w / dd;
-                tzx = tzx + uz * rx * w / dd; tzy = tzy + uz * ry * w / dd; tzz = tzz + uz * rz * w / dd;
-            }
-        });
+            const R d = dist3(x, y, z, r.p.x, r.p.y, r.p.z);
+            if (d < re) add(d, r.p, r.v);
+        },
+        each_of<R>(t, [&](int q, const R4<R>& Q) {
+            const R d = dist3(x, y, z, Q.x, Q.y, Q.z);
+            if (d < re) add(d, Q, svel[q]);
+        }));
     if (!alive) return;
     if (!sums) {
         turb_nu[s] = 0;

@@ -1,7 +1,8 @@
 """The neighbour sums of the matrix-core walk (predictor, PND, heat conduction, turbulence) against the
 oracle, bit for bit, where that walk changes its course: one particle in a wave's last, partial block;
 cells denser than a bit word, than a row of words (three passes over the stencil) and than a plane of
-the stencil (plain walk); waves of many sparse cells (several groups of cells); a grid a few cells thin,
+the stencil (plain walk); waves of many sparse cells (plain walk from 17 cells on, or several groups of
+cells), of 8 to 16 cells, which choose, and of both in a spray around a block; a grid a few cells thin,
 whose cell index wraps from face to face; dead slots inside the grid; particles outside the zone but
 inside the grid, and beyond the grid's far faces, whose index aliases into other cells."""
 import ctypes as C
@@ -23,7 +24,8 @@ def make(layout, rng):
     lib = load_library()
     nx, ny, nz, n = {"one": (4, 4, 4, 1), "partial": (6, 5, 7, 200), "lattice": (16, 14, 15, None),
                      "dense": (10, 8, 9, 4000), "very_dense": (6, 5, 6, 9000), "cluster": (8, 6, 8, 3000),
-                     "sparse": (40, 34, 36, 900), "thin": (20, 1, 1, 500)}[layout]
+                     "sparse": (40, 34, 36, 900), "loose": (26, 24, 25, 4000), "spray": (40, 34, 36, 6000),
+                     "thin": (20, 1, 1, 500)}[layout]
     case = cases.small_box(lib, nx=nx, ny=ny, nz=nz, velocity_jitter=0.05)
     l0 = case.meta["l0"]
     if n is None:
@@ -34,6 +36,8 @@ def make(layout, rng):
         pos = rng.uniform(0.02, 0.98, (n, 3)) * size
         if layout == "cluster":         # most particles in one cell's volume: over 54 words a plane
             pos[: n - 300] = size / 2 + rng.uniform(-1.2, 1.2, (n - 300, 3)) * l0
+        if layout == "spray":           # half of them a block of about 30 a cell
+            pos[: n // 2] = size * [0.1, 0.2, 0.1] + rng.uniform(0, 15, (n // 2, 3)) * l0
     pa = abi.ParticleArrays(n)
     pa.id[:] = np.arange(n)
     pa.position[:] = pos.astype(np.float32)
@@ -55,7 +59,7 @@ def make(layout, rng):
 
 
 @pytest.mark.parametrize("precision", [abi.MPSR_FP32, abi.MPSR_FP64])
-@pytest.mark.parametrize("layout", ["one", "partial", "lattice", "dense", "very_dense", "cluster", "sparse", "thin"])
+@pytest.mark.parametrize("layout", ["one", "partial", "lattice", "dense", "very_dense", "cluster", "sparse", "loose", "spray", "thin"])
 @pytest.mark.parametrize("lap", [3.1, 2.1, 4.3])
 def test_near_walk_sums_identical(layout, precision, lap):
     case = make(layout, np.random.default_rng(len(layout)))
