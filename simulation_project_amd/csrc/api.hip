@@ -155,6 +155,27 @@ template <typename R> static Consts<R> make_consts(const mpsr_params& P, const m
     return c;
 }
 
+// Whether the walls are so fine that a cell's stencil lists many triangles: with a median triangle of area a,
+// a plane wall has 9 cell^2 / a of them in the stencil's cross-section (and lists about twice as many).  The
+// line is at 10, between the drums of 9.4 mm edges at l0 = 2 mm (8) and 2.5 mm (12) (k_stl_distance).  The
+// median leaves a few large walls beside a fine mesh out of account, and moving walls keep it.
+template <typename R> static bool is_fine(const std::vector<TriD<R>>& t, int n, double cell) {
+    std::vector<double> area((size_t)std::max(0, n));
+    for (int i = 0; i < n; ++i) {
+        double a[3], b[3];
+        for (int k = 0; k < 3; ++k) {
+            a[k] = (double)t[i].v[3 + k] - t[i].v[k];
+            b[k] = (double)t[i].v[6 + k] - t[i].v[k];
+        }
+        const double x = a[1] * b[2] - a[2] * b[1], y = a[2] * b[0] - a[0] * b[2], z = a[0] * b[1] - a[1] * b[0];
+        const double s = 0.5 * std::sqrt(x * x + y * y + z * z);
+        area[i] = std::isfinite(s) ? s : 0.0;
+    }
+    if (area.empty()) return false;
+    std::nth_element(area.begin(), area.begin() + n / 2, area.end());
+    return 9.0 * cell * cell > 10.0 * area[n / 2];
+}
+
 // RotateTrianglePosition_Kernel's per-model angle logic (Kern :945-971) and the axis of
 // CalcNormal(Center, Second) (Utility_Inline.h:58-67), evaluated once per model and step.
 template <typename R> static RotCoef<R> rot_coef(const mpsr_tri_params& m, const mpsr_params& P, int step) {
@@ -555,6 +576,7 @@ template <typename R> struct Engine : EngineBase {
             q.is_drag = ci->models[T.ModelIDNumber].isDrag ? 1 : 0;
             th[t] = q;
         }
+        d.fine_walls = is_fine(th, d.ntri, (double)d.c.cell) ? 1 : 0;
         ALLOC(d.tris, std::max(1, d.ntri));
         HIPC(hipMemcpy(d.tris, th.data(), sizeof(TriD<R>) * std::max(1, d.ntri), hipMemcpyHostToDevice));
         ALLOC(tris0, std::max(1, d.ntri));

@@ -137,13 +137,14 @@ template <typename R> struct PState {
     R *p, *n, *temp, *nu, *solid;
 };
 
-// most triangles of a per-cell triangle walk (nearest_triangle_wave); a walk entry's key keeps
+// most triangles of a per-cell triangle walk (nearest_in_wave); a walk entry's key keeps
 // the walk position in its low 10 bits
 static constexpr int kStencilTris = 1024;
 static constexpr unsigned kWalkPosMask = 1023u;
 // pairs of a wave's nearest-triangle queue beyond which it is tested
 static constexpr int kNearestQueue = 192;
-// longest triangle lists that the lanes of a wave of few points walk each for itself
+// longest triangle lists that the lanes of a wave of 16 points walk each for itself (a tank of 14 triangles:
+// 8 us a pass, 16 us taken together; the 517k drum's 10-30: 113 us, 60 taken together)
 static constexpr int kNearestShort = 16;
 
 // Triangle record on the device: three vertices, the stored normal, the model, the model's
@@ -446,6 +447,7 @@ template <typename R> struct Dev {
     RotCoef<R>* rot = nullptr;        // [nmodel] for the current step, or the table base when
     const int* step_ctr = nullptr;    // ... this device step counter picks the row (graph replays)
     R* march_tab = nullptr;           // [kMarchTab] distances of a wall march: 0, then + cell each
+    int fine_walls = 0;               // 1: walls of small triangles, with long lists (api.hip, is_fine)
     float4* tri_sph = nullptr;        // [ntri] spheres around the triangles as last binned (tri_sphere)
     int walls_moved = 0;              // 1: the triangles moved since; spheres and walk bounds do not hold
     int* tri_emit = nullptr;          // [ntri + 1] emitted cell count per triangle

@@ -456,7 +456,7 @@ template <typename R> void launch_tri_count_total(Dev<R>& d, hipStream_t st) {
     exclusive_scan(d.tri_emit, d.tri_off, nullptr, d.ntri, d.ntri, d.pair_n, d.tsort, st);
 }
 
-// The walk of every cell that holds particles, for nearest_triangle_wave, in two passes, into a
+// The walk of every cell that holds particles, for nearest_in_wave, in two passes, into a
 // pool shared by the cells (head[cell] = (offset, count); count -1: no walk, the full one is taken).
 // First, per cell: a cell without particles gets -1, one whose stencil lists are all empty gets 0;
 // the others reserve min(total, kStencilTris) pool entries (total: the stencil lists' lengths,
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(256) void k_cell_walk_cells(int ncell, int gy, int 
 // kept when neither the ids kept so far (LDS, read 4 at a time) nor an earlier lane of the same 64
 // holds it: its first meeting.  More than kStencilTris kept ids give -1 (the full walk).  The kept
 // ids are then ordered by tri_box_bound over the cell's box (bitonic sort in LDS), each with its
-// position in the walk, and written at the cell's pool offset for nearest_triangle_wave.
+// position in the walk, and written at the cell's pool offset for nearest_in_wave.
 struct WalkLds {
     int off[28], beg[28];
     __align__(16) int kept[kStencilTris];
@@ -679,41 +679,51 @@ template <typename R> __device__ inline R4<R> mk4w(R x, R y, R z);
 template <> __device__ inline float4 mk4w<float>(float x, float y, float z) { return make_float4(x, y, z, 0.f); }
 template <> __device__ inline double4 mk4w<double>(double x, double y, double z) { return make_double4(x, y, z, 0.0); }
 
-// largest domain whose wall distances are searched by waves of 16 particles: a fine wall's particles are a
-// long chain for a wave of 64 (119 us against 41 at 62k, 96 against 45 at 126k), and a full chip gains
-// nothing from more waves (79 against 60 at 517k, 72 against 84 at 1M)
-static constexpr int kStlSplitMax = 700000;
-// P particles to a wave of the block (a power of two up to 64; the lanes beyond them only help to test)
+// P_ points to a wave (the lanes beyond them only help to test): 16 where the walls are fine and the lists
+// long (Dev::fine_walls), else 64, each with its own list: of four waves three would only find short lists
+// or none, and a lone lane's chain is short.  Two passes of rotating drums by 64 / by 16 (the median length
+// of the lists): 72 / 110 us at 517k particles (8), 141 / 189 at 1M (16), 72 / 69 at 126k (16), 150 / 121 at
+// 517k (23), 233 / 162 at 872k (31), 198 / 72 at 126k (48), 273 / 82 at 62k (69), 505 / 230 at 872k (71);
+// a tank of 12 triangles and 500k particles 27 / 37.
 template <typename R, int P_>
 __device__ inline void stl_distance_body(int blk, int N, Consts<R> c, const R4<R>* __restrict__ spos,
                                          const int* __restrict__ tstart, const int* __restrict__ tcount,
                                          const int* __restrict__ tids, const TriD<R>* __restrict__ tris,
                                          R* stl_mag, R4<R>* stl_dir, int* stl_id, const int2* __restrict__ ulist,
                                          const int2* __restrict__ uhead, const float4* __restrict__ sph,
-                                         int moved, NearestLds<R>* Lw) {
-    const int t = (int)(blk * (blockDim.x >> 6) + (threadIdx.x >> 6)) * P_ + lane_id();
+                                         int moved, NearestLds<R>* L) {
+    const int t = blk * P_ + lane_id();
     const bool mine = lane_id() < P_ && t < N;
     const R4<R> P = spos[mine ? t : 0];
+    const P3<R> p = p3(P.x, P.y, P.z);
+    const TriWalk k = walk_of(c, mine, p.x, p.y, p.z, uhead, moved);
     R best;
     P3<R> dir;
-    const int bid = nearest_triangle_wave(c, mine, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, sph, 0, moved,
-                                          &best, &dir, Lw[threadIdx.x >> 6],
-                                          P_ == 64 ? 2 * kNearestShort : kNearestShort);
+    int bid;
+    if (P_ < 64 && !moved && __any(mine && k.h.y > kNearestShort))
+        bid = nearest_in_wave(c, mine, p, k, ulist, tris, sph, &best, &dir, *L);
+    else bid = nearest_in_lane(mine, p, k, ulist, tris, 0, &best, &dir);
     if (!mine) return;
+    if (k.h.y < 0) bid = nearest_triangle(c, p.x, p.y, p.z, tstart, tcount, tids, tris, 0, &best, &dir);
     stl_mag[t] = best;
     stl_dir[t] = mk4w<R>(dir.x, dir.y, dir.z);
     stl_id[t] = bid;
 }
 template <typename R, int P_>
-__global__ __launch_bounds__(256) void k_stl_distance(int N, Consts<R> c, const R4<R>* __restrict__ spos,
+__global__ __launch_bounds__(256, sizeof(R) == 4 ? 5 : 3) void k_stl_distance(int N, Consts<R> c, const R4<R>* __restrict__ spos,
                                                        const int* __restrict__ tstart, const int* __restrict__ tcount,
                                                        const int* __restrict__ tids, const TriD<R>* __restrict__ tris,
                                                        R* stl_mag, R4<R>* stl_dir, int* stl_id,
                                                        const int2* __restrict__ ulist, const int2* __restrict__ uhead,
                                                        const float4* __restrict__ sph, int moved) {
-    __shared__ NearestLds<R> L[4];
-    stl_distance_body<R, P_>(blockIdx.x, N, c, spos, tstart, tcount, tids, tris, stl_mag, stl_dir, stl_id, ulist, uhead, sph,
-                         moved, L);
+    const int w = (int)(threadIdx.x >> 6);
+    NearestLds<R>* L = nullptr;
+    if constexpr (P_ < 64) {
+        __shared__ NearestLds<R> lds[4];
+        L = lds + w;
+    }
+    stl_distance_body<R, P_>(blockIdx.x * 4 + w, N, c, spos, tstart, tcount, tids, tris, stl_mag, stl_dir, stl_id, ulist,
+                             uhead, sph, moved, L);
 }
 
 
@@ -725,16 +735,17 @@ __device__ inline void drag_body(int blk, int N, Consts<R> c, const int* __restr
                                  const mpsr_tri_params* __restrict__ models,
                                  const mpsr_drag_params* __restrict__ drag, R4<R>* drag_acc,
                                  R* drag_temp, const int2* __restrict__ ulist, const int2* __restrict__ uhead,
-                                 const float4* __restrict__ sph, int moved, NearestLds<R>* Lw) {
+                                 int moved) {
     const int t = blk * blockDim.x + threadIdx.x;
     const int s = t < N ? perm[t] : 0;
     const bool live = t < N && out.id[s] >= 0;
     const R4<R> P = spos[t < N ? t : 0];
     R best;
     P3<R> dir;
-    const int bid = nearest_triangle_wave(c, live, P.x, P.y, P.z, ulist, uhead, tstart, tcount, tids, tris, sph, 1, moved,
-                                          &best, &dir, Lw[threadIdx.x >> 6]);
+    const TriWalk k = walk_of(c, live, P.x, P.y, P.z, uhead, moved);
+    int bid = nearest_in_lane(live, p3(P.x, P.y, P.z), k, ulist, tris, 1, &best, &dir);
     if (!live) return;
+    if (k.h.y < 0) bid = nearest_triangle(c, P.x, P.y, P.z, tstart, tcount, tids, tris, 1, &best, &dir);
     drag_acc[t] = mk4w<R>(0, 0, 0);
     drag_temp[t] = 0;
     out.type[s] = 0;
@@ -787,11 +798,9 @@ __global__ __launch_bounds__(kMaxBlock) void k_drag(int N, Consts<R> c, const in
                                                const mpsr_tri_params* __restrict__ models,
                                                const mpsr_drag_params* __restrict__ drag, R4<R>* drag_acc,
                                                R* drag_temp, const int2* __restrict__ ulist,
-                                               const int2* __restrict__ uhead, const float4* __restrict__ sph,
-                                               int moved) {
-    __shared__ NearestLds<R> L[kMaxBlock / 64];
+                                               const int2* __restrict__ uhead, int moved) {
     drag_body<R>(blockIdx.x, N, c, perm, in, out, spos, svel, tstart, tcount, tids, tris, models, drag, drag_acc,
-                 drag_temp, ulist, uhead, sph, moved, L);
+                 drag_temp, ulist, uhead, moved);
 }
 
 template <typename R>
@@ -842,9 +851,8 @@ __global__ __launch_bounds__(256) void k_rotate(int T, TriD<R>* tris, const RotC
 
 template <typename R> void launch_stl_distance(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
-    const bool few = d.N <= kStlSplitMax;
-    hipLaunchKernelGGL((few ? k_stl_distance<R, 16> : k_stl_distance<R, 64>), dim3(grid_for(d.N, few ? 64 : 256)),
-                       dim3(256), 0, st, d.N, d.c, d.spos,
+    hipLaunchKernelGGL((d.fine_walls ? k_stl_distance<R, 16> : k_stl_distance<R, 64>),
+                       dim3(grid_for(d.N, d.fine_walls ? 64 : 256)), dim3(256), 0, st, d.N, d.c, d.spos,
                        d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.stl_mag, d.stl_dir, d.stl_id,
                        d.cell_utri, d.cell_uhead, d.tri_sph, d.walls_moved);
 }
@@ -852,7 +860,7 @@ template <typename R> void launch_drag(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
     hipLaunchKernelGGL(k_drag<R>, dim3(grid_for(d.N, d.block)), dim3(d.block), 0, st, d.N, d.c, d.perm, d.in, d.out, d.spos,
                        d.svel, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.models, d.drag, d.drag_acc,
-                       d.drag_temp, d.cell_utri, d.cell_uhead, d.tri_sph, d.walls_moved);
+                       d.drag_temp, d.cell_utri, d.cell_uhead, d.walls_moved);
 }
 template <typename R> void launch_translate(const Dev<R>& d, hipStream_t st) {
     if (d.ntri <= 0) return;
@@ -897,22 +905,26 @@ template <typename R> struct OpPairs {
     }
 };
 // (a batched step searches the walls it has just binned)
-template <typename R, int P_> struct OpStl {
+template <typename R> struct OpStl {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
         __shared__ NearestLds<R> L[4];
-        stl_distance_body<R, P_>(b, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris, d.stl_mag,
-                             d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, 0, L);
+        const int w = (int)(threadIdx.x >> 6);   // an item is 64 particles: four waves' or one's
+        if (d.fine_walls)
+            stl_distance_body<R, 16>(4 * b + w, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris,
+                                     d.stl_mag, d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, 0, &L[w]);
+        else if (w == 0)
+            stl_distance_body<R, 64>(b, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris,
+                                     d.stl_mag, d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, 0, nullptr);
     }
 };
 template <typename R> struct OpDrag {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
         const Dev<R>& d = dv[k];
-        __shared__ NearestLds<R> L[kMaxBlock / 64];
         drag_body<R>(b, d.N, d.c, d.perm, d.in, d.out, d.spos, d.svel, d.cell_tri_start, d.cell_tri_count, d.uniq_tri,
-                     d.tris, d.models, d.drag, d.drag_acc, d.drag_temp, d.cell_utri, d.cell_uhead, d.tri_sph, 0, L);
+                     d.tris, d.models, d.drag, d.drag_acc, d.drag_temp, d.cell_utri, d.cell_uhead, 0);
     }
 };
 // the walks of the batched step: (bucket, block of 256 cells) items sort the cells as
@@ -980,8 +992,8 @@ void launch_cell_walks_b(const BatchLaunch<R>& b, WorkList c256, int2* work, int
     hipLaunchKernelGGL(k_cell_walks_b<R>, dim3(2048), dim3(64), 0, st, b.devs, work, nwork);
 }
 template <typename R> void launch_stl_distance_b(const BatchLaunch<R>& b, WorkList near, hipStream_t st) {
-    static_assert(kNearBlock == 64, "four waves of 16 particles to an item");
-    launch_batched<256>(OpStl<R, 16>{b.devs}, near, 256, st);
+    static_assert(kNearBlock == 64, "four waves to an item of 64 particles");
+    launch_batched<256>(OpStl<R>{b.devs}, near, 256, st);
 }
 template <typename R> void launch_drag_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
     launch_batched<kMaxBlock>(OpDrag<R>{b.devs}, p, b.block, st);

@@ -193,7 +193,56 @@ template <typename R> __device__ inline float4 tri_sphere(const TriD<R>& t) {
 // Both bounds are those of the walls as they were binned: where the triangles have moved since (`moved`),
 // every lane walks its whole list.
 //
-// One wave, a point per lane (`want` lanes only; every lane of the wave calls it).  A full distance is a
+// the walk of a point's cell, and whether its bounds hold for the point
+struct TriWalk {
+    int2 h;
+    int cut;
+};
+template <typename R>
+__device__ inline TriWalk walk_of(const Consts<R>& c, bool want, R x, R y, R z, const int2* __restrict__ uhead, int moved) {
+    int ci = 0, cj = 0, ck = 0;
+    long long cid = -1;
+    if (want && cell_coords(c, x, y, z, ci, cj, ck)) cid = cell_of(c, ci, cj, ck);
+    TriWalk w;
+    w.h = (cid >= 0 && cid < c.ncell) ? uhead[cid] : make_int2(0, -1);
+    const R slack = c.cell * (R)0.005;
+    const R lox = c.bminx + (R)ci * c.cell, loy = c.bminy + (R)cj * c.cell, loz = c.bminz + (R)ck * c.cell;
+    w.cut = !moved && x >= lox - slack && x <= lox + c.cell + slack && y >= loy - slack &&
+            y <= loy + c.cell + slack && z >= loz - slack && z <= loz + c.cell + slack;
+    return w;
+}
+
+// Each lane (of those with `want`) walks its own list, if it has one: the drag search, and lists so short that
+// the wave's search costs more.
+template <typename R>
+__device__ inline int nearest_in_lane(bool want, P3<R> p, const TriWalk& w, const int2* __restrict__ ulist,
+                                      const TriD<R>* __restrict__ tris, int want_drag, R* best, P3<R>* bdir) {
+    *best = (R)1e8;
+    *bdir = p3<R>(0, 0, 0);
+    int bid = -1, bpos = 0;
+    const int n = want ? w.h.y : 0;
+    int2 next = n > 0 ? ulist[w.h.x] : make_int2(0, 0);
+    for (int e = 0; e < n; ++e) {
+        const int2 en = next;
+        next = ulist[w.h.x + min(e + 1, n - 1)];   // on its way while this triangle's record is
+        if (w.cut && (R)__uint_as_float((unsigned)en.y & ~kWalkPosMask) > *best) break;
+        const TriD<R>& tr = tris[en.x];
+        if (tr.is_drag != want_drag) continue;
+        P3<R> dv;
+        const R dm = tri_distance(tr, p, &dv);
+        const int pos = (int)((unsigned)en.y & kWalkPosMask);
+        if (dm < *best || (dm == *best && bid >= 0 && pos < bpos)) {
+            *best = dm;
+            *bdir = dv;
+            bid = en.x;
+            bpos = pos;
+        }
+    }
+    return bid;
+}
+
+// The nearest listed wall (no drag triangle) by one wave, a point per lane (`want` lanes only; every lane of the
+// wave calls it).  A full distance is a
 // chain of about 250 instructions, and a particle near a fine wall has 70-130 listed triangles, of which a
 // few are near it.  So the points with a list are taken eight at a time, eight lanes to a point (lane
 // 8 j + q takes entries j, j + 8, ... of point q; the points of a cell read the same entries).  A first
@@ -202,10 +251,7 @@ template <typename R> __device__ inline float4 tri_sphere(const TriD<R>& t) {
 // queue is tested 64 pairs at a time.  A triangle left out is farther than the nearest, so it is neither
 // nearer nor as near, and the least (distance, position) does not depend on who tests what.
 // Per pass, each lane walking its own list / this (rotating drums): 141 / 41 us at 62k particles, 102 / 45 at
-// 126k, 75 / 60 at 517k, FP64 142 / 76 at 126k; 16 buckets of 730k particles 279 / 179.  Lists of at most `short_list` triangles stay with
-// their lanes: 16 (a tank of 14 triangles: 8 us a pass, 16 us taken together), or 32 where a wave holds 64
-// points (the 1M drum's 20-30 triangles: 72 us against 84; in waves of 16 points that walk loses, 113 us
-// against 60 at 517k).
+// 126k, 75 / 60 at 517k, FP64 142 / 76 at 126k; 16 buckets of 730k particles 279 / 179.
 template <typename R> struct NearestLds {
     unsigned long long best[64];   // bits of the nearest distance as a double
     P3<R> dir[64];
@@ -213,46 +259,16 @@ template <typename R> struct NearestLds {
     unsigned queue[kNearestQueue + 64];
 };
 template <typename R>
-__device__ inline int nearest_triangle_wave(const Consts<R>& c, bool want, R x, R y, R z, const int2* __restrict__ ulist,
-                                            const int2* __restrict__ uhead, const int* __restrict__ tstart,
-                                            const int* __restrict__ tcount, const int* __restrict__ tids,
-                                            const TriD<R>* __restrict__ tris, const float4* __restrict__ sph,
-                                            int want_drag, int moved, R* best, P3<R>* bdir, NearestLds<R>& L,
-                                            int short_list = kNearestShort) {
+__device__ inline int nearest_in_wave(const Consts<R>& c, bool want, P3<R> pt, const TriWalk& wk,
+                                      const int2* __restrict__ ulist, const TriD<R>* __restrict__ tris,
+                                      const float4* __restrict__ sph, R* best, P3<R>* bdir, NearestLds<R>& L) {
     const int lane = lane_id();
+    const R x = pt.x, y = pt.y, z = pt.z;
+    const int2 h = wk.h;
+    const int cut = wk.cut;
     *best = (R)1e8;
     *bdir = p3<R>(0, 0, 0);
-    int ci = 0, cj = 0, ck = 0;
-    long long cid = -1;
-    if (want && cell_coords(c, x, y, z, ci, cj, ck)) cid = cell_of(c, ci, cj, ck);
-    const int2 h = (cid >= 0 && cid < c.ncell) ? uhead[cid] : make_int2(0, -1);
-    const R slack = c.cell * (R)0.005;
-    const R lox = c.bminx + (R)ci * c.cell, loy = c.bminy + (R)cj * c.cell, loz = c.bminz + (R)ck * c.cell;
-    const int cut = !moved && x >= lox - slack && x <= lox + c.cell + slack && y >= loy - slack &&
-                    y <= loy + c.cell + slack && z >= loz - slack && z <= loz + c.cell + slack;
     const bool listed = want && h.y > 0;
-    if (moved || !__any(listed && h.y > short_list)) {
-        // short lists (walls of a few large triangles): each lane walks its own
-        int bid = -1, bpos = 0;
-        const P3<R> p = p3(x, y, z);
-        for (int e = 0; listed && e < h.y; ++e) {
-            const int2 en = ulist[h.x + e];
-            if (cut && (R)__uint_as_float((unsigned)en.y & ~kWalkPosMask) > *best) break;
-            const TriD<R>& tr = tris[en.x];
-            if (tr.is_drag != want_drag) continue;
-            P3<R> dv;
-            const R dm = tri_distance(tr, p, &dv);
-            const int pos = (int)((unsigned)en.y & kWalkPosMask);
-            if (dm < *best || (dm == *best && bid >= 0 && pos < bpos)) {
-                *best = dm;
-                *bdir = dv;
-                bid = en.x;
-                bpos = pos;
-            }
-        }
-        if (want && h.y < 0) bid = nearest_triangle(c, x, y, z, tstart, tcount, tids, tris, want_drag, best, bdir);
-        return bid;
-    }
     const unsigned long long mask = __ballot(listed);
     const int count = __popcll(mask), q = lane & 7, j = lane >> 3;
     L.best[lane] = (unsigned long long)__double_as_longlong(1e8);
@@ -334,7 +350,7 @@ __device__ inline int nearest_triangle_wave(const Consts<R>& c, bool want, R x, 
         walk(up, [&](bool on, int e, const float4& sp) {
             const float dx = px - sp.x, dy = py - sp.y, dz = pz - sp.z;
             const float u = (sqrtf(dx * dx + dy * dy + dz * dz) + fabsf(sp.w)) * 1.005f + margin;
-            if (on && (sp.w < 0.f) == (want_drag != 0) && u < up) {
+            if (on && !(sp.w < 0.f) && u < up) {
                 up = u;
                 eup = e;
             }
@@ -349,7 +365,7 @@ __device__ inline int nearest_triangle_wave(const Consts<R>& c, bool want, R x, 
         walk(up, [&](bool on, int e, const float4& sp) {
             const float dx = px - sp.x, dy = py - sp.y, dz = pz - sp.z;
             const float far = (up + margin) * 1.026f + fabsf(sp.w);
-            const bool take = on && e != eup && (sp.w < 0.f) == (want_drag != 0) && !(dx * dx + dy * dy + dz * dz > far * far);
+            const bool take = on && e != eup && !(sp.w < 0.f) && !(dx * dx + dy * dy + dz * dz > far * far);
             push(take, e);
             if (queued > kNearestQueue) flush();
         });
@@ -362,8 +378,6 @@ __device__ inline int nearest_triangle_wave(const Consts<R>& c, bool want, R x, 
             *best = (R)__longlong_as_double((long long)L.best[lane]);
             *bdir = L.dir[lane];
         }
-    } else if (want && h.y < 0) {
-        bid = nearest_triangle(c, x, y, z, tstart, tcount, tids, tris, want_drag, best, bdir);
     }
     return bid;
 }
