@@ -511,8 +511,11 @@ mpsr_status mpsr_calc_turbulence_viscosity(mpsr_handle *h);
 mpsr_status mpsr_get_turbulence(mpsr_handle *h, double *viscosity, double *kinetic_energy, int n);
 
 /* Launch shape of the per-particle kernels (block: a multiple of 64 in [64, 512]) and of the
- * particle sort (tile = 256 * sort_items keys, sort_items 4, 8 or 16).  Results do not depend on
- * it.  No counterpart in the reference (its launchers fix 256 threads, DeviceProcess.cu:29-304). */
+ * particle sort (tile = 256 * sort_items keys, sort_items 4, 8 or 16; until it is set, 4 up to 200,000
+ * particles and 8 above).  Results do not depend on it.  The kernels that work in single waves have a
+ * shape of their own: the neighbour sums (PND, heat conduction, turbulence, the predictor in FP64 and up
+ * to 200,000 particles) and the wall distance.  No counterpart in the reference (its launchers fix 256
+ * threads, DeviceProcess.cu:29-304). */
 mpsr_status mpsr_set_launch(mpsr_handle *h, int block, int sort_items);
 
 /* ---- batched buckets (no counterpart in the reference) ------------------------------------------

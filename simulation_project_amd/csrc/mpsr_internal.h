@@ -319,10 +319,10 @@ size_t scan_tmp_ints(int n_cap);
 // Stable LSD radix sort of (key, value) pairs on `bits` low key bits.  n is *d_n when d_n is
 // non-null (device-resident count, n_cap bounds it), else n_host.  The result ends in (k0, v0)
 // or in (s.k1, s.v1); the return value says which (0 or 1).
-// `items` (4, 8 or 16) sets the tile of 256 * items keys (4 up to 200k keys); every tile gives the same
-// result.
+// `items` (4, 8 or 16) sets the tile of 256 * items keys, 0 leaves it to the key count; every tile gives the
+// same result.
 int radix_sort_pairs(uint32_t* k0, int* v0, const int* d_n, int n_host, int n_cap, int bits,
-                     const SortScratch& s, hipStream_t st, int items = 8);
+                     const SortScratch& s, hipStream_t st, int items = 0);
 bool radix_items_valid(int items);
 // Exclusive scan of n ints (n = *d_n or n_host); *d_total (if non-null) receives the sum.
 void exclusive_scan(const int* in, int* out, const int* d_n, int n_host, int n_cap, int* d_total,
@@ -424,7 +424,7 @@ static constexpr int kMarchTab = 1024;
 template <typename R> struct Dev {
     int N = 0, cap = 0;
     int block = 256;                  // threads per block of the per-particle kernels (64..512)
-    int sort_items = 8;               // radix-sort tile = 256 * sort_items keys (4, 8, 16)
+    int sort_items = 0;               // radix-sort tile = 256 * sort_items keys (4, 8, 16); 0: by the key count
     int ntri = 0, nmodel = 0, ndrag = 0;
     Consts<R> c{};
     PState<R> in{}, out{};

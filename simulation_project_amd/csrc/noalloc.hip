@@ -127,7 +127,7 @@ extern "C" mpsr_status mpsr_register_particle_topology_noalloc(const mpsr_gridbo
     } else {
         hipLaunchKernelGGL(k_na_keys, dim3(grid_clearing(n, ncell, 256)), dim3(256), 0, st, n, c, id, px, py, pz,
                            (uint32_t*)sorted_keys, perm, cell_start, cell_end);
-        const int which = radix_sort_pairs((uint32_t*)sorted_keys, perm, nullptr, n, n, bits, ss, st, 8);
+        const int which = radix_sort_pairs((uint32_t*)sorted_keys, perm, nullptr, n, n, bits, ss, st);
         if (which)
             hipLaunchKernelGGL(k_na_copy, dim3(grid_for(n, 256)), dim3(256), 0, st, n, ss.k1, ss.v1,
                                (uint32_t*)sorted_keys, perm);

@@ -394,7 +394,7 @@ int radix_sort_pairs(uint32_t* k0, int* v0, const int* d_n, int n_host, int n_ca
     const int cap = d_n ? n_cap : n_host;
     if (cap <= 0 || bits <= 0) return 0;
     // few keys: smaller tiles, whose rounds are a chain (downsweep of 4k keys 9.5 us with 8 rounds a wave)
-    if (cap <= 200000) items = 4;
+    if (items == 0) items = cap <= 200000 ? 4 : 8;
     switch (items) {
         case 4: return radix_sort_tiles<4>(k0, v0, d_n, n_host, cap, bits, s, st);
         case 16: return radix_sort_tiles<16>(k0, v0, d_n, n_host, cap, bits, s, st);

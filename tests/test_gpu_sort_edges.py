@@ -1,6 +1,6 @@
 """The particle sort at the edges of its forms, against numpy's stable argsort of the keys: digits of one
 to nine bits and one to three passes (grids of 1 to over 2^18 cells), key counts around the tiles of
-1,024 and 2,048 keys and around the 200k keys where the tile changes."""
+1,024 and 2,048 keys and around the 200k keys where the tile changes, and the tiles that a caller sets."""
 import ctypes as C
 
 import numpy as np
@@ -15,6 +15,17 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 2, 1023, 1024, 1025, 2049, 199999, 200000, 200001, 262145])
 @pytest.mark.parametrize("side", [1, 3, 7, 8, 40, 70])
 def test_sort_is_the_stable_argsort(n, side):
+    check_sort(n, side, None)
+
+
+@pytest.mark.parametrize("n", [1, 4095, 4096, 4097, 200000, 262145])
+@pytest.mark.parametrize("side", [7, 40, 70])
+@pytest.mark.parametrize("items", [4, 8, 16])
+def test_sort_in_a_tile_of_the_callers(n, side, items):
+    check_sort(n, side, items)
+
+
+def check_sort(n, side, items):
     lib = load_library()
     case = cases.small_box(lib, nx=4, ny=4, nz=4)
     l0 = case.meta["l0"]
@@ -27,6 +38,8 @@ def test_sort_is_the_stable_argsort(n, side):
     pa.position[:] = (base + rng.uniform(0, side * 3.1 * l0, (n, 3))).astype(np.float32)
     case.particles = pa
     s = Solver(case)
+    if items:
+        s.set_launch(32 * items, items)
     s.RegisterParticleTopology()
     keys, perm, start, end = s.binning()
     g = s.gridbox
