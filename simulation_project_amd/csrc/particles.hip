@@ -224,7 +224,7 @@ __device__ inline void explicit_finish(int t, int s, const Consts<R>& c, const P
 // sums): FP32 107 / 186 us at 4k particles, 165 / 193 and 174 / 238 at 126k, 280 / 257 and 302 / 327 at
 // 245k, 534 / 473 and 570 / 560 at 517k, 928 / 801 and 998 / 968 at 1M; FP64 128 / 289 at 32k, 800 / 1063
 // at 517k, 1154 / 2062 at 1M.
-template <typename R> static bool near_explicit(long long n) { return sizeof(R) == 8 || n <= 200000; }
+static constexpr int kNearExplicitMax = 200000;   // in FP32; FP64 always takes the near walk
 template <typename R, bool NEAR>
 __device__ inline void explicit_body(int blk, int N, Consts<R> c, const int* __restrict__ perm,
                                      PState<R> in, PState<R> out, const R4<R>* __restrict__ spos,
@@ -847,11 +847,15 @@ __global__ __launch_bounds__(kNearBlock, 3) void k_turbulence(int N, Consts<R> c
 
 template <typename R> void launch_explicit(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0) return;
-    const bool near = near_explicit<R>(d.N);
-    const int block = near ? kNearBlock : d.block;
-    hipLaunchKernelGGL((near ? k_explicit<R, true> : k_explicit<R, false>), dim3(xcd_grid(d.N, block)), dim3(block), 0,
-                       st, d.N, d.c, d.perm, d.in, d.out, d.spos, d.svel, d.rel, d.skeys, d.cell_start, d.cell_end,
-                       d.stl_mag, d.stl_dir, d.stl_id, d.drag_acc, d.sph_dv, d.tris, d.models, d.turb_nu);
+    auto launch = [&](auto kernel, int block) {
+        hipLaunchKernelGGL(kernel, dim3(xcd_grid(d.N, block)), dim3(block), 0, st, d.N, d.c, d.perm, d.in, d.out, d.spos,
+                           d.svel, d.rel, d.skeys, d.cell_start, d.cell_end, d.stl_mag, d.stl_dir, d.stl_id, d.drag_acc,
+                           d.sph_dv, d.tris, d.models, d.turb_nu);
+    };
+    if constexpr (sizeof(R) == 4) {
+        if (d.N > kNearExplicitMax) return launch(k_explicit<R, false>, d.block);
+    }
+    launch(k_explicit<R, true>, kNearBlock);
 }
 template <typename R> void launch_turbulence(const Dev<R>& d, hipStream_t st) {
     if (d.N <= 0 || !d.turb_nu) return;
@@ -994,9 +998,11 @@ template <typename R> void launch_bin_ranges_b(const BatchLaunch<R>& b, WorkList
     launch_batched<kMaxBlock>(OpBinRanges<R>{b.devs}, p, b.block, st);
 }
 template <typename R> void launch_explicit_b(const BatchLaunch<R>& b, WorkList p, WorkList near, hipStream_t st) {
-    if (near_explicit<R>((long long)near.n * kNearBlock))
-        launch_batched<kNearBlock>(OpExplicit<R, true>{b.devs}, near, kNearBlock, st);
-    else launch_batched<kMaxBlock>(OpExplicit<R, false>{b.devs}, p, b.block, st);
+    if constexpr (sizeof(R) == 4) {
+        if ((long long)near.n * kNearBlock > kNearExplicitMax)
+            return launch_batched<kMaxBlock>(OpExplicit<R, false>{b.devs}, p, b.block, st);
+    }
+    launch_batched<kNearBlock>(OpExplicit<R, true>{b.devs}, near, kNearBlock, st);
 }
 template <typename R> void launch_relocate_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
     launch_batched<kMaxBlock>(OpRelocate<R>{b.devs}, p, b.block, st);
