@@ -856,14 +856,16 @@ __device__ inline void pcg_write(int mode, double s0, double s1, PcgStep w, doub
 }
 
 // The sums of k_pcg_reduce formed again by every workgroup that needs them, for solves of at most
-// kFoldMax partials (262,144 rows: one partial a thread of k_pcg_reduce, so the waves' sums and their
-// order are the same).  Two launches of 3.3-4.5 us an iteration go; at 62k particles their readers take
+// kFoldMax partials (163,840 rows; below 1,024, where a thread of k_pcg_reduce has one, so the waves' sums and
+// their order are the same).  Two launches of 3.3-4.5 us an iteration go; at 62k particles their readers take
 // 4.5 us for 4.0 (k_cell_pre), 3.6 for 1.9 (k_pcg_direction), 4.5 for 4.1 (k_pcg_update), and 327 launches a
-// step are left of 390.  With more partials every workgroup would read 31 KB and more (1M rows) against
-// 4.7 us of the one workgroup.  The scalars alternate between two copies: alpha's readers take scal and
+// step are left of 390.  The readers' workgroups and what each reads both grow with the rows: the solves of
+// a step, with the launches / folded (V-cycle), take 1,778 / 1,661 us at 62k rows, 2,352 / 2,276 at 126k, 2,354
+// / 2,347 at 155k, 2,749 / 2,792 at 206k and 2,763 / 2,844 at 245k; FP64 2,957 / 2,930 at 155k and 3,804 / 3,890 at
+// 245k.  The scalars alternate between two copies: alpha's readers take scal and
 // write scal + S_COUNT, beta's the other way round, so no workgroup reads what another of its launch
 // writes.
-static constexpr int kFoldMax = 1024;
+static constexpr int kFoldMax = 640;
 // the step's scalars for the whole workgroup, workgroup 0 writing them to `out`; false when the solve has
 // stopped (before this step or by it)
 __device__ inline bool pcg_fold(int blk, int mode, const double* __restrict__ part, int nb,

@@ -1,6 +1,6 @@
-"""The PCG's reductions, formed by their readers in solves of at most 1,024 partial sums (262,144 rows)
-and by a kernel of their own above: the residual b - A x, summed here in FP64 from the matrix and the
-solution the solver hands out, meets the tolerance on both sides of that line and where the partial
+"""The PCG's reductions, formed by their readers in solves of at most 640 partial sums (163,840 rows)
+and by a kernel of their own above, which has one sum a thread up to 1,024 (262,144 rows): the residual b - A x, summed here in FP64 from the matrix and the
+solution the solver hands out, meets the tolerance on both sides of those lines and where the partial
 sums fill one wave (16,384 rows), one more than a wave, or less than one."""
 import numpy as np
 import pytest
@@ -14,7 +14,8 @@ TOL = 1e-8
 
 
 @pytest.mark.parametrize("solver,precond", [(abi.MPSR_PCG_FP64, 0), (abi.MPSR_PCG_MIXED, abi.MPSR_PRECOND_CELL_VCYCLE)])
-@pytest.mark.parametrize("size", [(4, 4, 4), (16, 16, 64), (16, 16, 65), (64, 64, 64), (64, 64, 65)])
+@pytest.mark.parametrize("size", [(4, 4, 4), (16, 16, 64), (16, 16, 65), (64, 64, 40), (64, 64, 41), (64, 64, 64),
+                                  (64, 64, 65)])
 def test_residual_on_both_sides_of_the_line(solver, precond, size):
     lib = load_library()
     nx, ny, nz = size
