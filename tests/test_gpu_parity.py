@@ -352,8 +352,8 @@ def test_large_drum_binning_properties(lib):
 
 
 def test_large_drum_identical(lib):
-    # 10k triangles and 17-bit cell keys (three radix passes): the wall pairs and the particle
-    # permutation both go through the multi-tile, odd-pass sort path
+    # 10k triangles and 17-bit cell keys (two radix passes): the wall pairs and the particle
+    # permutation both go through the multi-tile sort
     case = cases.drum(lib, l0=2.5e-3)
     g, o = pair(case)
     assert g.cells > 65536
@@ -369,6 +369,25 @@ def test_large_drum_identical(lib):
     g.step_many(0, 3)
     o.step_many(0, 3)
     same_state(g, o, label="drum 3 steps")
+
+
+@pytest.mark.parametrize("precision", [abi.MPSR_FP32, abi.MPSR_FP64])
+def test_drum_in_a_large_grid_identical(lib, precision):
+    # over 2^18 cells (three radix passes): the sorted keys and permutation of the particles and the wall
+    # pairs end in the sort's scratch, and the lists, walks and steps read them there
+    case = cases.drum(lib, l0=5e-3)
+    hi = case.zone.m_MaxBound
+    hi.x, hi.y, hi.z = hi.x + 0.8, hi.y + 0.8, hi.z + 0.8
+    g, o = pair(case, precision=precision)
+    assert g.cells > 1 << 18
+    for phase in ("RegisterParticleTopology", "RegisterTriangleTopology"):
+        run_phase(phase, g, o)
+    for what in ("triangle_cells", "binning"):
+        for a, b in zip(getattr(g, what)(), getattr(o, what)()):
+            np.testing.assert_array_equal(a, b)
+    g.step_many(0, 3)
+    o.step_many(0, 3)
+    same_state(g, o, label="3 steps")
 
 
 @pytest.mark.parametrize("solver", [abi.MPSR_PCG_FP64, abi.MPSR_PCG_MIXED])
