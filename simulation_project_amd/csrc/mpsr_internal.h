@@ -61,7 +61,6 @@ template <typename R> struct Consts {
     R bminx, bminy, bminz;
     R cminx, cminy, cminz, cmaxx, cmaxy, cmaxz;
     R cell;
-    float far_eps;     // 2^-23 times the grid's largest coordinate: what a coordinate's rounding to float moves it
     int gx, gy, gz, ncell;
     R tol, l0, dt;
     // explicit predictor, Kern :283-441
@@ -85,6 +84,7 @@ template <typename R> struct Consts {
     R turb_cs, turb_fw;       // SmagorinskyConstant, FilterWidth
     R turb_numax, turb_kmax;  // TurbulanViscosityRatio, TurbulanceIntensity
     R turb_tk;                // 2 Cnue l0 l0 / Cepsilon
+    float far_eps;     // 2^-23 times the grid's largest coordinate: what a coordinate's rounding to float moves it
 };
 
 // per-model negative-pressure fields (radix CTriangleParameters, DataType.h:160-168)

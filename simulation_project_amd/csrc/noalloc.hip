@@ -50,11 +50,12 @@ __global__ __launch_bounds__(256) void k_na_keys(int N, Consts<float> c, const i
                                                  const float* __restrict__ pz, uint32_t* keys, int* vals, int* cs,
                                                  int* ce) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < N) {
+        keys[s] = bin_key(c, id[s], px[s], py[s], pz[s]);
+        vals[s] = s;
+    }
     // the cells are empty until k_na_ranges finds their particles
     for_cells(c.ncell, [&](unsigned i) { cs[i] = ce[i] = -1; });
-    if (s >= N) return;
-    keys[s] = bin_key(c, id[s], px[s], py[s], pz[s]);
-    vals[s] = s;
 }
 
 __global__ __launch_bounds__(256) void k_na_copy(int N, const uint32_t* __restrict__ ka, const int* __restrict__ va,
