@@ -904,21 +904,21 @@ template <typename R> struct OpPairs {
         else pair_ranges_body(b, d.uniq_n, d.uniq_cell, d.cell_tri_start, d.cell_tri_count);
     }
 };
-// (a batched step searches the walls it has just binned)
-template <typename R> struct OpStl {
-    const Dev<R>* dv;
-    __device__ void operator()(int k, int b) const {
-        const Dev<R>& d = dv[k];
-        __shared__ NearestLds<R> L[4];
-        const int w = (int)(threadIdx.x >> 6);   // an item is 64 particles: four waves' or one's
-        if (d.fine_walls)
-            stl_distance_body<R, 16>(4 * b + w, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris,
-                                     d.stl_mag, d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, 0, &L[w]);
-        else if (w == 0)
-            stl_distance_body<R, 64>(b, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris,
-                                     d.stl_mag, d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, 0, nullptr);
-    }
-};
+// (a batched step searches the walls it has just binned; five waves a SIMD as k_stl_distance)
+template <typename R>
+__global__ __launch_bounds__(256, sizeof(R) == 4 ? 5 : 3) void k_stl_distance_b(const Dev<R>* __restrict__ dv,
+                                                                                const int2* __restrict__ items) {
+    __shared__ NearestLds<R> L[4];
+    const int2 i = items[blockIdx.x];
+    const Dev<R>& d = dv[i.x];
+    const int w = (int)(threadIdx.x >> 6);   // an item is 64 particles: four waves' or one's
+    if (d.fine_walls)
+        stl_distance_body<R, 16>(4 * i.y + w, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris,
+                                 d.stl_mag, d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, 0, &L[w]);
+    else if (w == 0)
+        stl_distance_body<R, 64>(i.y, d.N, d.c, d.spos, d.cell_tri_start, d.cell_tri_count, d.uniq_tri, d.tris,
+                                 d.stl_mag, d.stl_dir, d.stl_id, d.cell_utri, d.cell_uhead, d.tri_sph, 0, nullptr);
+}
 template <typename R> struct OpDrag {
     const Dev<R>* dv;
     __device__ void operator()(int k, int b) const {
@@ -993,7 +993,7 @@ void launch_cell_walks_b(const BatchLaunch<R>& b, WorkList c256, int2* work, int
 }
 template <typename R> void launch_stl_distance_b(const BatchLaunch<R>& b, WorkList near, hipStream_t st) {
     static_assert(kNearBlock == 64, "four waves to an item of 64 particles");
-    launch_batched<256>(OpStl<R>{b.devs}, near, 256, st);
+    if (near.n > 0) hipLaunchKernelGGL(k_stl_distance_b<R>, dim3(near.n), dim3(256), 0, st, b.devs, near.items);
 }
 template <typename R> void launch_drag_b(const BatchLaunch<R>& b, WorkList p, hipStream_t st) {
     launch_batched<kMaxBlock>(OpDrag<R>{b.devs}, p, b.block, st);
