@@ -866,6 +866,8 @@ __device__ inline void pcg_write(int mode, double s0, double s1, PcgStep w, doub
 // write scal + S_COUNT, beta's the other way round, so no workgroup reads what another of its launch
 // writes.
 static constexpr int kFoldMax = 640;
+// in a batch, where the launches serve every bucket: as far as the sums' order is k_pcg_reduce's
+static constexpr int kFoldMaxBatch = 1024;
 // the step's scalars for the whole workgroup, workgroup 0 writing them to `out`; false when the solve has
 // stopped (before this step or by it)
 __device__ inline bool pcg_fold(int blk, int mode, const double* __restrict__ part, int nb,
@@ -2936,7 +2938,7 @@ template <typename R> struct OpPReduce {
             return;
         }
         if (mode == RED_ALPHA || mode == RED_BETA)
-            if (v.nb <= kFoldMax) return;   // their readers form the sums
+            if (v.nb <= kFoldMaxBatch) return;   // their readers form the sums
         pcg_reduce_body(b, mode == RED_ALPHA ? v.part + 2 * (size_t)v.nb : v.part, v.nb, mode == RED_ALPHA ? 1 : 2,
                         v.scal, mode);
     }
@@ -2978,7 +2980,7 @@ template <typename R> struct OpPUpdate {
     const PpeView<R>* pv;
     __device__ void operator()(int j, int b) const {
         const PpeView<R>& v = pv[j];
-        if (v.nb <= kFoldMax)
+        if (v.nb <= kFoldMaxBatch)
             pcg_update_body<double, true>(b, v.N, v.x, v.r, v.z, v.p, v.q, v.diag, v.scal, v.part,
                                           v.part + 2 * (size_t)v.nb, v.nb, v.scal + S_COUNT);
         else
@@ -2989,7 +2991,7 @@ template <typename R> struct OpPDirection {
     const PpeView<R>* pv;
     __device__ void operator()(int j, int b) const {
         const PpeView<R>& v = pv[j];
-        if (v.nb <= kFoldMax)
+        if (v.nb <= kFoldMaxBatch)
             pcg_direction_body<double, true>(b, v.N, v.z, v.p, v.scal + S_COUNT, v.part, v.nb, v.scal);
         else
             pcg_direction_body<double, false>(b, v.N, v.z, v.p, v.scal, nullptr, 0, nullptr);
@@ -3170,7 +3172,7 @@ template <typename R> void ppe_batch_pnd(PpeBatch<R>* b, const BatchLaunch<R>& b
 }
 template <typename R> void ppe_batch_iterate(PpeBatch<R>* b, int iters, hipStream_t st) {
     bool big = false;   // a bucket whose reductions are not folded
-    for (const PpeView<R>& v : b->hv) big |= v.nb > kFoldMax;
+    for (const PpeView<R>& v : b->hv) big |= v.nb > kFoldMaxBatch;
     for (int k = 0; k < iters; ++k) {
         launch_batched<PB>(OpPSpmv<R>{b->views}, b->wvec, PB, st);
         if (big) launch_batched<1024>(OpPReduce<R>{b->views, RED_ALPHA}, b->wone, 1024, st);
